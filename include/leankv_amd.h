@@ -290,6 +290,27 @@ int lkv_tq_prod_dequantize(const uint8_t* codes, const void* norms, int norm_dty
                            void* stream);
 
 /*
+ * TurboQuantCache.update of S >= 1 new tokens for one layer
+ * (leankv/turboquant/cache.py:84-159) on the static ring layout of
+ * lkv_tq_cache_append, the length before them (p0) given by the host: tokens
+ * max(0, p0 - hot_cap) .. p0 + S - hot_cap - 1 leave the fp16 window and are
+ * quantized (widened to fp32 as cache.py:141-142 does; those below p0 from
+ * their ring slots, the others from k_new / v_new) into their cold rows, and
+ * the newest min(S, hot_cap) tokens take their ring slots.  Keys and values in
+ * one launch.
+ *   k_new, v_new: fp16 rows of 128 [B][H][S], strides of B, H and S in
+ *     elements (host arrays of 3; multiples of 8), 16-byte aligned
+ *   k_hot, v_hot: fp16 [B * H, hot_cap, 128];  k_codes, v_codes: uint8
+ *   [B * H, cap, row_bytes];  k_norms, v_norms: fp32 [B * H, cap]
+ * Refused if p0 + S - hot_cap > cap.  Needs B * H * (S + hot_cap) < 2^31.
+ */
+int lkv_tq_cache_bulk_update(const void* k_new, const int64_t* k_strides, const void* v_new,
+                             const int64_t* v_strides, int64_t B, int64_t H, int64_t S, int64_t p0,
+                             void* k_hot, void* v_hot, uint8_t* k_codes, float* k_norms, uint8_t* v_codes,
+                             float* v_norms, const float* PiK, const float* PiV, const float* bounds, int bits,
+                             int64_t hot_cap, int64_t cap, void* stream);
+
+/*
  * Decode-step cache append of TurboQuantCache.update for one layer
  * (leankv/turboquant/cache.py:84-159) on a static ring layout.
  * Current length before the append is *pos (device int32, read by the

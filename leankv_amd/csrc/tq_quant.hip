@@ -8,6 +8,8 @@
 // 16-vector tiles so the Pi operand is read from L2 once per block, not once
 // per tile.  Codes go through LDS so that packed rows leave in coalesced
 // dword stores.
+#include <algorithm>
+
 #include "tq_common.h"
 
 namespace lkv {
@@ -18,48 +20,105 @@ using namespace tq;
 enum Mode { kQuant = 0, kRotate = 1, kDequant = 2, kAppend = 3 };
 
 // ---------------------------------------------------------------- quantize
-// Nibble layouts (3- and 4-bit codes): one wave owns a whole 16-vector tile
-// and computes all 8 output column tiles, so each vector is loaded and
-// normalised once (the 4-wave kernel below repeats both in every wave).
-// Column tile c holds output dims 8n + c (n = lane % 16): exactly nibble c
-// of packed dword n, so a lane packs the dwords of its 4 rows in registers
-// and stores them directly.  Each output's MFMA chain -- the same 32 k-steps
-// with the same operands in the same order as rotate_tile -- is unchanged,
-// so the codes equal every other quantizing kernel's bit for bit.  The B
-// operands of the 8 tiles are staged once per block in LDS in MFMA operand
-// order: s_b[c][kq][lane] = Pi[8n + c][32q + 4kq .. +3] for lane = 16q + n
-// (rows padded by one float4 so the staging writes do not collide in banks).
-// #(b < y) over the 2^BITS - 1 sorted decision boundaries by binary search
-// (BITS compares instead of 2^BITS - 1): the same count as bucket<BITS>.
-// Every boundary index is a compile-time constant (selects, no indexing).
+// One wave owns a whole 16-vector tile and computes all 8 output column
+// tiles, so each vector is loaded and normalised once.  Column tile c holds
+// output dims 8n + c (n = lane % 16): code field c of the 8 codes that lane
+// packs for each of its 4 rows and stores directly (a dword at 3 and 4 bits, 16
+// bits at 2, a byte at 1).  Each output's MFMA chain -- the same 32 k-steps
+// with the same operands in the same order as rotate_tile -- is that of every
+// other quantizing kernel, so the codes are equal bit for bit.  The B operands
+// of the 8 tiles are staged once per block in LDS in MFMA operand order:
+// s_b[c][kq][lane] = Pi[8n + c][32q + 4kq .. +3] for lane = 16q + n (rows
+// padded by one float4, so that the staging writes of 8 consecutive threads, 8
+// k-quarters, fall in different banks).
+typedef float4 PiTiles[8][8][65];  // 66.5 KB: two blocks per CU
+constexpr int kPiLoads = kD * kD / 4 / kThreads;
+
+// Pi, coalesced: thread tid holds float4 f = 256 i + tid (row f / 32, columns 4 (f % 32) ..).
+__device__ __forceinline__ void load_pi_coalesced(const float* __restrict__ Pi, float4 (&pr)[kPiLoads]) {
+#pragma unroll
+  for (int i = 0; i < kPiLoads; ++i) pr[i] = reinterpret_cast<const float4*>(Pi)[i * kThreads + threadIdx.x];
+}
+__device__ __forceinline__ void stage_pi(const float4 (&pr)[kPiLoads], PiTiles& s_b) {
+#pragma unroll
+  for (int i = 0; i < kPiLoads; ++i) {
+    const int f = i * kThreads + threadIdx.x;
+    const int j = f >> 5, c4 = f & 31;  // Pi row j = 8n' + c, columns 32q' + 4kq ..
+    s_b[j & 7][c4 & 7][16 * (c4 >> 3) + (j >> 3)] = pr[i];
+  }
+}
+
+__device__ __forceinline__ void rotate_wave_tile(const float (&a)[32], const PiTiles& s_b, int lane, f32x4 (&acc)[8]) {
+#pragma unroll
+  for (int c = 0; c < 8; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kq = 0; kq < 8; ++kq) {
+    float4 bv[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) bv[c] = s_b[c][kq][lane];
+#pragma unroll
+    for (int cc = 0; cc < 4; ++cc) {
+      const float av = a[4 * kq + cc];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const float b = cc == 0 ? bv[c].x : cc == 1 ? bv[c].y : cc == 2 ? bv[c].z : bv[c].w;
+        acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b, acc[c], 0, 0, 0);
+      }
+    }
+    // keeps the next k-quarter's LDS reads after these MFMAs (the compiler
+    // otherwise hoists all 256 operand values and spills)
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// #(b < y) over the 2^BITS - 1 sorted decision boundaries: the count of
+// bucket<BITS>, by binary search from 3 bits on.  3 bits: every boundary index
+// is a compile-time constant (selects, no indexing).  4 bits: a table in LDS,
+// the next boundary addressed by the bucket so far (kept in registers, the
+// selects between boundaries compile to an indexed load from a private,
+// memory-backed copy of the table).
 template <int BITS>
-__device__ __forceinline__ int bucket_bsearch(float y, const float (&bd)[(1 << BITS) - 1]) {
-  static_assert(BITS == 3 || BITS == 4, "nibble layouts");
+__device__ __forceinline__ int bucket_fast(float y, const float (&bd)[(1 << BITS) - 1], const float* s_bd) {
   if constexpr (BITS == 3) {
     const bool h2 = bd[3] < y;
     const bool h1 = (h2 ? bd[5] : bd[1]) < y;
     const float t0 = h2 ? (h1 ? bd[6] : bd[4]) : (h1 ? bd[2] : bd[0]);
     return (h2 ? 4 : 0) + (h1 ? 2 : 0) + (t0 < y ? 1 : 0);
+  } else if constexpr (BITS == 4) {
+    int k = s_bd[7] < y ? 8 : 0;
+    k += s_bd[k + 3] < y ? 4 : 0;
+    k += s_bd[k + 1] < y ? 2 : 0;
+    return k + (s_bd[k] < y ? 1 : 0);
   } else {
-    const bool h3 = bd[7] < y;
-    const bool h2 = (h3 ? bd[11] : bd[3]) < y;
-    const float t1 = h3 ? (h2 ? bd[13] : bd[9]) : (h2 ? bd[5] : bd[1]);
-    const bool h1 = t1 < y;
-    const float t0 = h3 ? (h2 ? (h1 ? bd[14] : bd[12]) : (h1 ? bd[10] : bd[8]))
-                        : (h2 ? (h1 ? bd[6] : bd[4]) : (h1 ? bd[2] : bd[0]));
-    return (h3 ? 8 : 0) + (h2 ? 4 : 0) + (h1 ? 2 : 0) + (t0 < y ? 1 : 0);
+    return bucket<BITS>(y, bd);
   }
 }
+template <int BITS>
+__device__ __forceinline__ void load_bounds(const float* __restrict__ bounds, float (&bd)[(1 << BITS) - 1],
+                                            float* s_bd) {
+#pragma unroll
+  for (int i = 0; i < (1 << BITS) - 1; ++i) bd[i] = BITS < 4 ? bounds[i] : 0.f;
+  if (BITS == 4 && threadIdx.x < (1 << BITS) - 1) s_bd[threadIdx.x] = bounds[threadIdx.x];
+}
 
-// The 4-bit search of bucket_bsearch on a boundary table in LDS: the same
-// comparisons, the next boundary addressed by the bucket so far (kept in
-// registers, the selects between boundaries compile to an indexed load from a
-// private, memory-backed copy of the table).
-__device__ __forceinline__ int bucket_bsearch4_lds(float y, const float* s_bd) {
-  int k = s_bd[7] < y ? 8 : 0;
-  k += s_bd[k + 3] < y ? 4 : 0;
-  k += s_bd[k + 1] < y ? 2 : 0;
-  return k + (s_bd[k] < y ? 1 : 0);
+// The 8 codes (dims 8n ..) of row 4 (lane / 16) + i, at pack_bits(BITS) each.
+template <int BITS>
+__device__ __forceinline__ uint32_t pack_codes8(const f32x4 (&acc)[8], int i, const float (&bd)[(1 << BITS) - 1],
+                                                const float* s_bd) {
+  uint32_t v = 0;
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+    v |= static_cast<uint32_t>(bucket_fast<BITS>(acc[c][i], bd, s_bd)) << (pack_bits(BITS) * c);
+  return v;
+}
+template <int BITS>
+__device__ __forceinline__ void store_codes8(uint8_t* __restrict__ row, int n, uint32_t v) {
+  if constexpr (pack_bits(BITS) == 4)
+    *reinterpret_cast<uint32_t*>(row + 4 * n) = v;
+  else if constexpr (pack_bits(BITS) == 2)
+    *reinterpret_cast<uint16_t*>(row + 2 * n) = static_cast<uint16_t>(v);
+  else
+    row[n] = static_cast<uint8_t>(v);
 }
 
 template <int BITS, bool F16>
@@ -68,10 +127,8 @@ __global__ __launch_bounds__(kThreads, 2) void quantize_wave_kernel(const void* 
                                                                     const float* __restrict__ bounds,
                                                                     uint8_t* __restrict__ packed,
                                                                     void* __restrict__ norms) {
-  static_assert(pack_bits(BITS) == 4 && row_bytes_for(BITS) == 64, "nibble layouts only");
-  __shared__ float4 s_b[8][8][65];  // 64 KB + one float4 of padding per row: the staging writes of 8
-                                     // consecutive threads (8 k-quarters) fall in different banks
-  __shared__ float s_bd[16];        // 4-bit boundaries
+  __shared__ PiTiles s_b;
+  __shared__ float s_bd[16];  // 4-bit boundaries
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int n = lane & 15, g = lane >> 4;
   const int64_t ntiles = (M + kRows - 1) / kRows;
@@ -87,21 +144,11 @@ __global__ __launch_bounds__(kThreads, 2) void quantize_wave_kernel(const void* 
       load_row_f32(static_cast<const float*>(xin) + rl * kD + 32 * g, a);
   };
   if (tile < ntiles) load_a(tile);
-  // Pi, coalesced: thread tid holds float4 f = 256 i + tid (row f / 32, columns
-  // 4 (f % 32) ..), written to its operand slot.
-  float4 pr[kD * kD / 4 / kThreads];
-#pragma unroll
-  for (int i = 0; i < kD * kD / 4 / kThreads; ++i) pr[i] = reinterpret_cast<const float4*>(Pi)[i * kThreads + threadIdx.x];
+  float4 pr[kPiLoads];
+  load_pi_coalesced(Pi, pr);
   float bd[(1 << BITS) - 1];
-#pragma unroll
-  for (int i = 0; i < (1 << BITS) - 1; ++i) bd[i] = BITS == 3 ? bounds[i] : 0.f;
-  if (BITS == 4 && threadIdx.x < (1 << BITS) - 1) s_bd[threadIdx.x] = bounds[threadIdx.x];
-#pragma unroll
-  for (int i = 0; i < kD * kD / 4 / kThreads; ++i) {
-    const int f = i * kThreads + threadIdx.x;
-    const int j = f >> 5, c4 = f & 31;  // Pi row j = 8n' + c, columns 32q' + 4kq ..
-    s_b[j & 7][c4 & 7][16 * (c4 >> 3) + (j >> 3)] = pr[i];
-  }
+  load_bounds<BITS>(bounds, bd, s_bd);
+  stage_pi(pr, s_b);
   __syncthreads();
   for (; tile < ntiles; tile += static_cast<int64_t>(gridDim.x) * 4) {
     const int64_t row0 = tile * kRows;
@@ -116,83 +163,151 @@ __global__ __launch_bounds__(kThreads, 2) void quantize_wave_kernel(const void* 
         static_cast<float*>(norms)[r] = nrm;
     }
     f32x4 acc[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kq = 0; kq < 8; ++kq) {
-      float4 bv[8];
-#pragma unroll
-      for (int c = 0; c < 8; ++c) bv[c] = s_b[c][kq][lane];
-#pragma unroll
-      for (int cc = 0; cc < 4; ++cc) {
-        const float av = a[4 * kq + cc];
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          const float b = cc == 0 ? bv[c].x : cc == 1 ? bv[c].y : cc == 2 ? bv[c].z : bv[c].w;
-          acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b, acc[c], 0, 0, 0);
-        }
-      }
-      // keeps the next k-quarter's LDS reads after these MFMAs (the compiler
-      // otherwise hoists all 256 operand values and spills)
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    rotate_wave_tile(a, s_b, lane, acc);
     const int64_t next = tile + static_cast<int64_t>(gridDim.x) * 4;
     if (next < ntiles) load_a(next);  // in flight during the bucketing and stores
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int64_t row = row0 + 4 * g + i;
-      uint32_t v = 0;
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        const int code = BITS == 3 ? bucket_bsearch<BITS>(acc[c][i], bd) : bucket_bsearch4_lds(acc[c][i], s_bd);
-        v |= static_cast<uint32_t>(code) << (4 * c);
-      }
-      if (row < M) *reinterpret_cast<uint32_t*>(packed + row * 64 + 4 * n) = v;
+      const uint32_t v = pack_codes8<BITS>(acc, i, bd, s_bd);
+      if (row < M) store_codes8<BITS>(packed + row * row_bytes_for(BITS), n, v);
     }
   }
 }
 
-template <int BITS, bool F16>
-__global__ __launch_bounds__(kThreads) void quantize_kernel(const void* __restrict__ xin, int64_t M,
-                                                            const float* __restrict__ Pi,
-                                                            const float* __restrict__ bounds,
-                                                            uint8_t* __restrict__ packed,
-                                                            void* __restrict__ norms) {
-  __shared__ uint8_t s_codes[kRows * kD];
+// -------------------------------------------------------------- bulk update
+// S > 1 new tokens of a cache layer (keys in grid row y = 0, values in y = 1),
+// one launch: the tokens that leave the fp16 window -- of positions c0 .. c1 - 1,
+// some still in the ring, the others new -- are quantized into the cold store,
+// and the newest tokens enter the ring.  fp16 rows are widened to fp32 before
+// the norm and the division (cache.py:141), so the codes and norms are
+// lkv_tq_quantize's of the widened rows, bit for bit.
+//
+// Tiles of 16 rows run over all evicted tokens of all R (batch, kv head) rows,
+// row = (cache row) * (c1 - c0) + token, as in quantize_wave_kernel.  A ring
+// slot whose token is quantized here always takes a new token: the lane that
+// loaded 64 bytes of the old token writes the same 64 bytes of the new one after
+// they arrived, so no slot is written before it was read.  New tokens whose
+// slot held none are copied first, by all threads.
+//
+// Bound by the fp32 MFMA chains (13.4 us for the 2 x 32 K vectors of a 4096-token
+// prompt layer at 154 TFLOP/s); it reads fp16 rows where they are (any row
+// strides) and writes the cache in place.  Measured against two widening
+// copies, two quantize launches, four strided copies into the store, index
+// arithmetic and two ring scatters per layer update: a 4096-token prompt layer
+// (8 kv heads, update and attention) 304 -> 244 us, four prompts of 1201
+// tokens in three chunks 536 -> 241 us.
+struct BulkSide {
+  const uint16_t* x;  // [R / H][H][S] rows of 128, strides sb, sh, ss (elements)
+  int64_t sb, sh, ss;
+  uint16_t* hot;      // [R][hot_cap][128]
+  uint8_t* codes;     // [R][cap][row bytes]
+  float* norms;       // [R][cap]
+  const float* Pi;
+};
+struct BulkArgs {
+  BulkSide side[2];
+  const float* bounds;
+  int64_t cap;
+  uint32_t R, H, p0, T, c0, c1, hot_cap;  // 32 bits: the kernel divides by several of them per row
+};
+template <int BITS>
+__global__ __launch_bounds__(kThreads, 2) void bulk_update_kernel(BulkArgs P) {
+  __shared__ PiTiles s_b;
+  __shared__ float s_bd[16];
+  const BulkSide& W = P.side[blockIdx.y];
+  const uint16_t* __restrict__ x = W.x;
+  const int64_t sb = W.sb, sh = W.sh, ss = W.ss;
+  const uint32_t hot_cap = P.hot_cap, p0 = P.p0, T = P.T, c0 = P.c0;
+  uint16_t* const hot = W.hot;
+  auto src_new = [&](uint32_t row, uint32_t t) {  // token t >= p0 of cache row `row`
+    return x + (row / P.H) * sb + (row % P.H) * sh + (t - p0) * ss;
+  };
+  auto slot_at = [&](uint32_t row, uint32_t slot) { return hot + (static_cast<size_t>(row) * hot_cap + slot) * kD; };
+  // ---- new tokens into ring slots that held no token: none once the window
+  // was full, else slots p0 % hot_cap .. hot_cap - 1
+  if (p0 < hot_cap) {
+    const uint32_t first = T > hot_cap && T - hot_cap > p0 ? T - hot_cap : p0;  // the newest min(S, hot_cap) tokens
+    const uint32_t ncopy = min(T, hot_cap) - p0;                                // slots p0 .. : one token each
+    const uint32_t total = P.R * ncopy;
+    const uint32_t c = threadIdx.x & 15;
+    for (uint32_t i = blockIdx.x * (kThreads / 16) + (threadIdx.x >> 4); i < total; i += gridDim.x * (kThreads / 16)) {
+      const uint32_t row = i / ncopy, slot = p0 + i % ncopy;
+      const uint32_t t = first + (slot + hot_cap - first % hot_cap) % hot_cap;  // the window's token of this slot
+      *reinterpret_cast<uint4*>(slot_at(row, slot) + 8 * c) =
+          *reinterpret_cast<const uint4*>(src_new(row, t) + 8 * c);
+    }
+  }
+  const uint32_t nq = P.c1 - c0, M = P.R * nq;
+  if (M == 0) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  float bd[(1 << BITS) - 1];
-#pragma unroll
-  for (int i = 0; i < (1 << BITS) - 1; ++i) bd[i] = bounds[i];
-  float b[2][32];
-  load_pi_operand(Pi, false, wave, lane, b);
-  const int64_t ntiles = (M + kRows - 1) / kRows;
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t row0 = tile * kRows;
-    const int64_t r = row0 + (lane & 15);
-    float a[32];
-    if (r < M) {
-      if (F16)
-        load_row_f16(static_cast<const uint16_t*>(xin) + r * kD + 32 * (lane >> 4), a);
-      else
-        load_row_f32(static_cast<const float*>(xin) + r * kD + 32 * (lane >> 4), a);
+  const int n = lane & 15, g = lane >> 4;
+  const uint32_t ntiles = (M + kRows - 1) / kRows;
+  uint32_t tile = blockIdx.x * 4 + wave;
+  uint4 raw[4];             // dims 32 g .. of the lane's row, fp16
+  uint16_t* slot_p = nullptr;       // the row's ring slot (dims 32 g ..) when it is a ring token
+  const uint16_t* refill = nullptr;  // and the new token that takes it
+  auto load_a = [&](uint32_t tl) {
+    const uint32_t r = tl * kRows + n;
+    const uint32_t rl = min(r, M - 1);  // rows past M read row M - 1 and are zeroed after
+    const uint32_t row = rl / nq, t = c0 + rl % nq;
+    const uint16_t* src;
+    slot_p = nullptr;
+    if (t < p0) {
+      uint16_t* s = slot_at(row, t % hot_cap) + 32 * g;
+      src = s;
+      if (r < M) {
+        slot_p = s;
+        refill = src_new(row, t + (T - 1 - t) / hot_cap * hot_cap) + 32 * g;
+      }
     } else {
+      src = src_new(row, t) + 32 * g;
+    }
 #pragma unroll
-      for (int s = 0; s < 32; ++s) a[s] = 0.f;
+    for (int v = 0; v < 4; ++v) raw[v] = reinterpret_cast<const uint4*>(src)[v];
+  };
+  if (tile < ntiles) load_a(tile);
+  float4 pr[kPiLoads];
+  load_pi_coalesced(W.Pi, pr);
+  float bd[(1 << BITS) - 1];
+  load_bounds<BITS>(P.bounds, bd, s_bd);
+  stage_pi(pr, s_b);
+  __syncthreads();
+  uint8_t* __restrict__ codes = W.codes;
+  float* __restrict__ norms = W.norms;
+  auto cold_row = [&](uint32_t r) { return static_cast<int64_t>(r / nq) * P.cap + c0 + r % nq; };
+  for (; tile < ntiles; tile += gridDim.x * 4) {
+    const uint32_t row0 = tile * kRows;
+    const uint32_t r = row0 + n;
+    float a[32];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const uint32_t w[4] = {raw[v].x, raw[v].y, raw[v].z, raw[v].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        a[8 * v + 2 * i] = r < M ? h2f(static_cast<uint16_t>(w[i] & 0xffffu)) : 0.f;
+        a[8 * v + 2 * i + 1] = r < M ? h2f(static_cast<uint16_t>(w[i] >> 16)) : 0.f;
+      }
     }
-    const float nrm = normalize_row<F16>(a);
-    if (wave == 0 && lane < 16 && r < M) {
-      if (F16)
-        static_cast<uint16_t*>(norms)[r] = f2h(nrm);
-      else
-        static_cast<float*>(norms)[r] = nrm;
+    const float nrm = normalize_row<false>(a);
+    if (slot_p) {  // the old token is in registers (the norm has used it)
+      uint4 nw[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) nw[v] = reinterpret_cast<const uint4*>(refill)[v];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) reinterpret_cast<uint4*>(slot_p)[v] = nw[v];
     }
-    f32x4 acc[2];
-    rotate_tile(a, b, acc);
-    codes_to_lds<BITS>(acc, bd, wave, lane, s_codes);
-    __syncthreads();
-    pack_store<BITS>(s_codes, packed, row0, M,
-                     [](int64_t rr) { return rr * static_cast<int64_t>(row_bytes_for(BITS)); });
-    __syncthreads();
+    if (g == 0 && r < M) norms[cold_row(r)] = nrm;
+    f32x4 acc[8];
+    rotate_wave_tile(a, s_b, lane, acc);
+    const uint32_t next = tile + gridDim.x * 4;
+    if (next < ntiles) load_a(next);  // in flight during the bucketing and stores
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t rr = row0 + 4 * g + i;
+      const uint32_t v = pack_codes8<BITS>(acc, i, bd, s_bd);
+      if (rr < M) store_codes8<BITS>(codes + cold_row(rr) * row_bytes_for(BITS), n, v);
+    }
   }
 }
 
@@ -416,30 +531,14 @@ extern "C" int lkv_tq_quantize(const void* x, int x_dtype, int64_t M, const floa
   LKV_REQUIRE(aligned16(x) && aligned16(Pi) && aligned4(packed),
               "tq_quantize: x and Pi must be 16-byte aligned, packed 4-byte aligned");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (bits >= 3) {  // nibble layouts: one wave per 16-vector tile
-    const int64_t ntiles = (M + kRows - 1) / kRows;
-    const int64_t cap = 2 * static_cast<int64_t>(device_cu_count());  // 64 KB of LDS: 2 blocks per CU
-    const int gw = static_cast<int>(std::min<int64_t>((ntiles + 3) / 4, cap));
-    if (x_dtype == LKV_DTYPE_F16) {
-      if (bits == 3)
-        hipLaunchKernelGGL((quantize_wave_kernel<3, true>), dim3(gw), dim3(kThreads), 0, st, x, M, Pi, bounds, packed, norms);
-      else
-        hipLaunchKernelGGL((quantize_wave_kernel<4, true>), dim3(gw), dim3(kThreads), 0, st, x, M, Pi, bounds, packed, norms);
-    } else {
-      if (bits == 3)
-        hipLaunchKernelGGL((quantize_wave_kernel<3, false>), dim3(gw), dim3(kThreads), 0, st, x, M, Pi, bounds, packed, norms);
-      else
-        hipLaunchKernelGGL((quantize_wave_kernel<4, false>), dim3(gw), dim3(kThreads), 0, st, x, M, Pi, bounds, packed, norms);
-    }
-    LKV_LAUNCH_CHECK("tq_quantize");
-    return LKV_OK;
-  }
-  const int g = grid_for(M);
+  const int64_t ntiles = (M + kRows - 1) / kRows;  // one wave per 16-vector tile
+  const int64_t cap = 2 * static_cast<int64_t>(device_cu_count());  // 66 KB of LDS: 2 blocks per CU
+  const int g = static_cast<int>(std::min<int64_t>((ntiles + 3) / 4, cap));
   if (x_dtype == LKV_DTYPE_F16) {
-    LKV_BITS_SWITCH(bits, hipLaunchKernelGGL((quantize_kernel<B_, true>), dim3(g), dim3(kThreads), 0, st,
+    LKV_BITS_SWITCH(bits, hipLaunchKernelGGL((quantize_wave_kernel<B_, true>), dim3(g), dim3(kThreads), 0, st,
                                              x, M, Pi, bounds, packed, norms))
   } else {
-    LKV_BITS_SWITCH(bits, hipLaunchKernelGGL((quantize_kernel<B_, false>), dim3(g), dim3(kThreads), 0, st,
+    LKV_BITS_SWITCH(bits, hipLaunchKernelGGL((quantize_wave_kernel<B_, false>), dim3(g), dim3(kThreads), 0, st,
                                              x, M, Pi, bounds, packed, norms))
   }
   LKV_LAUNCH_CHECK("tq_quantize");
@@ -540,5 +639,64 @@ extern "C" int lkv_tq_cache_append(const void* k_new, const void* v_new, void* k
                                            static_cast<uint16_t*>(k_hot), static_cast<uint16_t*>(v_hot), k_codes,
                                            k_norms, v_codes, v_norms, PiK, PiV, bounds, pos, R, hot_cap, cap))
   LKV_LAUNCH_CHECK("tq_cache_append");
+  return LKV_OK;
+}
+
+extern "C" int lkv_tq_cache_bulk_update(const void* k_new, const int64_t* k_strides, const void* v_new,
+                                        const int64_t* v_strides, int64_t B, int64_t H, int64_t S, int64_t p0,
+                                        void* k_hot, void* v_hot, uint8_t* k_codes, float* k_norms, uint8_t* v_codes,
+                                        float* v_norms, const float* PiK, const float* PiV, const float* bounds,
+                                        int bits, int64_t hot_cap, int64_t cap, void* stream) {
+  const char* who = "tq_cache_bulk_update";
+  if (int e = check_bits(bits, who)) return e;
+  LKV_REQUIRE(B >= 0 && H >= 0 && S >= 0 && p0 >= 0 && hot_cap >= 1 && cap >= 0,
+              "%s: bad sizes B=%lld H=%lld S=%lld p0=%lld hot_cap=%lld cap=%lld", who, (long long)B, (long long)H,
+              (long long)S, (long long)p0, (long long)hot_cap, (long long)cap);
+  if (B == 0 || H == 0 || S == 0) return LKV_OK;
+  LKV_REQUIRE(p0 < (1ll << 30) && S < (1ll << 30) && hot_cap < (1ll << 30) && B < (1ll << 31) && H < (1ll << 31) &&
+                  B * H < (1ll << 31) && B * H * (S + hot_cap) < (1ll << 31),
+              "%s: problem too large", who);
+  const int64_t T = p0 + S, c0 = std::max<int64_t>(0, p0 - hot_cap), c1 = std::max<int64_t>(0, T - hot_cap);
+  LKV_REQUIRE(c1 <= cap, "%s: %lld cold tokens exceed cap=%lld", who, (long long)c1, (long long)cap);
+  LKV_REQUIRE(k_new && k_strides && v_new && v_strides && k_hot && v_hot && k_codes && k_norms && v_codes &&
+                  v_norms && PiK && PiV && bounds,
+              "%s: null pointer", who);
+  LKV_REQUIRE(aligned16(k_new) && aligned16(v_new) && aligned16(k_hot) && aligned16(v_hot) && aligned16(PiK) &&
+                  aligned16(PiV) && aligned4(k_codes) && aligned4(v_codes),
+              "%s: fp16 rows and Pi must be 16-byte aligned, codes 4-byte aligned", who);
+  BulkArgs P{};
+  const int64_t* strides[2] = {k_strides, v_strides};
+  for (int w = 0; w < 2; ++w) {
+    for (int i = 0; i < 3; ++i)
+      LKV_REQUIRE(strides[w][i] % 8 == 0, "%s: row stride %lld breaks the 16-byte alignment of rows", who,
+                  (long long)strides[w][i]);
+    BulkSide& W = P.side[w];
+    W.x = static_cast<const uint16_t*>(w ? v_new : k_new);
+    W.sb = strides[w][0];
+    W.sh = strides[w][1];
+    W.ss = strides[w][2];
+    W.hot = static_cast<uint16_t*>(w ? v_hot : k_hot);
+    W.codes = w ? v_codes : k_codes;
+    W.norms = w ? v_norms : k_norms;
+    W.Pi = w ? PiV : PiK;
+  }
+  P.bounds = bounds;
+  P.cap = cap;
+  P.R = static_cast<uint32_t>(B * H);
+  P.H = static_cast<uint32_t>(H);
+  P.p0 = static_cast<uint32_t>(p0);
+  P.T = static_cast<uint32_t>(T);
+  P.c0 = static_cast<uint32_t>(c0);
+  P.c1 = static_cast<uint32_t>(c1);
+  P.hot_cap = static_cast<uint32_t>(hot_cap);
+  // a wave per 16-row tile of one side, or a block per 16 rows of ring copies where those are the most; both
+  // sides together fill the 2 blocks per CU that the staged matrix leaves room for
+  const int64_t ntiles = (B * H * (c1 - c0) + kRows - 1) / kRows;
+  const int64_t copies = p0 < hot_cap ? B * H * (std::min(T, hot_cap) - p0) : 0;
+  const int64_t want = std::max<int64_t>({(ntiles + 3) / 4, (copies + 15) / 16, int64_t(1)});
+  const unsigned g = static_cast<unsigned>(std::min<int64_t>(want, device_cu_count()));
+  LKV_BITS_SWITCH(bits, hipLaunchKernelGGL((bulk_update_kernel<B_>), dim3(g, 2), dim3(kThreads), 0,
+                                           static_cast<hipStream_t>(stream), P))
+  LKV_LAUNCH_CHECK(who);
   return LKV_OK;
 }

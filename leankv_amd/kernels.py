@@ -12,6 +12,7 @@ the dispatcher; the Python entry points below skip the dispatcher.
 
 from __future__ import annotations
 
+import ctypes
 import math
 
 import torch
@@ -113,8 +114,6 @@ def sparse_gemm_batched_multi_out(x: torch.Tensor, weights, thresholds, outs, ep
     EPI_SWIGLU (two products g, u of one shape: outs[0] = fp16(fp16(silu(fp16 g)) * fp16 u)), EPI_RESIDUAL
     (one product: outs[0] = fp16(residual + fp16 product); outs[0] may be residual) or EPI_ROPE (q, k[, v]:
     rope_f16_ on the first two products' heads of 128 dims with the position's fp16 factors cos / sin [128])."""
-    import ctypes
-
     n = len(weights)
     if not 1 <= n <= 3 or len(thresholds) != n:
         raise LeanKVError("sparse_gemm_batched_multi: 1 to 3 weights with one threshold each")
@@ -201,8 +200,6 @@ def sparse_gemm_batched_qkv_rope_out(x: torch.Tensor, weights, cos: torch.Tensor
     EPI_ROPE), and with k_hot / v_hot [B * Hkv, hot_cap, 128] the new token of every row also written into ring
     slot pos % hot_cap (pos_dev: int32 device position), as lkv_tq_cache_append writes it
     (lkv_sparse_gemm_batched_qkv_rope)."""
-    import ctypes
-
     if len(weights) != 3 or len(outs) != 3:
         raise LeanKVError("sparse_gemm_batched_qkv_rope: q, k and v weights and outputs")
     shapes = [colmajor_rows(w) for w in weights]
@@ -326,8 +323,6 @@ def sparse_qkv(x: torch.Tensor, wq: torch.Tensor, wk: torch.Tensor, wv: torch.Te
         if o.dtype != torch.float16 or o.numel() != n or not o.is_contiguous():
             raise LeanKVError("sparse_qkv: outputs must be contiguous float16 with %s elements" % (Ns,))
     lib = _lib_handle()
-    import ctypes
-
     n_arr = (ctypes.c_int64 * 3)(*Ns)
     nbytes = lib.lkv_sparse_gemv_multi_workspace_bytes(3, n_arr, Z)
     ws = workspaces.get(x.device, "qkv", nbytes)
@@ -533,13 +528,49 @@ def tq_cache_append(k_new, v_new, k_hot, v_hot, k_codes, k_norms, v_codes, v_nor
     )
 
 
+def _row_strided(t: torch.Tensor) -> torch.Tensor:
+    """t itself where its last-dim rows are dense, 16-byte aligned and a multiple of 16 bytes apart, else a copy."""
+    if t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % 8 == 0 for s in t.stride()[:-1]):
+        return t
+    return t.contiguous()
+
+
+def tq_cache_bulk_update(k_new, v_new, p0: int, k_hot, v_hot, k_codes, k_norms, v_codes, v_norms, PiK, PiV, bounds,
+                         bits: int) -> None:
+    """S new tokens k_new, v_new fp16 [B, H, S, 128] (any row strides) appended at position p0 to one layer's static
+    ring layout, keys and values in one launch (lkv_tq_cache_bulk_update): the tokens leaving the window are
+    quantized into the cold rows, the newest take their ring slots."""
+    require_cuda(k_new, v_new, k_hot, v_hot, k_codes, v_codes)
+    if k_new.dim() != 4 or k_new.shape[-1] != HEAD_DIM or v_new.shape != k_new.shape:
+        raise LeanKVError("tq_cache_bulk_update: k_new and v_new must be alike, [B, H, S, %d]" % HEAD_DIM)
+    if k_new.dtype != torch.float16 or v_new.dtype != torch.float16:
+        raise LeanKVError("tq_cache_bulk_update: k_new and v_new must be float16")
+    B, H, S, _ = k_new.shape
+    hot_cap, cap, rb = k_hot.shape[-2], k_codes.shape[-2], packed_row_bytes(bits)
+    for t, nm, dt, n in ((k_hot, "k_hot", torch.float16, hot_cap * HEAD_DIM), (k_codes, "k_codes", torch.uint8, cap * rb),
+                         (k_norms, "k_norms", torch.float32, cap), (v_hot, "v_hot", torch.float16, hot_cap * HEAD_DIM),
+                         (v_codes, "v_codes", torch.uint8, cap * rb), (v_norms, "v_norms", torch.float32, cap)):
+        if t.dtype != dt or not t.is_contiguous() or t.numel() != B * H * n:
+            raise LeanKVError("tq_cache_bulk_update: %s must be contiguous %s of %d rows" % (nm, dt, B * H))
+    dev = k_new.device
+    k_new, v_new = _row_strided(k_new), _row_strided(v_new)
+    PiK, PiV = _pi(PiK, dev), _pi(PiV, dev)
+    bounds = _vec(bounds, dev, (1 << bits) - 1, "decision boundaries")
+    strides = ctypes.c_int64 * 3
+    check(
+        _lib_handle().lkv_tq_cache_bulk_update(ptr(k_new), strides(*k_new.stride()[:3]), ptr(v_new),
+                                               strides(*v_new.stride()[:3]), B, H, S, int(p0), ptr(k_hot), ptr(v_hot),
+                                               ptr(k_codes), ptr(k_norms), ptr(v_codes), ptr(v_norms), ptr(PiK),
+                                               ptr(PiV), ptr(bounds), int(bits), hot_cap, cap, stream_handle(dev)),
+        "lkv_tq_cache_bulk_update",
+    )
+
+
 def tq_cache_evict(layers, bounds, bits: int, pos_dev: torch.Tensor) -> None:
     """The eviction half of tq_cache_append for every layer in one launch (lkv_tq_cache_evict): layers is a list
     of (k_codes, k_norms, v_codes, v_norms, k_hot, v_hot, PiK, PiV) on the static ring layout, R = B x kv heads
     rows each; the token at position pos_dev - hot_cap leaves ring slot pos_dev % hot_cap for cold slot
     pos_dev - hot_cap.  Run before the step's ring write."""
-    import ctypes
-
     class _Layer(ctypes.Structure):
         _fields_ = [(n, ctypes.c_void_p) for n in ("k_codes", "k_norms", "v_codes", "v_norms", "k_hot", "v_hot",
                                                    "PiK", "PiV")]

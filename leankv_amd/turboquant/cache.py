@@ -97,16 +97,24 @@ class TurboQuantCache:
         self.storage_generation = 0
 
     # ----------------------------------------------------------- storage
+    def _zeros(self, *specs) -> list:
+        """Zeroed tensors of (shape, dtype) as 256-byte-aligned parts of one buffer, cleared by one launch (a queued
+        launch costs ~4.5 us however small).  Tensors replaced together when the store grows share a buffer."""
+        sizes = [math.prod(shape) * dtype.itemsize for shape, dtype in specs]
+        at = [0]
+        for n in sizes:
+            at.append(at[-1] + -(-n // 256) * 256)
+        buf = torch.zeros(at[-1], dtype=torch.uint8, device=self._device)
+        return [buf[o:o + n].view(dtype).view(shape) for o, n, (shape, dtype) in zip(at, sizes, specs)]
+
     def _alloc(self, layer: int, B: int, H: int, cap: int) -> None:
-        dev = self._device
-        self._k_codes[layer] = torch.zeros(B, H, cap, self._row_bytes, dtype=torch.uint8, device=dev)
-        self._v_codes[layer] = torch.zeros(B, H, cap, self._row_bytes, dtype=torch.uint8, device=dev)
-        self._k_norms[layer] = torch.zeros(B, H, cap, dtype=torch.float32, device=dev)
-        self._v_norms[layer] = torch.zeros(B, H, cap, dtype=torch.float32, device=dev)
-        self._k_hot[layer] = torch.zeros(B, H, self.hot_buffer_size, self.head_dim, dtype=torch.float16, device=dev)
-        self._v_hot[layer] = torch.zeros_like(self._k_hot[layer])
-        self._pos_dev[layer] = torch.zeros(1, dtype=torch.int32, device=dev)
-        self._len_dev[layer] = torch.zeros(1, dtype=torch.int32, device=dev)
+        rows = (B, H, cap)
+        (self._k_codes[layer], self._v_codes[layer], self._k_norms[layer], self._v_norms[layer]) = self._zeros(
+            ((*rows, self._row_bytes), torch.uint8), ((*rows, self._row_bytes), torch.uint8), (rows, torch.float32),
+            (rows, torch.float32))
+        ring = ((B, H, self.hot_buffer_size, self.head_dim), torch.float16)
+        (self._k_hot[layer], self._v_hot[layer], self._pos_dev[layer], self._len_dev[layer]) = self._zeros(
+            ring, ring, ((1,), torch.int32), ((1,), torch.int32))
         self.storage_generation += 1
 
     def _ensure_cap(self, layer: int, cold_needed: int) -> None:
@@ -179,38 +187,10 @@ class TurboQuantCache:
         return self._get_full_cache(layer_idx)
 
     def _bulk_update(self, li: int, k16: torch.Tensor, v16: torch.Tensor, p0: int) -> None:
-        """Append S > 1 tokens: quantize every token that leaves the hot window, refill the ring.
-
-        One gather of the ring slots that leave it and one scatter of the new window per layer (slot
-        indices made on the device, no per-slot copies)."""
-        hot = self.hot_buffer_size
-        dev = self._device
-        S = k16.shape[2]
-        T = p0 + S
-        c0, c1 = self._cold_len(p0), self._cold_len(T)
-        if c1 > c0:
-            # tokens [c0, c1) in position order: some still in the ring, the rest new
-            fk = fv = None
-            if min(c1, p0) > c0:
-                slots = torch.arange(c0, min(c1, p0), device=dev) % hot
-                fk = self._k_hot[li].index_select(2, slots)
-                fv = self._v_hot[li].index_select(2, slots)
-            if c1 > p0:
-                nk, nv = k16[:, :, : c1 - p0], v16[:, :, : c1 - p0]
-                fk = nk if fk is None else torch.cat([fk, nk], dim=2)
-                fv = nv if fv is None else torch.cat([fv, nv], dim=2)
-            pk, nk_ = torch.ops.leankv.tq_quantize(fk.float().contiguous(), self.PiK[li], self.decision_boundaries,
-                                                   self.bits)
-            pv, nv_ = torch.ops.leankv.tq_quantize(fv.float().contiguous(), self.PiV[li], self.decision_boundaries,
-                                                   self.bits)
-            self._k_codes[li][:, :, c0:c1] = pk
-            self._v_codes[li][:, :, c0:c1] = pv
-            self._k_norms[li][:, :, c0:c1] = nk_
-            self._v_norms[li][:, :, c0:c1] = nv_
-        first = max(p0, T - hot)  # the newest min(S, hot) tokens enter the ring, each in slot p % hot
-        slots = torch.arange(first, T, device=dev) % hot
-        self._k_hot[li].index_copy_(2, slots, k16[:, :, first - p0:])
-        self._v_hot[li].index_copy_(2, slots, v16[:, :, first - p0:])
+        """Append S > 1 tokens: quantize every token that leaves the hot window, refill the ring (one launch)."""
+        _k.tq_cache_bulk_update(k16, v16, p0, self._k_hot[li], self._v_hot[li], self._k_codes[li], self._k_norms[li],
+                                self._v_codes[li], self._v_norms[li], self.PiK[li], self.PiV[li],
+                                self.decision_boundaries, self.bits)
 
     def _get_full_cache(self, layer_idx: int):
         """cat(dequantize(cold).fp16, hot) in position order (cache.py:169-189)."""

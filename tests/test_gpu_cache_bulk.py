@@ -1,0 +1,74 @@
+"""lkv_tq_cache_bulk_update: S new tokens of one layer in one launch (leankv/turboquant/cache.py:84-159).
+
+Expected contents come from a token-by-token restatement: tokens below T - hot are quantized (lkv_tq_quantize of
+the fp16 rows widened to fp32, the same arithmetic, so bytes and norms are equal bit for bit), the others sit in ring
+slot p % hot."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# (p0, S, hot): empty window, part-filled and full; fewer and more new tokens than the window; tile edges
+SHAPES = [(0, 2, 64), (0, 64, 64), (0, 65, 64), (0, 333, 64), (1, 63, 64), (40, 30, 64), (40, 300, 64), (63, 17, 64),
+          (64, 2, 64), (64, 64, 64), (70, 63, 64), (130, 200, 64), (5, 3, 1), (0, 5, 1), (250, 16, 256), (300, 31, 16)]
+
+
+@pytest.mark.parametrize("bits", [1, 2, 3, 4])
+@pytest.mark.parametrize("p0,S,hot", SHAPES)
+def test_bulk_update_equals_token_by_token(p0, S, hot, bits):
+    from leankv_amd import kernels as K
+    from leankv_amd.turboquant.codebook import get_codebook_tensors
+    from leankv_amd.turboquant.rotation import generate_rotation_matrix
+
+    dev, B, H, D = "cuda", 2, 3, 128
+    T, rb = p0 + S, K.packed_row_bytes(bits)
+    cap = max(1, T - hot) + 5
+    g = torch.Generator().manual_seed(7 * p0 + S + bits)
+    bounds = get_codebook_tensors(D, bits, dev)[1][1:-1].contiguous()
+    sides = []
+    for j in range(2):
+        x = torch.randn(B, H, T, D, generator=g).half().to(dev)
+        x[0, 0, T // 2] = 0
+        pi = generate_rotation_matrix(D, dev, seed=42 + j)
+        codes, norms = K.tq_quantize(x.float(), pi, bounds, bits)
+        hotb = torch.full((B, H, hot, D), 9.0, dtype=torch.float16, device=dev)
+        for p in range(max(0, p0 - hot), p0):
+            hotb[:, :, p % hot] = x[:, :, p]
+        new = x[:, :, p0:]
+        # the layouts attention hands over: a transposed [B, S, H, D] view, and a slice of a longer tensor
+        new = new.transpose(1, 2).contiguous().transpose(1, 2) if j else new
+        want = hotb.clone()
+        for p in range(max(p0, T - hot), T):
+            want[:, :, p % hot] = x[:, :, p]
+        sides.append(dict(new=new, pi=pi, codes=codes, norms=norms, hot=hotb, want=want,
+                          c=torch.full((B, H, cap, rb), 0xA5, dtype=torch.uint8, device=dev),
+                          n=torch.full((B, H, cap), -7.0, device=dev)))
+    k, v = sides
+    K.tq_cache_bulk_update(k["new"], v["new"], p0, k["hot"], v["hot"], k["c"], k["n"], v["c"], v["n"], k["pi"], v["pi"],
+                           bounds, bits)
+    c0, c1 = max(0, p0 - hot), max(0, T - hot)
+    for s in sides:
+        assert torch.equal(s["hot"], s["want"])
+        assert torch.equal(s["c"][:, :, c0:c1], s["codes"][:, :, c0:c1])
+        assert torch.equal(s["n"][:, :, c0:c1], s["norms"][:, :, c0:c1])
+        for t, fill in ((s["c"], 0xA5), (s["n"], -7.0)):  # nothing else of the store is written
+            assert bool((t[:, :, :c0] == fill).all()) and bool((t[:, :, c1:] == fill).all())
+
+
+def test_bulk_update_refuses_bad_calls():
+    from leankv_amd import kernels as K
+    from leankv_amd._lib import LeanKVError
+
+    def call(S=4, p0=62, cap=8, dtype=torch.float16, hot=64):
+        z = lambda *s, dt=torch.float16: torch.zeros(*s, dtype=dt, device="cuda")  # noqa: E731
+        x = z(1, 1, S, 128, dt=dtype)
+        K.tq_cache_bulk_update(x, x, p0, z(1, 1, hot, 128), z(1, 1, hot, 128), z(1, 1, cap, 64, dt=torch.uint8),
+                               z(1, 1, cap, dt=torch.float32), z(1, 1, cap, 64, dt=torch.uint8),
+                               z(1, 1, cap, dt=torch.float32), z(128, 128, dt=torch.float32),
+                               z(128, 128, dt=torch.float32), z(7, dt=torch.float32), 3)
+
+    call()
+    with pytest.raises(LeanKVError):
+        call(S=20)  # 18 cold tokens do not fit 8 rows
+    with pytest.raises(LeanKVError):
+        call(dtype=torch.float32)
