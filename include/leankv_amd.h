@@ -311,6 +311,20 @@ int lkv_tq_cache_bulk_update(const void* k_new, const int64_t* k_strides, const 
                              int64_t hot_cap, int64_t cap, void* stream);
 
 /*
+ * TurboQuantCache._get_full_cache for one layer (leankv/turboquant/
+ * cache.py:169-189): K and V of tokens 0 .. n - 1 in position order, fp16
+ * [R, n, 128] (R = batch * kv_heads): tokens below n - hot_cap dequantized
+ * (x_hat = (centroids[codes] @ Pi) * norm in fp32, rounded to fp16), the
+ * others from their ring slots.  Layout as for lkv_tq_cache_append; codes,
+ * rings, Pi and outputs 16-byte aligned.  Refused if n - hot_cap > cap.
+ * Needs R * n < 2^31.
+ */
+int lkv_tq_cache_read(const uint8_t* k_codes, const float* k_norms, const uint8_t* v_codes, const float* v_norms,
+                      const void* k_hot, const void* v_hot, const float* PiK, const float* PiV,
+                      const float* centroids, int bits, int64_t R, int64_t n, int64_t cap, int64_t hot_cap,
+                      void* k_out, void* v_out, void* stream);
+
+/*
  * Decode-step cache append of TurboQuantCache.update for one layer
  * (leankv/turboquant/cache.py:84-159) on a static ring layout.
  * Current length before the append is *pos (device int32, read by the

@@ -54,6 +54,8 @@ SIGNATURES = {
                                    _c_p, _i64, _i64, _i64, _c_p]),
     "lkv_tq_cache_bulk_update": (_int, [_c_p, _c_p, _c_p, _c_p, _i64, _i64, _i64, _i64, _c_p, _c_p, _c_p, _c_p, _c_p,
                                         _c_p, _c_p, _c_p, _c_p, _int, _i64, _i64, _c_p]),
+    "lkv_tq_cache_read": (_int, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _int, _i64, _i64, _i64, _i64, _c_p,
+                                 _c_p, _c_p]),
     "lkv_tq_decode_attn_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),
     "lkv_tq_decode_attn": (_int, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _int, _c_p,
                                   _i64, _i64, _i64, _i64, _i64, _i64, _f32, _c_p, _c_p, _sz, _c_p]),

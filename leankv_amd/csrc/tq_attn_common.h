@@ -67,6 +67,46 @@ __device__ __forceinline__ void decode_half(uint32_t w, int half, const uint32_t
   }
 }
 
+// Code rows of stored width CB (4: nibbles, 64 B per token; 2: four codes per
+// byte; 1: eight per byte) widened to nibble dwords as they are loaded, so the
+// decode after the load is the nibble one (bits 1 and 2 through the v_perm
+// table, zero-padded past 2^bits centroids).
+__device__ __forceinline__ uint32_t nib2(uint32_t x) {  // 8 two-bit codes -> 8 nibbles
+  uint32_t t = x & 0xffffu;
+  t = (t | (t << 8)) & 0x00ff00ffu;
+  t = (t | (t << 4)) & 0x0f0f0f0fu;
+  return (t | (t << 2)) & 0x33333333u;
+}
+__device__ __forceinline__ uint32_t nib1(uint32_t x) {  // 8 one-bit codes -> 8 nibbles
+  uint32_t t = x & 0xffu;
+  t = (t | (t << 12)) & 0x000f000fu;
+  t = (t | (t << 6)) & 0x03030303u;
+  return (t | (t << 3)) & 0x11111111u;
+}
+// dims 32k .. 32k + 31 of a row whose code bytes start at p (row byte 4 CB k)
+template <int CB>
+__device__ __forceinline__ uint4 codes32(const uint8_t* p) {
+  if constexpr (CB == 4) {
+    return *reinterpret_cast<const uint4*>(p);
+  } else if constexpr (CB == 2) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    return uint4{nib2(v.x), nib2(v.x >> 16), nib2(v.y), nib2(v.y >> 16)};
+  } else {
+    const uint32_t v = *reinterpret_cast<const uint32_t*>(p);
+    return uint4{nib1(v), nib1(v >> 8), nib1(v >> 16), nib1(v >> 24)};
+  }
+}
+// dims 8k .. 8k + 7 (row byte CB k)
+template <int CB>
+__device__ __forceinline__ uint32_t codes8(const uint8_t* p) {
+  if constexpr (CB == 4)
+    return *reinterpret_cast<const uint32_t*>(p);
+  else if constexpr (CB == 2)
+    return nib2(*reinterpret_cast<const uint16_t*>(p));
+  else
+    return nib1(*p);
+}
+
 __device__ __forceinline__ float vmax(float a, float b) {
   float r;
   asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));

@@ -566,6 +566,33 @@ def tq_cache_bulk_update(k_new, v_new, p0: int, k_hot, v_hot, k_codes, k_norms, 
     )
 
 
+def tq_cache_read(k_codes, k_norms, v_codes, v_norms, k_hot, v_hot, PiK, PiV, centroids, bits: int, n: int):
+    """(K, V) fp16 [B, H, n, 128] of one layer's static ring layout in position order, one launch
+    (lkv_tq_cache_read): cold tokens dequantized, the newest min(n, hot) from their ring slots."""
+    require_cuda(k_codes, v_codes, k_hot, v_hot)
+    B, H, cap, rb = k_codes.shape
+    hot_cap = k_hot.shape[-2]
+    _check_code_rows(k_codes, v_codes, bits, "tq_cache_read")
+    for t, nm, dt, m in ((k_codes, "k_codes", torch.uint8, cap * rb), (v_codes, "v_codes", torch.uint8, cap * rb),
+                         (k_norms, "k_norms", torch.float32, cap), (v_norms, "v_norms", torch.float32, cap),
+                         (k_hot, "k_hot", torch.float16, hot_cap * HEAD_DIM),
+                         (v_hot, "v_hot", torch.float16, hot_cap * HEAD_DIM)):
+        if t.dtype != dt or not t.is_contiguous() or t.numel() != B * H * m:
+            raise LeanKVError("tq_cache_read: %s must be contiguous %s of %d rows" % (nm, dt, B * H))
+    dev = k_codes.device
+    PiK, PiV = _pi(PiK, dev), _pi(PiV, dev)
+    centroids = _vec(centroids, dev, 1 << bits, "centroids")
+    k = torch.empty(B, H, n, HEAD_DIM, dtype=torch.float16, device=dev)
+    v = torch.empty_like(k)
+    check(
+        _lib_handle().lkv_tq_cache_read(ptr(k_codes), ptr(k_norms), ptr(v_codes), ptr(v_norms), ptr(k_hot), ptr(v_hot),
+                                        ptr(PiK), ptr(PiV), ptr(centroids), int(bits), B * H, int(n), cap, hot_cap,
+                                        ptr(k), ptr(v), stream_handle(dev)),
+        "lkv_tq_cache_read",
+    )
+    return k, v
+
+
 def tq_cache_evict(layers, bounds, bits: int, pos_dev: torch.Tensor) -> None:
     """The eviction half of tq_cache_append for every layer in one launch (lkv_tq_cache_evict): layers is a list
     of (k_codes, k_norms, v_codes, v_norms, k_hot, v_hot, PiK, PiV) on the static ring layout, R = B x kv heads

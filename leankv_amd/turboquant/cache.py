@@ -194,19 +194,11 @@ class TurboQuantCache:
 
     def _get_full_cache(self, layer_idx: int):
         """cat(dequantize(cold).fp16, hot) in position order (cache.py:169-189)."""
-        n = self._seq_lengths[layer_idx]
-        c = self._cold_len(n)
-        hot = self.hot_buffer_size
-        idx = torch.arange(c, n, device=self._device) % hot  # ring slots in position order
-        hk = self._k_hot[layer_idx].index_select(2, idx)
-        hv = self._v_hot[layer_idx].index_select(2, idx)
-        if c == 0:
-            return hk.to(self._dtype), hv.to(self._dtype)
-        ck = torch.ops.leankv.tq_dequantize(self._k_codes[layer_idx][:, :, :c], self._k_norms[layer_idx][:, :, :c],
-                                            self.PiK[layer_idx], self.centroids, self.bits, torch.float16)
-        cv = torch.ops.leankv.tq_dequantize(self._v_codes[layer_idx][:, :, :c], self._v_norms[layer_idx][:, :, :c],
-                                            self.PiV[layer_idx], self.centroids, self.bits, torch.float16)
-        return (torch.cat([ck, hk], dim=2).to(self._dtype), torch.cat([cv, hv], dim=2).to(self._dtype))
+        li = layer_idx
+        k, v = _k.tq_cache_read(self._k_codes[li], self._k_norms[li], self._v_codes[li], self._v_norms[li],
+                                self._k_hot[li], self._v_hot[li], self.PiK[li], self.PiV[li], self.centroids,
+                                self.bits, self._seq_lengths[li])
+        return k.to(self._dtype), v.to(self._dtype)
 
     # ----------------------------------------------------------- fused decode attention
     def decode_attention(self, layer_idx: int, query: torch.Tensor, scaling: float | None = None) -> torch.Tensor:
