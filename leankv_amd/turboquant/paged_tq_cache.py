@@ -157,23 +157,21 @@ class PagedTurboQuantCache:
         values = torch.zeros_like(keys)
         for b in range(batch_size):
             n = self._lengths[li][b]
+            if not n:
+                continue
             c = max(0, n - hot)
-            if c:
-                pages = self._seq_pages[b]
-                pg = torch.tensor([pages[p // ps] for p in range(c)], dtype=torch.long, device=self._device)
-                sl = torch.tensor([p % ps for p in range(c)], dtype=torch.long, device=self._device)
-                kc = self.k_codes[li][pg, :, sl].transpose(0, 1).contiguous()  # [Hkv, c, row bytes]
-                vc = self.v_codes[li][pg, :, sl].transpose(0, 1).contiguous()
-                kn = self.k_norms[li][pg, :, sl].t().contiguous()
-                vn = self.v_norms[li][pg, :, sl].t().contiguous()
-                keys[b, :, :c] = _k.tq_dequantize(kc, kn, self.PiK[li], self.centroids, self.bits,
-                                                  out_dtype=torch.float16)
-                values[b, :, :c] = _k.tq_dequantize(vc, vn, self.PiV[li], self.centroids, self.bits,
-                                                    out_dtype=torch.float16)
-            if n > c:
-                idx = torch.tensor([p % hot for p in range(c, n)], dtype=torch.long, device=self._device)
-                keys[b, :, c:n] = self.k_hot[li, b].index_select(1, idx)
-                values[b, :, c:n] = self.v_hot[li, b].index_select(1, idx)
+            rows = max(c, 1)  # the sequence's store in position order (an unread row when nothing is cold)
+            pages = self._seq_pages[b]
+            pg = torch.tensor([pages[p // ps] for p in range(c)] or [0], dtype=torch.long, device=self._device)
+            sl = torch.tensor([p % ps for p in range(c)] or [0], dtype=torch.long, device=self._device)
+            kc, vc = (t[li][pg, :, sl].transpose(0, 1).reshape(1, -1, rows, self._row_bytes)
+                      for t in (self.k_codes, self.v_codes))
+            kn, vn = (t[li][pg, :, sl].t().reshape(1, -1, rows) for t in (self.k_norms, self.v_norms))
+            k, v = _k.tq_cache_read(kc.contiguous(), kn.contiguous(), vc.contiguous(), vn.contiguous(),
+                                    self.k_hot[li, b:b + 1], self.v_hot[li, b:b + 1], self.PiK[li], self.PiV[li],
+                                    self.centroids, self.bits, n)
+            keys[b, :, :n] = k[0]
+            values[b, :, :n] = v[0]
         return keys, values
 
     def cold_arrays(self, layer_idx: int, b: int):
