@@ -128,60 +128,6 @@ struct AttnParams {
 __host__ __device__ __forceinline__ int rec_acc_off(int G) { return (2 * G + 3) & ~3; }
 __host__ __device__ __forceinline__ int rec_floats(int G) { return rec_acc_off(G) + G * kD; }
 
-// Code rows by stored width CB: 4 = nibble rows (3- and 4-bit codes, 64 B per
-// token), 2 = four 2-bit codes per byte (32 B), 1 = eight 1-bit codes per byte
-// (16 B), the packings of leankv/turboquant/quantizer.py:38-62.  Narrow rows
-// are widened to nibbles in registers as they arrive, so the decode after
-// that (v_perm over a centroid table padded with zeros) is the 3-bit one.
-template <int CB>
-__host__ __device__ constexpr int code_row_bytes() {
-  return kD * CB / 8;
-}
-// 16 bits of 2-bit codes (dims 0..7 at bits 2d) -> dims at bits 4d.
-__device__ __forceinline__ uint32_t nib_from2(uint32_t x) {
-  uint32_t t = x & 0xffffu;
-  t = (t | (t << 8)) & 0x00ff00ffu;
-  t = (t | (t << 4)) & 0x0f0f0f0fu;
-  return (t | (t << 2)) & 0x33333333u;
-}
-// 8 bits of 1-bit codes (dim d at bit d) -> dims at bits 4d.
-__device__ __forceinline__ uint32_t nib_from1(uint32_t x) {
-  uint32_t t = x & 0xffu;
-  t = (t | (t << 12)) & 0x000f000fu;
-  t = (t | (t << 6)) & 0x03030303u;
-  return (t | (t << 3)) & 0x11111111u;
-}
-// Dims 32k .. 32k+31 of a code row as 4 nibble dwords; voff/soff address the
-// row's byte 4*CB*k.
-template <int CB>
-__device__ __forceinline__ u32x4 load_codes32(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-  if constexpr (CB == 4) {
-    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
-  } else if constexpr (CB == 2) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
-    const uint32_t lo = v[0], hi = v[1];
-    return u32x4{nib_from2(lo), nib_from2(lo >> 16), nib_from2(hi), nib_from2(hi >> 16)};
-  } else {
-    const uint32_t v = __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
-    return u32x4{nib_from1(v), nib_from1(v >> 8), nib_from1(v >> 16), nib_from1(v >> 24)};
-  }
-}
-// Dims 8k .. 8k+7 of a code row as one nibble dword (row byte CB*k).
-template <int CB>
-__device__ __forceinline__ uint32_t load_codes8(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-  if constexpr (CB == 4)
-    return __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
-  else if constexpr (CB == 2)
-    return nib_from2(__builtin_amdgcn_raw_buffer_load_b16(r, voff, soff, 0));
-  else
-    return nib_from1(__builtin_amdgcn_raw_buffer_load_b8(r, voff, soff, 0));
-}
-
-// Buffer resource over `bytes` bytes at base (raw addressing, stride 0).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
-}
-
 // The (batch, kv head) slice of the cold store as four buffer resources.
 struct ColdRsrc {
   __amdgpu_buffer_rsrc_t kc, vc, kn, vn;

@@ -67,22 +67,60 @@ __device__ __forceinline__ void decode_half(uint32_t w, int half, const uint32_t
   }
 }
 
-// Code rows of stored width CB (4: nibbles, 64 B per token; 2: four codes per
-// byte; 1: eight per byte) widened to nibble dwords as they are loaded, so the
-// decode after the load is the nibble one (bits 1 and 2 through the v_perm
-// table, zero-padded past 2^bits centroids).
-__device__ __forceinline__ uint32_t nib2(uint32_t x) {  // 8 two-bit codes -> 8 nibbles
+// Code rows by stored width CB: 4 = nibble rows (3- and 4-bit codes, 64 B per
+// token), 2 = four 2-bit codes per byte (32 B), 1 = eight 1-bit codes per byte
+// (16 B), the packings of leankv/turboquant/quantizer.py:38-62.  Narrow rows
+// are widened to nibbles in registers as they arrive, so the decode after
+// that (v_perm over a centroid table padded with zeros) is the 3-bit one.
+template <int CB>
+__host__ __device__ constexpr int code_row_bytes() {
+  return 16 * CB;
+}
+// 16 bits of 2-bit codes (dims 0..7 at bits 2d) -> dims at bits 4d.
+__device__ __forceinline__ uint32_t nib_from2(uint32_t x) {
   uint32_t t = x & 0xffffu;
   t = (t | (t << 8)) & 0x00ff00ffu;
   t = (t | (t << 4)) & 0x0f0f0f0fu;
   return (t | (t << 2)) & 0x33333333u;
 }
-__device__ __forceinline__ uint32_t nib1(uint32_t x) {  // 8 one-bit codes -> 8 nibbles
+// 8 bits of 1-bit codes (dim d at bit d) -> dims at bits 4d.
+__device__ __forceinline__ uint32_t nib_from1(uint32_t x) {
   uint32_t t = x & 0xffu;
   t = (t | (t << 12)) & 0x000f000fu;
   t = (t | (t << 6)) & 0x03030303u;
   return (t | (t << 3)) & 0x11111111u;
 }
+// Dims 32k .. 32k+31 of a code row as 4 nibble dwords; voff/soff address the
+// row's byte 4*CB*k.
+template <int CB>
+__device__ __forceinline__ u32x4 load_codes32(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  if constexpr (CB == 4) {
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+  } else if constexpr (CB == 2) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
+    const uint32_t lo = v[0], hi = v[1];
+    return u32x4{nib_from2(lo), nib_from2(lo >> 16), nib_from2(hi), nib_from2(hi >> 16)};
+  } else {
+    const uint32_t v = __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
+    return u32x4{nib_from1(v), nib_from1(v >> 8), nib_from1(v >> 16), nib_from1(v >> 24)};
+  }
+}
+// Dims 8k .. 8k+7 of a code row as one nibble dword (row byte CB*k).
+template <int CB>
+__device__ __forceinline__ uint32_t load_codes8(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  if constexpr (CB == 4)
+    return __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
+  else if constexpr (CB == 2)
+    return nib_from2(__builtin_amdgcn_raw_buffer_load_b16(r, voff, soff, 0));
+  else
+    return nib_from1(__builtin_amdgcn_raw_buffer_load_b8(r, voff, soff, 0));
+}
+
+// Buffer resource over `bytes` bytes at base (raw addressing, stride 0).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
+}
+
 // dims 32k .. 32k + 31 of a row whose code bytes start at p (row byte 4 CB k)
 template <int CB>
 __device__ __forceinline__ uint4 codes32(const uint8_t* p) {
@@ -90,23 +128,12 @@ __device__ __forceinline__ uint4 codes32(const uint8_t* p) {
     return *reinterpret_cast<const uint4*>(p);
   } else if constexpr (CB == 2) {
     const uint2 v = *reinterpret_cast<const uint2*>(p);
-    return uint4{nib2(v.x), nib2(v.x >> 16), nib2(v.y), nib2(v.y >> 16)};
+    return uint4{nib_from2(v.x), nib_from2(v.x >> 16), nib_from2(v.y), nib_from2(v.y >> 16)};
   } else {
     const uint32_t v = *reinterpret_cast<const uint32_t*>(p);
-    return uint4{nib1(v), nib1(v >> 8), nib1(v >> 16), nib1(v >> 24)};
+    return uint4{nib_from1(v), nib_from1(v >> 8), nib_from1(v >> 16), nib_from1(v >> 24)};
   }
 }
-// dims 8k .. 8k + 7 (row byte CB k)
-template <int CB>
-__device__ __forceinline__ uint32_t codes8(const uint8_t* p) {
-  if constexpr (CB == 4)
-    return *reinterpret_cast<const uint32_t*>(p);
-  else if constexpr (CB == 2)
-    return nib2(*reinterpret_cast<const uint16_t*>(p));
-  else
-    return nib1(*p);
-}
-
 __device__ __forceinline__ float vmax(float a, float b) {
   float r;
   asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));

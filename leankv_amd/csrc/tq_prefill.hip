@@ -20,25 +20,36 @@
 //      A block owns 256 (query, head) columns: 256 / G consecutive queries x
 //      the G heads of one kv head, 32 columns per wave.  Its prologue rotates
 //      the block's queries, q_rot = (q @ PiK^T) * scale * log2(e) in fp16 (the
-//      score operand), on the same MFMA with PiK split as in 1 (PiK staged in
-//      the tile buffers, each wave its own 32 columns).  It walks the keys in
-//      tiles of 64; per tile the block decodes the codes once into LDS --
-//      keys as [key][dim] fp16 centroid values (waves 0-3), values transposed
-//      as [dim][key] (waves 4-7) -- and every wave runs, on
-//      v_mfma_f32_16x16x32_f16,
-//      * scores transposed, A = 16 keys x 32 dims from LDS, B = its rotated
-//        queries (registers), so a lane holds 8 keys of one column;
-//      * the online softmax per lane (key norms, causal mask, exp2 domain,
-//        max and sum across the 4 lanes of a column by permlane swaps; the
-//        offset keeps a headroom above the max, so most tiles skip the
-//        rescale of the accumulators);
-//      * values transposed, A = 16 dims x 32 keys from LDS, B = p * n_t from
-//        the lane's own softmax registers.
-//      Each thread loads its share of a tile's codes two tiles ahead into
-//      registers and decodes them into one of two LDS buffers: one barrier
-//      per tile.  In its epilogue the block un-rotates its normalised rows,
-//      out = rows @ PiV on the same MFMA (PiV staged in the free tile buffers,
-//      both operands split into hi + lo), and writes them as fp16.
+//      score operand), with PiK split as in 1 and staged in the tile buffers.
+//      It walks the keys in tiles of 64, decoded once per block into LDS as
+//      fp16 centroid values [key][dim] (key codes by waves 0-3, value codes by
+//      waves 4-7), and every wave runs, on v_mfma_f32_32x32x16_f16,
+//      * scores transposed, A = 32 keys x 16 dims from LDS, B = its rotated
+//        queries (registers), so a lane holds 32 keys of one column (the
+//        other half of a tile's keys in lane ^ 32);
+//      * the online softmax per lane (key norms, causal mask, exp2 domain).
+//        The offset keeps a headroom above the max, so most tiles need neither
+//        a max over the column's lanes nor a rescale of the accumulators: they
+//        only check that no score passes the offset;
+//      * values transposed, A = 32 dims x 16 keys gathered from the [key][dim]
+//        rows by transposed LDS reads, B = p * n_t from the lane's own softmax
+//        registers.
+//      In its epilogue the block un-rotates its normalised rows, out = rows @
+//      PiV on the same MFMA (PiV staged in the free tile buffers, both operands
+//      split into hi + lo), and writes them as fp16.
+//
+// What bounds it: two waves per SIMD (256 registers each), so LDS latency,
+// vector work (~200 instructions per wave and tile) and the matrix products
+// (1024 cycles) overlap in part only.  16x16x32 products cost an issue slot of
+// the vector port each (16 of them beside 48 vector instructions take 367
+// cycles, alone 271): the 32x32 form halves that.  Measured, one block's cost
+// per 64-key tile 2.47 -> 1.83 us, and per call (4096 tokens, 32/8 heads) 225 ->
+// 201 us on one box, 512 queries over 2048 keys 102 -> 82 us: one column per
+// lane, no cross-lane max on most tiles (2.47 -> 2.1), code loads through
+// scalar descriptors and a decode without per-lane branches (2.02 -> 1.83).
+// One wave per SIMD with 64 columns was slower (384 us: the compiler moves the
+// accumulators between register files); four tile buffers instead of two, more
+// reads in flight and interleaved products and softmax changed little.
 #include "kernels.h"
 #include "tq_attn_common.h"
 #include "tq_common.h"
@@ -49,45 +60,26 @@ namespace {
 constexpr int kD = 128;
 constexpr int kThreads = 256;   // rotate16_kernel
 constexpr int kKT = 64;         // keys per tile
-#ifndef LKV_PREFILL_WAVES
-#define LKV_PREFILL_WAVES 8
-#endif
-// Waves of an attention block, 32 (query, head) columns each.  With 8, the
-// key codes of a tile are decoded by waves 0-3 and the value codes by waves
-// 4-7, so each decoded tile serves twice the columns of a 4-wave block.
-constexpr int kPWaves = LKV_PREFILL_WAVES;
-static_assert(kPWaves == 4 || kPWaves == 8, "4 or 8 waves per attention block");
+// Waves of an attention block, 32 (query, head) columns each; waves 0-3 decode
+// the key codes of a tile, waves 4-7 the value codes.
+constexpr int kPWaves = 8;
 constexpr int kPThreads = 64 * kPWaves;
-constexpr bool kSplitDecode = kPWaves == 8;
 constexpr int kCols = 32 * kPWaves;  // (query, head) columns per block
 constexpr int kKRow = kD + 8;   // fp16 row of the decoded key tile (padded)
-#ifndef LKV_PREFILL_VTR
-#define LKV_PREFILL_VTR 1
-#endif
-// Value tile layout.  1: [key][column] rows as decoded (columns in the keys'
-// dim order), the MFMA's V^T operand gathered by ds_read_b64_tr_b16; 0:
-// transposed [dim][key] by v_perm in the decode.
-constexpr bool kVTr = LKV_PREFILL_VTR;
-constexpr int kVRow = kKT + 4;    // [dim][key] row (padded: conflict-free 8-byte reads)
-// [key][column] row: 72 dwords, so the 8-byte chunks of a transposed read (rows 4 g + i, 4 chunks each)
-// fall in distinct banks
-constexpr int kVRowT = kD + 16;
-constexpr int kVBuf = kVTr ? kKT * kVRowT : kD * kVRow;  // fp16 per value buffer
+// Value rows [key][column] as decoded, 72 dwords: the MFMA's V^T operand is
+// gathered by ds_read_b64_tr_b16, whose 8-byte chunks (rows 4 g + i, 4 chunks
+// each) then fall in distinct banks.
+constexpr int kVRow = kD + 16;
+constexpr int kKBuf = kKT * kKRow, kVBuf = kKT * kVRow;  // fp16 per tile buffer
+constexpr int kBufs = 4;                                 // two pairs of tiles
 static_assert(kKT == 64, "the decode / compute lane maps assume 64-key tiles");
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kXcds = 8;  // MI355X: 8 accelerator complex dies, one L2 each
 
-#ifndef LKV_PREFILL_QROT
-#define LKV_PREFILL_QROT 1
-#endif
-// 1: the attention kernel rotates its own queries in its prologue; 0: one
-// rotate16_kernel launch writes them first.  Same bits either way.
-constexpr bool kQRotIn = LKV_PREFILL_QROT;
-
 struct PrefillParams {
-  const uint16_t* q16;     // [B, Hq, S, 128] fp16: q (kQRotIn) or (q @ PiK^T) * scale * log2(e)
-  const float* PiK;        // [128, 128] (kQRotIn)
-  float scale_log2;        // scale * log2(e) (kQRotIn)
+  const uint16_t* q16;     // [B, Hq, S, 128] fp16
+  const float* PiK;        // [128, 128]
+  float scale_log2;        // scale * log2(e)
   const float* PiV;        // [128, 128]: the output rows are un-rotated in the epilogue
   uint16_t* out;           // [B, Hq, S, 128] fp16
   const uint8_t* k_codes;  // [B, Hkv, cap, 64]
@@ -264,19 +256,58 @@ __device__ __forceinline__ uint4 perm_group(uint4 a) {
                __builtin_amdgcn_perm(a.y, a.x, 0x07060302u), __builtin_amdgcn_perm(a.w, a.z, 0x07060302u)};
 }
 
+// Largest of a lane's 32 scores.
+__device__ __forceinline__ float max32(const float (&s)[32]) {
+  float a = vmax3(s[0], s[1], s[2]), b = vmax3(s[3], s[4], s[5]);
+#pragma unroll
+  for (int j = 6; j < 30; j += 4) {
+    a = vmax3(a, s[j], s[j + 1]);
+    b = vmax3(b, s[j + 2], s[j + 3]);
+  }
+  return vmax(vmax3(a, s[30], s[31]), b);
+}
+// Max / sum over the two lanes l, l ^ 32 that share a column.
+__device__ __forceinline__ float xhalf_max(float v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return vmax(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+__device__ __forceinline__ float xhalf_sum(float v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(a[0]) + __uint_as_float(a[1]);
+}
+// fp16(a b) in the low half, fp16(c d) in the high half, each product rounded once.
+__device__ __forceinline__ uint32_t mul2h(float a, float b, float c, float d) {
+  uint32_t r;
+  asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(r) : "v"(a), "v"(b));
+  asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(r) : "v"(c), "v"(d));
+  return r;
+}
+__device__ __forceinline__ void split_hl(float x, uint16_t& hi, uint16_t& lo) {
+  hi = f2h(x);
+  lo = f2h((x - h2f(hi)) * 2048.f);
+}
+__device__ __forceinline__ uint32_t pair16(uint16_t lo, uint16_t hi) { return lo | (static_cast<uint32_t>(hi) << 16); }
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+// D (lane l: column l % 32, rows 8 (i / 4) + 4 (l / 32) + i % 4, i = 0..15) += A (row l % 32) x B (column l % 32),
+// both with k slots 8 (l / 32) + j, j = 0..7
+__device__ __forceinline__ f32x16 mfma32x32x16(const u32x4& a, const u32x4& b, const f32x16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
 template <bool PERM, int CB>
-__global__ __launch_bounds__(kPThreads, 8 / kPWaves) void tq_prefill_attn_kernel(PrefillParams P) {
+__global__ __launch_bounds__(kPThreads, 1) void tq_prefill_attn_kernel(PrefillParams P) {
   static_assert(CB == 4 || PERM, "narrow code rows use the v_perm decode");
   constexpr int RB = kD * CB / 8;  // code bytes per token
-  __shared__ __align__(16) uint16_t sK[2 * kKT * kKRow];  // two buffers of decoded keys
-  __shared__ __align__(16) uint16_t sVt[2 * kVBuf];  // two buffers of decoded values
-  __shared__ __align__(16) float sN[2][2][kKT];           // [buffer][key, value] norms (1 hot, 0 past the end)
+  __shared__ __align__(16) uint16_t sK[kBufs * kKBuf];   // decoded keys
+  __shared__ __align__(16) uint16_t sVt[kBufs * kVBuf];  // decoded values
+  __shared__ __align__(16) float sN[kBufs][2][kKT];    // [buffer][key, value] norms (1 hot, 0 past the end)
   __shared__ uint32_t s_lut[256];
-  __shared__ uint16_t s_cent[16];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int h16 = lane & 15, g = lane >> 4;
+  const int c32 = lane & 31, hf = lane >> 5;
   const int G = P.G, QT = kCols / G;
   // The latest queries see the most keys: their tiles are dispatched first.
   // Workgroups go to the 8 XCDs round-robin by linear id and every query tile
@@ -302,15 +333,75 @@ __global__ __launch_bounds__(kPThreads, 8 / kPWaves) void tq_prefill_attn_kernel
       item = p / nx;
       t = p % nx;
     }
-    qtile = nx - 1 - t;
-    kvh = item % static_cast<int>(gridDim.y);
-    b = item / static_cast<int>(gridDim.y);
+    // (divisions leave them in vector registers: made scalar again)
+    qtile = __builtin_amdgcn_readfirstlane(nx - 1 - t);
+    kvh = __builtin_amdgcn_readfirstlane(item % static_cast<int>(gridDim.y));
+    b = __builtin_amdgcn_readfirstlane(item / static_cast<int>(gridDim.y));
   }
   const int q0 = qtile * QT;
   const int qpos0 = P.kv_len - P.S;  // position of query 0
   const size_t bh = static_cast<size_t>(b) * P.Hkv + kvh;
   const int cold_len = P.cold_len, kv_len = P.kv_len;
 
+  // ---- per-thread code registers of a key tile (as nibbles), loaded an
+  // iteration before their decode:
+  //   waves 0-3: key codes of key tid / 4, dims 32 (tid % 4) .. +32
+  //   waves 4-7: value codes of keys 4 kp + e, dims 8 j4 .. +8 (the 16 lanes of a row group take the 16 column
+  //              chunks of one row: conflict-free 16-byte stores, coalesced code loads)
+  // and key (wave 0) and value norms (wave 4) of key lane
+  const uint8_t* kcod = P.k_codes + bh * static_cast<size_t>(P.cap) * RB;
+  const uint8_t* vcod = P.v_codes + bh * static_cast<size_t>(P.cap) * RB;
+  const bool key_thr = wave < 4;  // wave-uniform
+  const float* norms = (key_thr ? P.k_norms : P.v_norms) + bh * static_cast<size_t>(P.cap);
+  const bool nrm_thr = wave == 0 || wave == 4;
+  const int kk = (tid & 255) >> 2, part = tid & 3;
+  const int kp = (tid & 255) >> 4, j4 = tid & 15;
+  const uint8_t* const cod = key_thr ? kcod : vcod;
+  const int voff = key_thr ? kk * RB + 4 * CB * part : 4 * kp * RB + CB * j4;
+  uint32_t tw[2][4];
+  float tn[2] = {0.f, 0.f};
+  // through buffer descriptors over the tile's cold rows (rows past them read 0, their values come from
+  // elsewhere): constant lane offsets, the tile's position in the scalar base
+  auto load_tile = [&](int t0, int u) {
+    const int n = __builtin_amdgcn_readfirstlane(max(0, min(kKT, cold_len - t0)));  // (the clamp compiles to vector code)
+    const __amdgpu_buffer_rsrc_t rc = make_rsrc(cod + static_cast<size_t>(t0) * RB, n * RB);
+    if (key_thr) {
+      const u32x4 w = load_codes32<CB>(rc, voff, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) tw[u][e] = w[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) tw[u][e] = load_codes8<CB>(rc, voff + e * RB, 0);
+    }
+    if (nrm_thr)
+      tn[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(make_rsrc(norms + t0, n * 4), 4 * lane, 0, 0));
+  };
+
+  // ---- prologue loads, all in flight together: the first tile's codes, the
+  // block's queries, the rotation matrices
+  load_tile(0, 0);
+  load_tile(kKT, 1);
+  // the wave's (query, head) column c = 32 wave + lane % 32: query q0 + c / G, head c % G
+  const int qq = q0 + (32 * wave + c32) / G, qh = (32 * wave + c32) % G;
+  const size_t qrow = ((static_cast<size_t>(b) * P.Hq + kvh * G + qh) * P.S + min(qq, P.S - 1)) * kD;
+  u32x4 bq[8];  // B: the column's q row, dims 16 kb + 8 hf .. +7
+#pragma unroll
+  for (int kb = 0; kb < 8; ++kb) {
+    const uint4 u = *reinterpret_cast<const uint4*>(P.q16 + qrow + 16 * kb + 8 * hf);
+    bq[kb] = u32x4{u.x, u.y, u.z, u.w};
+  }
+  constexpr int kPiRows = kPThreads / 32, kPiLd = kD / kPiRows;  // thread: input dims 4 (tid % 32) .. of 8 rows
+  float4 pk[kPiLd];
+  // PiK row for staged row R = 32 t + r: the column of the key tile that output element (lane, i) of row tile
+  // t belongs to (r = 8 (i / 4) + 4 hf + i % 4), C = 16 (2 t + i / 8) + 8 hf + i % 8, so that the product's
+  // output is the score operand, k step 2 t + i / 8, slot i % 8; the dim of C in the decode's order
+#pragma unroll
+  for (int j = 0; j < kPiLd; ++j) {
+    const int R = tid / 32 + kPiRows * j, r = R & 31;
+    const int C = (R & ~31) + 16 * (r >> 4) + 8 * ((r >> 2) & 1) + 4 * ((r >> 3) & 1) + (r & 3);
+    const int dim = PERM ? (C & ~7) + ((C & 3) << 1) + ((C >> 2) & 1) : C;
+    pk[j] = *reinterpret_cast<const float4*>(P.PiK + dim * kD + 4 * (tid & 31));
+  }
   // ---- centroid tables
   uint32_t tab[4] = {0u, 0u, 0u, 0u};
   if constexpr (PERM) {
@@ -325,473 +416,270 @@ __global__ __launch_bounds__(kPThreads, 8 / kPWaves) void tq_prefill_attn_kernel
     const int cmax = P.ncent - 1;
     if (tid < 256) s_lut[tid] = pack2h(P.centroids[min(tid & 15, cmax)], P.centroids[min(tid >> 4, cmax)]);
   }
-  if (tid < 16) s_cent[tid] = f2h(P.centroids[min(tid, P.ncent - 1)]);
 
-  // ---- query operands: column c = 32 wave + 16 ct + lane % 16 is query
-  // q0 + c / G, head c % G; B operand dims 32 kb + 8 (lane / 16) + position.
-  int lim[2];  // keys [0, lim) visible to the lane's column (0: no such query)
-  u32x4 qa[2][4];
-  int wmin = 0x7fffffff;
-  if constexpr (kQRotIn) {
-    // q_rot = (q @ PiK^T) * scale * log2(e) on fp16 MFMA, rotate16_kernel's arithmetic (PiK split into
-    // fp16 hi + lo / 2048, the same products in the same k order, so the same bits), transposed: A = 16
-    // rows of PiK, B = the wave's 16 query rows of a column tile.  Staged row R = 32 kb + 16 hf + 4 g' + i
-    // holds the PiK row of the key tile's column 32 kb + 8 g' + 4 hf + i (its dim in the decode's order),
-    // so the output lane (h16, g) of row tile 2 kb + hf holds that column tile's score operand positions
-    // 4 hf + i of dims block kb: qa[ct][kb] directly.  PiK hi in sK, lo in sVt (the tile buffers are free
-    // until the first decode).
-    {
-      const int e4 = tid & 31;  // input dims 4 e4 .. +3
+  // ---- q_rot = (q @ PiK^T) * scale * log2(e) in fp16 (the score operand):
+  // A = 32 rows of PiK (split into fp16 hi + lo / 2048, in the tile buffers,
+  // free until the first decode), B = the wave's 32 query rows
 #pragma unroll
-      for (int j = 0; j < kD / (kPThreads / 32); ++j) {
-        const int R = tid / 32 + (kPThreads / 32) * j;
-        const int C = (R & ~31) + 8 * ((R >> 2) & 3) + 4 * ((R >> 4) & 1) + (R & 3);
-        const int dim = PERM ? (C & ~7) + ((C & 3) << 1) + ((C >> 2) & 1) : C;
-        const float4 pv = *reinterpret_cast<const float4*>(P.PiK + dim * kD + 4 * e4);
-        const float x[4] = {pv.x, pv.y, pv.z, pv.w};
-        uint16_t hi[4], lo[4];
+  for (int j = 0; j < kPiLd; ++j) {
+    const int R = tid / 32 + kPiRows * j, e4 = tid & 31;
+    const float x[4] = {pk[j].x, pk[j].y, pk[j].z, pk[j].w};
+    uint16_t hi[4], lo[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          hi[i] = f2h(x[i]);
-          lo[i] = f2h((x[i] - h2f(hi[i])) * 2048.f);
-        }
-        *reinterpret_cast<uint2*>(sK + R * kKRow + 4 * e4) =
-            uint2{hi[0] | (static_cast<uint32_t>(hi[1]) << 16), hi[2] | (static_cast<uint32_t>(hi[3]) << 16)};
-        *reinterpret_cast<uint2*>(sVt + R * kKRow + 4 * e4) =
-            uint2{lo[0] | (static_cast<uint32_t>(lo[1]) << 16), lo[2] | (static_cast<uint32_t>(lo[3]) << 16)};
-      }
-    }
-    u32x4 bq[2][4];  // B: the column's q row, dims 32 kb + 8 g .. +7
-#pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
-      const int c = 32 * wave + 16 * ct + h16;
-      const int qq = q0 + c / G, hh = c % G;
-      const uint16_t* src =
-          P.q16 + ((static_cast<size_t>(b) * P.Hq + kvh * G + hh) * P.S + min(qq, P.S - 1)) * kD + 8 * g;
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        const uint4 u = *reinterpret_cast<const uint4*>(src + 32 * kb);
-        bq[ct][kb] = u32x4{u.x, u.y, u.z, u.w};
-      }
-    }
-    __syncthreads();  // PiK staged
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-      f32x4 accl[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        const u32x4 ah = *reinterpret_cast<const u32x4*>(sK + (16 * t + h16) * kKRow + 32 * kb + 8 * g);
-        const u32x4 al = *reinterpret_cast<const u32x4*>(sVt + (16 * t + h16) * kKRow + 32 * kb + 8 * g);
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct) {
-          acc[ct] = mfma16x16x32(ah, bq[ct][kb], acc[ct]);
-          accl[ct] = mfma16x16x32(al, bq[ct][kb], accl[ct]);
-        }
-      }
-#pragma unroll
-      for (int ct = 0; ct < 2; ++ct) {
-        float v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = (acc[ct][i] + accl[ct][i] * (1.f / 2048.f)) * P.scale_log2;
-        qa[ct][t >> 1][2 * (t & 1)] = static_cast<uint32_t>(f2h(v[0])) | (static_cast<uint32_t>(f2h(v[1])) << 16);
-        qa[ct][t >> 1][2 * (t & 1) + 1] = static_cast<uint32_t>(f2h(v[2])) | (static_cast<uint32_t>(f2h(v[3])) << 16);
-      }
-    }
-    __syncthreads();  // every wave is past its PiK reads: the tile buffers are free
+    for (int i = 0; i < 4; ++i) split_hl(x[i], hi[i], lo[i]);
+    *reinterpret_cast<uint2*>(sK + R * kKRow + 4 * e4) = uint2{pair16(hi[0], hi[1]), pair16(hi[2], hi[3])};
+    *reinterpret_cast<uint2*>(sVt + R * kKRow + 4 * e4) = uint2{pair16(lo[0], lo[1]), pair16(lo[2], lo[3])};
   }
+  static_assert(kD * kKRow <= kBufs * kKBuf && kD * kKRow <= kBufs * kVBuf, "PiK staging fits the tile buffers");
+  __syncthreads();  // PiK staged
+  const bool ok = qq < P.S;
+  const int lim = ok ? qpos0 + qq + 1 : 0;  // keys [0, lim) visible to the lane's column (0: no such query)
+  u32x4 qa[8];
 #pragma unroll
-  for (int ct = 0; ct < 2; ++ct) {
-    const int c = 32 * wave + 16 * ct + h16;
-    const int qq = q0 + c / G, hh = c % G;
-    const bool ok = qq < P.S;
-    lim[ct] = ok ? qpos0 + qq + 1 : 0;
-    if (ok) wmin = min(wmin, lim[ct]);
-    if constexpr (kQRotIn) {
+  for (int t = 0; t < 4; ++t) {
+    f32x16 acc = {}, accl = {};
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) qa[ct][kb] = ok ? qa[ct][kb] : u32x4{0u, 0u, 0u, 0u};
-    } else {
-      const uint16_t* src =
-          P.q16 + ((static_cast<size_t>(b) * P.Hq + kvh * G + hh) * P.S + min(qq, P.S - 1)) * kD + 8 * g;
+    for (int kb = 0; kb < 8; ++kb) {
+      const u32x4 ah = *reinterpret_cast<const u32x4*>(sK + (32 * t + c32) * kKRow + 16 * kb + 8 * hf);
+      const u32x4 al = *reinterpret_cast<const u32x4*>(sVt + (32 * t + c32) * kKRow + 16 * kb + 8 * hf);
+      acc = mfma32x32x16(ah, bq[kb], acc);
+      accl = mfma32x32x16(al, bq[kb], accl);
+    }
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        uint4 u = *reinterpret_cast<const uint4*>(src + 32 * kb);
-        if constexpr (PERM) u = perm_group(u);
-        const u32x4 v = u32x4{u.x, u.y, u.z, u.w};
-        qa[ct][kb] = ok ? v : u32x4{0u, 0u, 0u, 0u};
-      }
+    for (int i = 0; i < 16; i += 2) {
+      const float v0 = (acc[i] + accl[i] * (1.f / 2048.f)) * P.scale_log2;
+      const float v1 = (acc[i + 1] + accl[i + 1] * (1.f / 2048.f)) * P.scale_log2;
+      qa[2 * t + (i >> 3)][(i & 7) >> 1] = ok ? pack2h(v0, v1) : 0u;
     }
   }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) wmin = min(wmin, __shfl_xor(wmin, o));
-  wmin = __builtin_amdgcn_readfirstlane(wmin);
+  // the fewest keys a column of the wave sees: its first column's (queries ascend); none past the last query
+  const int wq = q0 + 32 * wave / G;
+  const int wmin = wq < P.S ? qpos0 + wq + 1 : 0x7fffffff;
+  __syncthreads();  // every wave is past its PiK reads: the tile buffers are free
 
   // keys [0, kend) are visible to some column of the block
   const int kend = qpos0 + min(q0 + QT, P.S);
   const int ntile = (kend + kKT - 1) / kKT;
 
-  // ---- per-thread code registers of one key tile, loaded two tiles ahead:
-  //   kw   key codes of key tid / 4, dims 32 (tid % 4) .. +32 (as nibbles)
-  //   vw   value codes of keys 4 kp + e, dims 8 j4 .. +8 (as nibbles)
-  //   nrm  threads < 128: key (tid < 64) or value norm of key tid % 64
-  // with vt = tid; with the split decode, threads below 256 hold kw only and
-  // threads vt + 256 hold vw only.
-  const uint8_t* kcod = P.k_codes + bh * static_cast<size_t>(P.cap) * RB;
-  const uint8_t* vcod = P.v_codes + bh * static_cast<size_t>(P.cap) * RB;
-  const float* norms = ((tid >> 6) & 1 ? P.v_norms : P.k_norms) + bh * static_cast<size_t>(P.cap);
-  const int kk = (tid & 255) >> 2, part = tid & 3;  // key decode
-  // value decode: with the [key][column] tile, the 16 lanes of a row group take the 16 column chunks of
-  // one row (conflict-free 16-byte stores, coalesced code loads); transposed, the 16 key quads of a column
-  const int vt = tid & 255, kp = kVTr ? vt >> 4 : vt & 15, j4 = kVTr ? vt & 15 : vt >> 4;
-  const bool key_thr = !kSplitDecode || tid < 256, val_thr = !kSplitDecode || tid >= 256;  // wave-uniform
-  struct TileRegs {
-    uint4 kw;
-    uint32_t vw[4];
-    float nrm;
-  };
-  auto load_tile = [&](TileRegs& R, int t0) {
-    if (cold_len > 0) {  // rows past cold_len read the last cold row (valid memory), decoded from elsewhere
-      if (key_thr) R.kw = codes32<CB>(kcod + static_cast<size_t>(min(t0 + kk, cold_len - 1)) * RB + 4 * CB * part);
-      if (val_thr) {
+  // decode the loaded tile into LDS buffer `buf`: keys and values [key][dim], dims in kPermDim order within
+  // 8-dim groups with PERM; in a tile that reaches past the cold store the rows from cold_len on are then written
+  // again (by the thread that wrote them)
+  uint16_t* const kdst = sK + kk * kKRow + 32 * part;
+  uint16_t* const vdst = sVt + 4 * kp * kVRow + 8 * j4;
+  auto decode_tile = [&](int t0, int buf, int u) {
+    uint16_t* dst = key_thr ? kdst + buf * kKBuf : vdst + buf * kVBuf;
+    const int step = key_thr ? 8 : kVRow;  // keys: the row's four chunks; values: four rows' chunk
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          R.vw[e] = codes8<CB>(vcod + static_cast<size_t>(min(t0 + 4 * kp + e, cold_len - 1)) * RB + CB * j4);
+    for (int e = 0; e < 4; ++e) {
+      uint32_t d[4];
+      decode_dw<PERM>(tw[u][e], tab, s_lut, d);
+      *reinterpret_cast<uint4*>(dst + e * step) = uint4{d[0], d[1], d[2], d[3]};
+    }
+    if (nrm_thr) {
+      const int tk = t0 + lane;
+      sN[buf][key_thr ? 0 : 1][lane] = tk < cold_len ? tn[u] : (tk < kv_len ? 1.f : 0.f);
+    }
+    if (t0 + kKT > cold_len) {  // uniform
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int tk = key_thr ? t0 + kk : t0 + 4 * kp + e;
+        if (tk < cold_len) continue;
+        uint4 v = uint4{0u, 0u, 0u, 0u};
+        if (tk < kv_len) {
+          v = *reinterpret_cast<const uint4*>((key_thr ? P.hk : P.hv) +
+                                              (bh * P.hot_cap + static_cast<size_t>(tk % P.hot_cap)) * kD +
+                                              (key_thr ? 32 * part + 8 * e : 8 * j4));
+          if constexpr (PERM) v = perm_group(v);
+        }
+        *reinterpret_cast<uint4*>(dst + e * step) = v;
       }
     }
-    if (tid < 128) {
-      const int tk = t0 + (tid & 63);
-      const float n = cold_len > 0 ? norms[min(tk, cold_len - 1)] : 0.f;
-      R.nrm = tk < cold_len ? n : (tk < kv_len ? 1.f : 0.f);
-    }
-  };
-  // decode a tile's registers into LDS buffer `buf`: keys [key][dim] (kPermDim
-  // order within 8-dim groups with PERM), values transposed [dim][key]
-  auto decode_tile = [&](const TileRegs& R, int t0, int buf) {
-    uint16_t* sKb = sK + buf * (kKT * kKRow);
-    uint16_t* sVb = sVt + buf * kVBuf;
-    if (key_thr) {
-      const int tk = t0 + kk;
-      uint4 o[4];
-      if (tk < cold_len) {
-        const uint32_t w[4] = {R.kw.x, R.kw.y, R.kw.z, R.kw.w};
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          uint32_t d[4];
-          decode_dw<PERM>(w[q], tab, s_lut, d);
-          o[q] = uint4{d[0], d[1], d[2], d[3]};
-        }
-      } else if (tk < kv_len) {
-        const uint4* src = reinterpret_cast<const uint4*>(
-            P.hk + (bh * P.hot_cap + static_cast<size_t>(tk % P.hot_cap)) * kD + 32 * part);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          o[q] = src[q];
-          if constexpr (PERM) o[q] = perm_group(o[q]);
-        }
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) o[q] = uint4{0u, 0u, 0u, 0u};
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q) *reinterpret_cast<uint4*>(sKb + kk * kKRow + 32 * part + 8 * q) = o[q];
-    }
-    if (val_thr && kVTr) {
-      // keys tb .. tb + 3, columns 8 j4 .. 8 j4 + 7 (dims in the keys' order): one 16-byte chunk each
-      const int tb = t0 + 4 * kp;
-      uint4 o[4];
-      if (tb + 4 <= cold_len) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          uint32_t d[4];
-          decode_dw<PERM>(R.vw[e], tab, s_lut, d);
-          o[e] = uint4{d[0], d[1], d[2], d[3]};
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int tk = tb + e;
-          if (tk < cold_len) {
-            uint32_t d[4];
-            decode_dw<PERM>(R.vw[e], tab, s_lut, d);
-            o[e] = uint4{d[0], d[1], d[2], d[3]};
-          } else if (tk < kv_len) {
-            o[e] = *reinterpret_cast<const uint4*>(P.hv + (bh * P.hot_cap + static_cast<size_t>(tk % P.hot_cap)) * kD +
-                                                  8 * j4);
-            if constexpr (PERM) o[e] = perm_group(o[e]);
-          } else {
-            o[e] = uint4{0u, 0u, 0u, 0u};
-          }
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) *reinterpret_cast<uint4*>(sVb + (4 * kp + e) * kVRowT + 8 * j4) = o[e];
-    } else if (val_thr) {
-      const int tb = t0 + 4 * kp;
-      uint32_t pr[2][8];  // fp16 pairs (key tb + 2 hp, key tb + 2 hp + 1) of dim 8 j4 + dd
-      if (tb + 4 <= cold_len) {
-#pragma unroll
-        for (int hp = 0; hp < 2; ++hp) {
-          const uint32_t w0 = R.vw[2 * hp], w1 = R.vw[2 * hp + 1];
-          if constexpr (PERM) {
-            // decode8 pairs: [0] dims (0, 2), [1] (4, 6), [2] (1, 3), [3] (5, 7)
-            uint32_t a[4], c[4];
-            decode8(w0, tab, a);
-            decode8(w1, tab, c);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int dlo = (q & 1) * 4 + (q >> 1);  // first dim of pair q: 0, 4, 1, 5
-              pr[hp][dlo] = __builtin_amdgcn_perm(c[q], a[q], 0x05040100u);
-              pr[hp][dlo + 2] = __builtin_amdgcn_perm(c[q], a[q], 0x07060302u);
-            }
-          } else {
-#pragma unroll
-            for (int bt = 0; bt < 4; ++bt) {
-              const uint32_t x0 = s_lut[(w0 >> (8 * bt)) & 0xffu], x1 = s_lut[(w1 >> (8 * bt)) & 0xffu];
-              pr[hp][2 * bt] = __builtin_amdgcn_perm(x1, x0, 0x05040100u);
-              pr[hp][2 * bt + 1] = __builtin_amdgcn_perm(x1, x0, 0x07060302u);
-            }
-          }
-        }
-      } else {
-#pragma unroll
-        for (int hp = 0; hp < 2; ++hp)
-#pragma unroll
-          for (int dd = 0; dd < 8; ++dd) pr[hp][dd] = 0u;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int tk = tb + e;
-          uint32_t v[8];
-          if (tk < cold_len) {
-#pragma unroll
-            for (int dd = 0; dd < 8; ++dd) v[dd] = s_cent[(R.vw[e] >> (4 * dd)) & 15u];
-          } else if (tk < kv_len) {
-            const uint4 h = *reinterpret_cast<const uint4*>(
-                P.hv + (bh * P.hot_cap + static_cast<size_t>(tk % P.hot_cap)) * kD + 8 * j4);
-            const uint32_t w[4] = {h.x, h.y, h.z, h.w};
-#pragma unroll
-            for (int dd = 0; dd < 8; ++dd) v[dd] = (w[dd >> 1] >> (16 * (dd & 1))) & 0xffffu;
-          } else {
-#pragma unroll
-            for (int dd = 0; dd < 8; ++dd) v[dd] = 0u;
-          }
-#pragma unroll
-          for (int dd = 0; dd < 8; ++dd) pr[e >> 1][dd] |= v[dd] << (16 * (e & 1));
-        }
-      }
-#pragma unroll
-      for (int dd = 0; dd < 8; ++dd)
-        *reinterpret_cast<uint2*>(sVb + (8 * j4 + dd) * kVRow + 4 * kp) = uint2{pr[0][dd], pr[1][dd]};
-    }
-    if (tid < 128) sN[buf][tid >> 6][tid & 63] = R.nrm;
   };
 
-  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};
-  f32x4 o[2][8];
+  // columns past the last query keep offset 0 over their zero scores: they never ask for the general path
+  float m = ok ? -INFINITY : 0.f, l = 0.f;
+  f32x16 o[4];  // element i: column's output dim (in the key tile's order) 32 db + 8 (i / 4) + 4 hf + i % 4
 #pragma unroll
-  for (int ct = 0; ct < 2; ++ct)
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) o[ct][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int db = 0; db < 4; ++db) o[db] = f32x16{};
 
-  // one key tile from LDS buffer `buf`: the lane's keys are t0 + 16 tt + 4 g + i
-  // (tt 0..3, i 0..3); the value MFMA takes them in two halves of 32 keys
+  // one key tile from LDS buffer `buf`: element i of key block kt is key t0 + 32 kt + 8 (i / 4) + 4 hf + i % 4
   auto compute_tile = [&](int t0, int buf) {
-    const uint16_t* sKb = sK + buf * (kKT * kKRow);
+    const uint16_t* sKb = sK + buf * kKBuf;
     const uint16_t* sVb = sVt + buf * kVBuf;
-    f32x4 sc[2][4];
+    const float* sNb = &sN[buf][0][0];
+    f32x16 sc[2];
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
+    for (int kt = 0; kt < 2; ++kt) {
+      sc[kt] = f32x16{};
 #pragma unroll
-      for (int tt = 0; tt < 4; ++tt) sc[ct][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        const u32x4 a = *reinterpret_cast<const u32x4*>(sKb + (16 * tt + h16) * kKRow + 32 * kb + 8 * g);
-        sc[0][tt] = mfma16x16x32(a, qa[0][kb], sc[0][tt]);
-        sc[1][tt] = mfma16x16x32(a, qa[1][kb], sc[1][tt]);
-      }
-    const bool masked = t0 + kKT > wmin;  // wave-uniform
-    u32x4 pb[2][2];
-#pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
-      float s[16];
-#pragma unroll
-      for (int tt = 0; tt < 4; ++tt) {
-        const f32x4 kn = *reinterpret_cast<const f32x4*>(&sN[buf][0][16 * tt + 4 * g]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) s[4 * tt + i] = sc[ct][tt][i] * kn[i];
-      }
-      if (masked) {
-#pragma unroll
-        for (int jj = 0; jj < 16; ++jj)
-          s[jj] = t0 + 16 * (jj >> 2) + 4 * g + (jj & 3) < lim[ct] ? s[jj] : -INFINITY;
-      }
-      float mx = vmax3(s[0], s[1], s[2]);
-#pragma unroll
-      for (int jj = 3; jj < 16; jj += 2) mx = jj + 1 < 16 ? vmax3(mx, s[jj], s[jj + 1]) : vmax(mx, s[jj]);
-      mx = xgroup_max(mx);
-      const float mn = mx > m[ct] ? mx + kHeadroom : m[ct];  // -inf stays -inf
-      const float mu = mn == -INFINITY ? 0.f : mn;
-      const float alpha = fast_exp2(m[ct] - mu);
-      m[ct] = mn;
-      float ps = 0.f;
-#pragma unroll
-      for (int jj = 0; jj < 16; ++jj) {
-        s[jj] = fast_exp2(s[jj] - mu);
-        ps += s[jj];
-      }
-      l[ct] = l[ct] * alpha + ps;
-      if (wave_ballot(alpha != 1.f) != 0) {
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) o[ct][dt] = o[ct][dt] * alpha;
-      }
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const f32x4 v0 = *reinterpret_cast<const f32x4*>(&sN[buf][1][32 * hh + 4 * g]);
-        const f32x4 v1 = *reinterpret_cast<const f32x4*>(&sN[buf][1][32 * hh + 16 + 4 * g]);
-        const float* p = s + 8 * hh;
-        pb[ct][hh] = u32x4{pack2h(p[0] * v0[0], p[1] * v0[1]), pack2h(p[2] * v0[2], p[3] * v0[3]),
-                           pack2h(p[4] * v1[0], p[5] * v1[1]), pack2h(p[6] * v1[2], p[7] * v1[3])};
-      }
+      for (int kb = 0; kb < 8; ++kb)
+        sc[kt] = mfma32x32x16(
+            *reinterpret_cast<const u32x4*>(sKb + (32 * kt + c32) * kKRow + 16 * kb + 8 * hf), qa[kb], sc[kt]);
     }
-    // values: O^T tiles [ct][dt] += V^T (columns 16 dt .., the lane's 8 keys of half hh) x P^T
+    // log2 weights relative to the running offset: score * key norm - m.  Most
+    // tiles hold no masked key and no score above the offset (which keeps a
+    // headroom above the max): they need no max over the column's two lanes and
+    // no rescale.  The others, and the first (m = -inf), go through the general
+    // path.
+    float s[32];
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
+    for (int q = 0; q < 8; ++q) {
+      const f32x4 kn = *reinterpret_cast<const f32x4*>(sNb + 8 * q + 4 * hf);
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        u32x4 a;
-        if constexpr (kVTr) {
-          // ds_read_b64_tr_b16: in each 16-lane group, lane l receives element l % 4 of the 8 bytes that
-          // lanes 4 i + l / 4 (i = 0..3) address.  Lane (h16, g) addresses key 32 hh + 4 g + h16 / 4 (+16),
-          // columns 16 dt + 4 (h16 % 4) .. +3, so it receives column 16 dt + h16 of keys 32 hh + 4 g + i.
-          const uint16_t* src = sVb + (32 * hh + 4 * g + (h16 >> 2)) * kVRowT + 16 * dt + 4 * (h16 & 3);
-          typedef short v4s __attribute__((ext_vector_type(4)));
-          typedef __attribute__((address_space(3))) v4s lds_v4s;
-          const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(src));
-          const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(src + 16 * kVRowT));
-          const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
-          a = u32x4{l2.x, l2.y, h2.x, h2.y};
-        } else {
-          const uint16_t* row = sVb + (16 * dt + h16) * kVRow;
-          const uint2 lo = *reinterpret_cast<const uint2*>(row + 32 * hh + 4 * g);
-          const uint2 hi = *reinterpret_cast<const uint2*>(row + 32 * hh + 16 + 4 * g);
-          a = u32x4{lo.x, lo.y, hi.x, hi.y};
+      for (int i = 0; i < 4; ++i) s[4 * q + i] = fmaf(sc[q >> 2][4 * (q & 3) + i], kn[i], -m);
+    }
+    // wave-uniform; a NaN score passes as it would below
+    if (t0 + kKT > wmin || wave_ballot(max32(s) > 0.f) != 0) {
+      const int left = lim - t0 - 4 * hf;  // key 8 q + i of the lane is visible below this
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const f32x4 kn = *reinterpret_cast<const f32x4*>(sNb + 8 * q + 4 * hf);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float v = sc[q >> 2][4 * (q & 3) + i] * kn[i];
+          s[4 * q + i] = 8 * q + i < left ? v : -INFINITY;
         }
-        o[0][dt] = mfma16x16x32(a, pb[0][hh], o[0][dt]);
-        o[1][dt] = mfma16x16x32(a, pb[1][hh], o[1][dt]);
       }
+      const float mx = xhalf_max(max32(s));
+      const float mn = mx > m ? mx + kHeadroom : m;  // -inf stays -inf
+      const float mu = mn == -INFINITY ? 0.f : mn;
+      const float alpha = fast_exp2(m - mu);
+      m = mn;
+      l *= alpha;
+#pragma unroll
+      for (int db = 0; db < 4; ++db) o[db] = o[db] * alpha;
+#pragma unroll
+      for (int j = 0; j < 32; ++j) s[j] -= mu;
     }
-  };
-
-  // Two register sets and two LDS buffers in turn: tile it decodes from the
-  // registers loaded two tiles earlier into buffer it % 2, then the loads of
-  // tile it + 2 go out, one barrier, and the tile is computed.  Buffer it % 2
-  // was last read by the compute of tile it - 2, which every wave finished
-  // before the barrier of tile it - 1.
-  TileRegs ra, rb;
-  ra.kw = uint4{0u, 0u, 0u, 0u};
-  ra.vw[0] = ra.vw[1] = ra.vw[2] = ra.vw[3] = 0u;
-  ra.nrm = 0.f;
-  rb = ra;
-  load_tile(ra, 0);
-  if (ntile > 1) load_tile(rb, kKT);
-  for (int it = 0;;) {
-    decode_tile(ra, it * kKT, 0);
-    if (it + 2 < ntile) load_tile(ra, (it + 2) * kKT);
-    __syncthreads();
-    compute_tile(it * kKT, 0);
-    if (++it >= ntile) break;
-    decode_tile(rb, it * kKT, 1);
-    if (it + 2 < ntile) load_tile(rb, (it + 2) * kKT);
-    __syncthreads();
-    compute_tile(it * kKT, 1);
-    if (++it >= ntile) break;
-  }
-
-  // ---- normalise, un-rotate (out = o_rot @ PiV) and write fp16 rows.  One MFMA
-  // contraction per 16 output dims x 16 columns with the input dims in a
-  // permuted k order: in 32-dim block kb, k slot 8 g + j stands for dim
-  // 32 kb + 4 g + j (j < 4) or 32 kb + 16 + 4 g + j - 4 -- the dims this lane
-  // holds in o[ct][2 kb] and o[ct][2 kb + 1] -- so the B operand (o^T, column =
-  // the lane's column) is the lane's own registers, and A = PiV^T in the same k
-  // order comes from LDS.  Both are split exactly into fp16 hi + lo / 2048
-  // (hi.hi + hi.lo + lo.hi, the x_lo.Pi_lo term dropped: ~2^-22 relative).
-  u32x4 obh[2][4], obl[2][4];
+    // weights, and p * value norm in fp16: the value MFMA's operand (slots = the lane's 8 keys of a 16-key step)
+    u32x4 pb[4];
+    float ps[2] = {0.f, 0.f};
 #pragma unroll
-  for (int ct = 0; ct < 2; ++ct) {
-    const float L = xgroup_sum(l[ct]);
-    const float inv = L > 0.f ? 1.f / L : 0.f;
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      const f32x4 u = o[ct][2 * kb] * inv, w = o[ct][2 * kb + 1] * inv;
-      const float v[8] = {u[0], u[1], u[2], u[3], w[0], w[1], w[2], w[3]};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint16_t h0 = f2h(v[2 * j]), h1 = f2h(v[2 * j + 1]);
-        obh[ct][kb][j] = static_cast<uint32_t>(h0) | (static_cast<uint32_t>(h1) << 16);
-        obl[ct][kb][j] = pack2h((v[2 * j] - h2f(h0)) * 2048.f, (v[2 * j + 1] - h2f(h1)) * 2048.f);
-      }
-    }
-  }
-  __syncthreads();  // every wave is past its last tile: the key / value buffers are free
-  // PiV^T into LDS, [e][c] rows of kKRow: hi in sK, lo in sVt (128 x 136 fp16 each).  Column c holds
-  // input dim c, or with the [key][column] value tile under PERM the dim its column c of o carries
-  // (8 (c / 8) + kPermDim[c % 8], the keys' dim order).
-  static_assert(kD * kKRow <= 2 * kKT * kKRow && kD * kKRow <= 2 * kVBuf, "PiV staging fits the tile buffers");
-  {
-    // thread: output dim e = tid % 128, input dims kSpan (tid / 128) .. +kSpan - 1 four at a time
-    // (global loads coalesced over e, one 8-byte LDS store per four dims)
-    constexpr int kSpan = kD / (kPThreads / kD);
-    const int e = tid % kD, dbase = (tid / kD) * kSpan;
-#pragma unroll 4
-    for (int d = dbase; d < dbase + kSpan; d += 4) {
-      uint16_t hi[4], lo[4];
+    for (int q = 0; q < 8; ++q) {
+      const f32x4 vn = *reinterpret_cast<const f32x4*>(sNb + kKT + 8 * q + 4 * hf);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int c = d + i;
-        const int dim = (kVTr && PERM) ? (c & ~7) + ((c & 3) << 1) + ((c >> 2) & 1) : c;
-        const float pv = P.PiV[dim * kD + e];
-        hi[i] = f2h(pv);
-        lo[i] = f2h((pv - h2f(hi[i])) * 2048.f);
+        s[4 * q + i] = fast_exp2(s[4 * q + i]);
+        ps[i & 1] += s[4 * q + i];
       }
-      *reinterpret_cast<uint2*>(sK + e * kKRow + d) =
-          uint2{hi[0] | (static_cast<uint32_t>(hi[1]) << 16), hi[2] | (static_cast<uint32_t>(hi[3]) << 16)};
-      *reinterpret_cast<uint2*>(sVt + e * kKRow + d) =
-          uint2{lo[0] | (static_cast<uint32_t>(lo[1]) << 16), lo[2] | (static_cast<uint32_t>(lo[3]) << 16)};
+      pb[q >> 1][2 * (q & 1)] = mul2h(s[4 * q], vn[0], s[4 * q + 1], vn[1]);
+      pb[q >> 1][2 * (q & 1) + 1] = mul2h(s[4 * q + 2], vn[2], s[4 * q + 3], vn[3]);
     }
-  }
+    l += ps[0] + ps[1];
+    // values: O^T (32 dims x 32 columns) += V^T (the lane's keys 16 ks + 4 hf + .., and 8 further on) x P^T.
+    // ds_read_b64_tr_b16: in each 16-lane group, lane l receives element l % 4 of the 8 bytes that
+    // lanes 4 i + l / 4 (i = 0..3) address: a lane addresses key l / 4 of the group's four, columns 4 (l % 4) ..
+    // +3 of the group's 16, and receives its own column of those four keys.
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+        const uint16_t* src = sVb + (16 * ks + 4 * hf + ((lane & 15) >> 2)) * kVRow + 32 * db + 16 * ((lane >> 4) & 1) +
+                              4 * (lane & 3);
+        typedef short v4s __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) v4s lds_v4s;
+        const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(src));
+        const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(src + 8 * kVRow));
+        const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+        o[db] = mfma32x32x16(u32x4{l2.x, l2.y, h2.x, h2.y}, pb[ks], o[db]);
+      }
+  };
+
+  // Two tiles per barrier and two pairs of LDS buffers in turn: while pair it is
+  // computed, pair it + 1 is decoded into the other buffers (last read by the
+  // compute of pair it - 1, before the last barrier) from registers loaded an
+  // iteration earlier.  Waves 4-7 decode before they compute, waves 0-3 after,
+  // so the two waves of a SIMD are out of step: the matrix products and LDS
+  // reads of one run under the softmax arithmetic of the other.
+  const int npair = (ntile + 1) / 2;
+  auto next_pair = [&](int it) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) decode_tile((2 * it + u) * kKT, (2 * it + u) % kBufs, u);
+    if (it + 1 < npair) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) load_tile((2 * it + 2 + u) * kKT, u);
+    }
+  };
+  next_pair(0);
   __syncthreads();
-#pragma unroll 2
-  for (int et = 0; et < kD / 16; ++et) {
-    f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-    f32x4 accl[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-    const int er = (16 * et + h16) * kKRow;
+#pragma unroll 1
+  for (int it = 0; it < npair; ++it) {
+    if (!key_thr && it + 1 < npair) next_pair(it + 1);
+#pragma unroll 1
+    for (int u = 2 * it; u < min(2 * it + 2, ntile); ++u) compute_tile(u * kKT, u % kBufs);
+    if (key_thr && it + 1 < npair) next_pair(it + 1);
+    __syncthreads();
+  }
+
+  // ---- PiV^T in LDS, [e][c], hi in sK, lo in sVt (the tile buffers are free): thread's blocks of 4 output dims e
+  // = 4 (tid % 32) .. x 4 columns c of the key tile's order (one 8-byte store per dim and part)
+  {
+    const int e0 = 4 * (tid & 31);
+    constexpr int kStep = 4 * kPThreads / 32;  // columns per round
+    float4 pv[kD / kStep][4];
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      const int d0 = 32 * kb + 4 * g;
-      const uint2 h0 = *reinterpret_cast<const uint2*>(sK + er + d0);
-      const uint2 h1 = *reinterpret_cast<const uint2*>(sK + er + d0 + 16);
-      const uint2 l0 = *reinterpret_cast<const uint2*>(sVt + er + d0);
-      const uint2 l1 = *reinterpret_cast<const uint2*>(sVt + er + d0 + 16);
-      const u32x4 ah = u32x4{h0.x, h0.y, h1.x, h1.y}, al = u32x4{l0.x, l0.y, l1.x, l1.y};
+    for (int r = 0; r < kD / kStep; ++r)
 #pragma unroll
-      for (int ct = 0; ct < 2; ++ct) {
-        acc[ct] = mfma16x16x32(ah, obh[ct][kb], acc[ct]);
-        accl[ct] = mfma16x16x32(ah, obl[ct][kb], accl[ct]);
-        accl[ct] = mfma16x16x32(al, obh[ct][kb], accl[ct]);
+      for (int i = 0; i < 4; ++i) {
+        const int c = kStep * r + 4 * (tid >> 5) + i;
+        pv[r][i] = *reinterpret_cast<const float4*>(
+            P.PiV + (PERM ? (c & ~7) + ((c & 3) << 1) + ((c >> 2) & 1) : c) * kD + e0);
       }
-    }
-    // D: output dims 16 et + 4 g + i of column 32 wave + 16 ct + h16
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
-      const int c = 32 * wave + 16 * ct + h16;
-      const int qq = q0 + c / G, hh = c % G;
-      if (qq < P.S) {
-        uint16_t* dst = P.out + ((static_cast<size_t>(b) * P.Hq + kvh * G + hh) * P.S + qq) * kD + 16 * et + 4 * g;
-        const float r0 = acc[ct][0] + accl[ct][0] * (1.f / 2048.f), r1 = acc[ct][1] + accl[ct][1] * (1.f / 2048.f);
-        const float r2 = acc[ct][2] + accl[ct][2] * (1.f / 2048.f), r3 = acc[ct][3] + accl[ct][3] * (1.f / 2048.f);
-        *reinterpret_cast<uint2*>(dst) = uint2{static_cast<uint32_t>(f2h(r0)) | (static_cast<uint32_t>(f2h(r1)) << 16),
-                                              static_cast<uint32_t>(f2h(r2)) | (static_cast<uint32_t>(f2h(r3)) << 16)};
+    for (int r = 0; r < kD / kStep; ++r)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        uint16_t hi[4], lo[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          split_hl(k == 0 ? pv[r][i].x : k == 1 ? pv[r][i].y : k == 2 ? pv[r][i].z : pv[r][i].w, hi[i], lo[i]);
+        const int at = (e0 + k) * kKRow + kStep * r + 4 * (tid >> 5);
+        *reinterpret_cast<uint2*>(sK + at) = uint2{pair16(hi[0], hi[1]), pair16(hi[2], hi[3])};
+        *reinterpret_cast<uint2*>(sVt + at) = uint2{pair16(lo[0], lo[1]), pair16(lo[2], lo[3])};
+      }
+  }
+  // ---- normalise, un-rotate (out = o_rot @ PiV) and write fp16 rows: A = 32
+  // output dims of PiV^T, B = the lane's own normalised sums (k slots of step
+  // (db, u): its dims 32 db + 16 u + 4 hf + .., and 8 further on), both split
+  // exactly into fp16 hi + lo / 2048 (hi.hi + hi.lo + lo.hi, the lo.lo term
+  // dropped: ~2^-22 relative).
+  const float L = xhalf_sum(l);
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  u32x4 obh[8], obl[8];
+#pragma unroll
+  for (int st = 0; st < 8; ++st)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      uint16_t h0, l0, h1, l1;
+      split_hl(o[st >> 1][8 * (st & 1) + 2 * j] * inv, h0, l0);
+      split_hl(o[st >> 1][8 * (st & 1) + 2 * j + 1] * inv, h1, l1);
+      obh[st][j] = pair16(h0, h1);
+      obl[st][j] = pair16(l0, l1);
+    }
+  __syncthreads();  // PiV staged
+#pragma unroll 1
+  for (int et = 0; et < 4; ++et) {
+    f32x16 acc = {}, accl = {}, accm = {};
+    const int er = (32 * et + c32) * kKRow + 4 * hf;
+#pragma unroll
+    for (int st = 0; st < 8; ++st) {
+      const uint2 h0 = *reinterpret_cast<const uint2*>(sK + er + 16 * st);
+      const uint2 h1 = *reinterpret_cast<const uint2*>(sK + er + 16 * st + 8);
+      const uint2 l0 = *reinterpret_cast<const uint2*>(sVt + er + 16 * st);
+      const uint2 l1 = *reinterpret_cast<const uint2*>(sVt + er + 16 * st + 8);
+      const u32x4 ah = u32x4{h0.x, h0.y, h1.x, h1.y}, al = u32x4{l0.x, l0.y, l1.x, l1.y};
+      acc = mfma32x32x16(ah, obh[st], acc);
+      accl = mfma32x32x16(ah, obl[st], accl);
+      accm = mfma32x32x16(al, obh[st], accm);
+    }
+    if (ok) {
+      uint16_t* dst = P.out + qrow + 32 * et + 4 * hf;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float r[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = acc[4 * q + i] + (accl[4 * q + i] + accm[4 * q + i]) * (1.f / 2048.f);
+        *reinterpret_cast<uint2*>(dst + 8 * q) = uint2{pack2h(r[0], r[1]), pack2h(r[2], r[3])};
       }
     }
   }
@@ -806,9 +694,8 @@ extern "C" size_t lkv_tq_prefill_attn_workspace_bytes(int64_t B, int64_t Hq, int
                                                       int64_t hot_cap) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || S <= 0 || hot_cap <= 0) return 0;
   auto al = [](size_t v) { return (v + 255) / 256 * 256; };
-  const size_t rows = kQRotIn ? 0 : static_cast<size_t>(B * Hq * S) * kD;
   const size_t hot = static_cast<size_t>(B * Hkv * hot_cap) * kD * 2;
-  return al(rows * 2) + 2 * al(hot);  // q_rot fp16 (without kQRotIn), hot rings (the output is un-rotated in the kernel)
+  return 2 * al(hot);  // the rotated hot rings (queries and outputs are rotated in the kernel)
 }
 
 extern "C" int lkv_tq_prefill_attn(const void* q, const uint8_t* k_codes, const float* k_norms,
@@ -841,24 +728,19 @@ extern "C" int lkv_tq_prefill_attn(const void* q, const uint8_t* k_codes, const 
               workspace_bytes);
   hipStream_t st = static_cast<hipStream_t>(stream);
   auto al = [](size_t v) { return (v + 255) / 256 * 256; };
-  const int64_t nrows = B * Hq * S;
-  char* ws = static_cast<char*>(workspace);
-  uint16_t* q16 = kQRotIn ? const_cast<uint16_t*>(static_cast<const uint16_t*>(q)) : reinterpret_cast<uint16_t*>(ws);
-  uint16_t* hk = reinterpret_cast<uint16_t*>(ws + (kQRotIn ? 0 : al(static_cast<size_t>(nrows) * kD * 2)));
-  uint16_t* hv = reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(hk) +
+  uint16_t* hk = static_cast<uint16_t*>(workspace);
+  uint16_t* hv = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) +
                                              al(static_cast<size_t>(B * Hkv * hot_cap) * kD * 2));
   const int64_t cold_len = kv_len > hot_cap ? kv_len - hot_cap : 0;
 
-  // q_rot * scale * log2(e) in fp16 (the score operand); the hot rings in the rotated domains
-  // (one launch; every hot slot is rotated, only the current tokens' slots are read)
+  // the hot rings in the rotated domains (one launch; every hot slot is rotated, only the current tokens' are read)
   {
-    const int64_t nhot = kv_len > cold_len ? B * Hkv * hot_cap : 0;
-    const RotSeg segs[3] = {{q, PiK, q16, kQRotIn ? 0 : nrows, scale * kLog2e}, {k_hot, PiK, hk, nhot, 1.f},
-                            {v_hot, PiV, hv, nhot, 1.f}};
-    if (int e = rotate16_segs<true, true, false>(segs, 3, st)) return e;
+    const int64_t nhot = B * Hkv * hot_cap;
+    const RotSeg segs[2] = {{k_hot, PiK, hk, nhot, 1.f}, {v_hot, PiV, hv, nhot, 1.f}};
+    if (int e = rotate16_segs<true, true, false>(segs, 2, st)) return e;
   }
   PrefillParams P;
-  P.q16 = q16;
+  P.q16 = static_cast<const uint16_t*>(q);
   P.PiK = PiK;
   P.scale_log2 = scale * kLog2e;
   P.PiV = PiV;
