@@ -13,6 +13,7 @@ the dispatcher; the Python entry points below skip the dispatcher.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 
 import torch
@@ -21,6 +22,7 @@ from . import _lib
 from ._lib import LeanKVError, check, dtype_code, ptr, require_cuda, stream_handle, workspaces
 
 HEAD_DIM = 128
+_I64x3, _PTRx3, _F32x3 = ctypes.c_int64 * 3, ctypes.c_void_p * 3, ctypes.c_float * 3
 
 
 def _lib_handle():
@@ -33,7 +35,7 @@ def colmajor_rows(weight: torch.Tensor) -> tuple[int, int]:
     if weight.dim() != 2:
         raise LeanKVError("sparse_gemv: weight must be 2-D [N, Z], got %s" % (tuple(weight.shape),))
     N, Z = weight.shape
-    if not weight.t().is_contiguous():
+    if weight.stride() != (1, N) and not weight.t().is_contiguous():  # (sizes of 1 leave strides free)
         raise LeanKVError(
             "sparse_gemv: weight must be column-major (strides (1, N)) as produced by "
             "prepare_weight_for_sparse_gemv; got strides %s" % (weight.stride(),)
@@ -46,7 +48,7 @@ def _check_x(x: torch.Tensor, Z: int, what: str) -> torch.Tensor:
         raise LeanKVError("%s: x must be float16, got %s" % (what, x.dtype))
     if x.numel() != Z:
         raise LeanKVError("%s: x has %d elements, weight expects Z=%d" % (what, x.numel(), Z))
-    return x.reshape(Z).contiguous()
+    return x if x.is_contiguous() else x.reshape(Z).contiguous()
 
 
 def sparse_gemv_out(x: torch.Tensor, weight: torch.Tensor, threshold: float, out: torch.Tensor) -> torch.Tensor:
@@ -70,9 +72,9 @@ def sparse_gemv_out(x: torch.Tensor, weight: torch.Tensor, threshold: float, out
 
 
 def sparse_gemv(x: torch.Tensor, weight: torch.Tensor, threshold: float) -> torch.Tensor:
-    N, _ = colmajor_rows(weight)
-    out = torch.empty(N, dtype=torch.float16, device=x.device)
-    return sparse_gemv_out(x, weight, threshold, out)
+    if weight.dim() != 2:
+        colmajor_rows(weight)  # raises
+    return sparse_gemv_out(x, weight, threshold, x.new_empty(weight.shape[0], dtype=torch.float16))
 
 
 def sparse_gemm_batched_out(x: torch.Tensor, weight: torch.Tensor, threshold: float, out: torch.Tensor) -> torch.Tensor:
@@ -298,9 +300,10 @@ def sparse_gateup_swiglu_out(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.
 
 
 def sparse_gateup_swiglu(x, w_gate, w_up, t_gate, t_up):
-    N, _ = colmajor_rows(w_gate)
-    out = torch.empty(N, dtype=torch.float16, device=x.device)
-    return sparse_gateup_swiglu_out(x, w_gate, w_up, t_gate, t_up, out)
+    if w_gate.dim() != 2:
+        colmajor_rows(w_gate)  # raises
+    return sparse_gateup_swiglu_out(x, w_gate, w_up, t_gate, t_up,
+                                    x.new_empty(w_gate.shape[0], dtype=torch.float16))
 
 
 def sparse_qkv(x: torch.Tensor, wq: torch.Tensor, wk: torch.Tensor, wv: torch.Tensor, tq: float, tk: float,
@@ -318,18 +321,18 @@ def sparse_qkv(x: torch.Tensor, wq: torch.Tensor, wk: torch.Tensor, wv: torch.Te
         raise LeanKVError("sparse_qkv: weights must be float16")
     Ns = [n for n, _ in shapes]
     if out is None:
-        out = tuple(torch.empty(n, dtype=torch.float16, device=x.device) for n in Ns)
-    for o, n in zip(out, Ns):
-        if o.dtype != torch.float16 or o.numel() != n or not o.is_contiguous():
-            raise LeanKVError("sparse_qkv: outputs must be contiguous float16 with %s elements" % (Ns,))
+        out = tuple(x.new_empty(n, dtype=torch.float16) for n in Ns)
+    else:
+        for o, n in zip(out, Ns):
+            if o.dtype != torch.float16 or o.numel() != n or not o.is_contiguous():
+                raise LeanKVError("sparse_qkv: outputs must be contiguous float16 with %s elements" % (Ns,))
     lib = _lib_handle()
-    n_arr = (ctypes.c_int64 * 3)(*Ns)
+    n_arr = _I64x3(*Ns)
     nbytes = lib.lkv_sparse_gemv_multi_workspace_bytes(3, n_arr, Z)
     ws = workspaces.get(x.device, "qkv", nbytes)
     check(
-        lib.lkv_sparse_gemv_multi(ptr(xf), 3, (ctypes.c_void_p * 3)(*[ptr(w) for w in ws_]),
-                                  (ctypes.c_float * 3)(float(tq), float(tk), float(tv)), n_arr, Z,
-                                  (ctypes.c_void_p * 3)(*[ptr(o) for o in out]), ptr(ws), ws.numel(),
+        lib.lkv_sparse_gemv_multi(ptr(xf), 3, _PTRx3(*[ptr(w) for w in ws_]), _F32x3(float(tq), float(tk), float(tv)),
+                                  n_arr, Z, _PTRx3(*[ptr(o) for o in out]), ptr(ws), ws.numel(),
                                   stream_handle(x.device)),
         "lkv_sparse_gemv_multi",
     )
@@ -337,6 +340,7 @@ def sparse_qkv(x: torch.Tensor, wq: torch.Tensor, wk: torch.Tensor, wv: torch.Te
 
 
 # ----------------------------------------------------------------- TurboQuant
+@functools.lru_cache(maxsize=None)
 def packed_row_bytes(bits: int) -> int:
     n = _lib_handle().lkv_tq_packed_row_bytes(int(bits))
     if n < 0:
@@ -358,11 +362,15 @@ def _pi(Pi: torch.Tensor, device) -> torch.Tensor:
     """
     if tuple(Pi.shape) != (HEAD_DIM, HEAD_DIM):
         raise LeanKVError("TurboQuant: rotation must be [128, 128], got %s" % (tuple(Pi.shape),))
+    if Pi.dtype == torch.float32 and Pi.device == device and Pi.is_contiguous():
+        return Pi
     return Pi.to(device=device, dtype=torch.float32).contiguous()
 
 
 def _vec(t: torch.Tensor, device, n: int | None = None, what: str = "table") -> torch.Tensor:
-    v = t.to(device=device, dtype=torch.float32).contiguous()
+    v = t
+    if t.dtype != torch.float32 or t.device != device or not t.is_contiguous():
+        v = t.to(device=device, dtype=torch.float32).contiguous()
     if n is not None and v.numel() != n:
         raise LeanKVError("TurboQuant: %s must have %d entries, got %d" % (what, n, v.numel()))
     return v
@@ -375,11 +383,9 @@ def tq_quantize(x: torch.Tensor, Pi: torch.Tensor, bounds: torch.Tensor, bits: i
     xc = x.contiguous()
     lib = _lib_handle()
     rb = packed_row_bytes(bits)
-    packed = torch.empty(*x.shape[:-1], rb, dtype=torch.uint8, device=x.device)
-    norms = torch.empty(x.shape[:-1], dtype=x.dtype, device=x.device)
-    b = bounds.to(device=x.device, dtype=torch.float32).contiguous()
-    if b.numel() != (1 << bits) - 1:
-        raise LeanKVError("tq_quantize: %d decision boundaries for bits=%d" % (b.numel(), bits))
+    packed = x.new_empty((*x.shape[:-1], rb), dtype=torch.uint8)
+    norms = x.new_empty(x.shape[:-1])
+    b = _vec(bounds, x.device, (1 << bits) - 1, "decision boundaries")
     Pc = _pi(Pi, x.device)  # held until the call returns: a temporary's memory could be reused
     check(
         lib.lkv_tq_quantize(ptr(xc), dtype_code(x.dtype), M, ptr(Pc), ptr(b), int(bits),
@@ -556,10 +562,9 @@ def tq_cache_bulk_update(k_new, v_new, p0: int, k_hot, v_hot, k_codes, k_norms, 
     k_new, v_new = _row_strided(k_new), _row_strided(v_new)
     PiK, PiV = _pi(PiK, dev), _pi(PiV, dev)
     bounds = _vec(bounds, dev, (1 << bits) - 1, "decision boundaries")
-    strides = ctypes.c_int64 * 3
     check(
-        _lib_handle().lkv_tq_cache_bulk_update(ptr(k_new), strides(*k_new.stride()[:3]), ptr(v_new),
-                                               strides(*v_new.stride()[:3]), B, H, S, int(p0), ptr(k_hot), ptr(v_hot),
+        _lib_handle().lkv_tq_cache_bulk_update(ptr(k_new), _I64x3(*k_new.stride()[:3]), ptr(v_new),
+                                               _I64x3(*v_new.stride()[:3]), B, H, S, int(p0), ptr(k_hot), ptr(v_hot),
                                                ptr(k_codes), ptr(k_norms), ptr(v_codes), ptr(v_norms), ptr(PiK),
                                                ptr(PiV), ptr(bounds), int(bits), hot_cap, cap, stream_handle(dev)),
         "lkv_tq_cache_bulk_update",
