@@ -23,7 +23,9 @@ fp16 run, scripts/raw_baseline.py, as torch executes it).
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import gc
 import math
 
 import torch
@@ -33,6 +35,21 @@ from . import _lib
 from .turboquant.cache import TurboQuantCache
 
 STEP_BITS = (1, 2, 3, 4)  # code widths the fused B = 1 decode step (lkv_decode_*) is built for
+
+
+@contextlib.contextmanager
+def _capture(graph, stream):
+    """torch.cuda.graph without cyclic garbage collection meanwhile: an older engine's graph that only the collector
+    can free (a model, its fast-path forward and its engine refer to each other) synchronizes the device when it is
+    destroyed, which fails during a capture and, in a destructor, ends the process."""
+    on = gc.isenabled()
+    gc.disable()
+    try:
+        with torch.cuda.graph(graph, stream=stream):
+            yield
+    finally:
+        if on:
+            gc.enable()
 
 
 def _rms(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
@@ -98,7 +115,7 @@ class _Base:
         s.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(s):
             g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g, stream=s):
+            with _capture(g, s):
                 self._step()
         torch.cuda.current_stream().wait_stream(s)
         self.graph = g
@@ -441,7 +458,7 @@ class BatchedEngine:
             s = torch.cuda.Stream()
             s.wait_stream(torch.cuda.current_stream())
             with torch.cuda.stream(s):
-                with torch.cuda.graph(g, stream=s):
+                with _capture(g, s):
                     self._step()
             torch.cuda.current_stream().wait_stream(s)
             self.graph = g
