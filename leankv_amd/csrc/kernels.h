@@ -208,34 +208,35 @@ __device__ __forceinline__ f32x4 mfma16x16x32(const u32x4& a, const u32x4& b, co
 // hi = fp16(x) (toward zero) and lo = fp16((x - hi) * 2^11) (toward zero),
 // q is fp16, so both products run on v_mfma_f32_16x16x32_f16 with exact
 // fp32 products: q_rot = acc_hi + acc_lo * 2^-11, error ~2^-20 relative.
-// The tile is transposed (rows = output dims, columns = heads).  Wave w
-// covers input dims 32w .. 32w+31 (lane group g' holding 32w + 8g' .. +7)
-// for 8 output tiles; tile c row r is output dim 32(r/4) + 4c + r%4, so lane
-// (h = lane%16, g = lane/16) ends with dims 32g .. 32g+31 of head h.  The 4
-// wave partials are summed through LDS in the fixed order ((w0+w1)+w2)+w3.
-// Called by all 4 waves of a 256-thread block (one __syncthreads inside).
-//   qb   this lane's q[h][32w + 8g .. +7] as fp16 pairs (zero for unused h)
+// The tile is transposed (rows = output dims, columns = heads): tile c row r
+// is output dim 32(r/4) + 4c + r%4, so lane (h = lane%16, g = lane/16) gets
+// dims 32g + 4c .. +3 of head h.  Waves w, w + 4, ... of a block of 4 (8 / NC)
+// waves cover input dims 32 (w % 4) .. +31 (lane group g' holding 8g' .. +7 of
+// them), NC of the 8 tiles each, and leave their partial sums in LDS; after a
+// barrier rotated_sum adds the four in the fixed order ((p0+p1)+p2)+p3.
+//   qb   this lane's q[h][32 (wave % 4) + 8g .. +7] as fp16 pairs (zero for unused h)
 //   part LDS scratch, 4 x 16 rows of `ld` floats (ld >= 128, ld % 4 == 0)
-//   out  out[i] = q_rot[h][32g + 4i .. 4i+3]
-// The PiK operand of rotate_query_hilo, loadable ahead of the query (the
-// decode step issues it before summing the query's partials).
+// The PiK operand is loadable ahead of the query (the decode step issues it
+// before summing the query's partials).
+template <int NC>
 __device__ __forceinline__ void load_pik_operand(const float* __restrict__ PiK, int wave, int lane,
-                                                 float4 (&pa)[8][2]) {
+                                                 float4 (&pa)[NC][2]) {
   const int h = lane & 15, g = lane >> 4;
 #pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const int row = 32 * (h >> 2) + 4 * c + (h & 3);  // lane % 16 is the A row here
-    const float4* src = reinterpret_cast<const float4*>(PiK + row * 128 + 32 * wave + 8 * g);
+  for (int c = 0; c < NC; ++c) {
+    const int row = 32 * (h >> 2) + 4 * (NC * (wave >> 2) + c) + (h & 3);  // lane % 16 is the A row here
+    const float4* src = reinterpret_cast<const float4*>(PiK + row * 128 + 32 * (wave & 3) + 8 * g);
     pa[c][0] = src[0];
     pa[c][1] = src[1];
   }
 }
 
-__device__ __forceinline__ void rotate_query_hilo_loaded(const float4 (&pa)[8][2], const u32x4& qb, int wave,
-                                                         int lane, float* part, int ld, float4 (&out)[8]) {
+template <int NC>
+__device__ __forceinline__ void rotate_query_partials(const float4 (&pa)[NC][2], const u32x4& qb, int wave, int lane,
+                                                      float* part, int ld) {
   const int h = lane & 15, g = lane >> 4;
 #pragma unroll
-  for (int c = 0; c < 8; ++c) {
+  for (int c = 0; c < NC; ++c) {
     const float x[8] = {pa[c][0].x, pa[c][0].y, pa[c][0].z, pa[c][0].w,
                         pa[c][1].x, pa[c][1].y, pa[c][1].z, pa[c][1].w};
     u32x4 hi, lo;
@@ -249,26 +250,16 @@ __device__ __forceinline__ void rotate_query_hilo_loaded(const float4 (&pa)[8][2
     }
     const f32x4 ah = mfma16x16x32(hi, qb, f32x4{0.f, 0.f, 0.f, 0.f});
     const f32x4 al = mfma16x16x32(lo, qb, f32x4{0.f, 0.f, 0.f, 0.f});
-    *reinterpret_cast<float4*>(part + (wave * 16 + h) * ld + 32 * g + 4 * c) =
+    *reinterpret_cast<float4*>(part + ((wave & 3) * 16 + h) * ld + 32 * g + 4 * (NC * (wave >> 2) + c)) =
         make_float4(fmaf(al[0], 1.f / 2048.f, ah[0]), fmaf(al[1], 1.f / 2048.f, ah[1]),
                     fmaf(al[2], 1.f / 2048.f, ah[2]), fmaf(al[3], 1.f / 2048.f, ah[3]));
   }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    float4 p[4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) p[w] = *reinterpret_cast<const float4*>(part + (w * 16 + h) * ld + 32 * g + 4 * i);
-    out[i] = make_float4(((p[0].x + p[1].x) + p[2].x) + p[3].x, ((p[0].y + p[1].y) + p[2].y) + p[3].y,
-                         ((p[0].z + p[1].z) + p[2].z) + p[3].z, ((p[0].w + p[1].w) + p[2].w) + p[3].w);
-  }
 }
-
-__device__ __forceinline__ void rotate_query_hilo(const float* __restrict__ PiK, const u32x4& qb, int wave,
-                                                  int lane, float* part, int ld, float4 (&out)[8]) {
-  float4 pa[8][2];
-  load_pik_operand(PiK, wave, lane, pa);
-  rotate_query_hilo_loaded(pa, qb, wave, lane, part, ld, out);
+__device__ __forceinline__ float rotated_sum(const float* part, int ld, int h, int d) {
+  float p[4];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) p[w] = part[(w * 16 + h) * ld + d];
+  return ((p[0] + p[1]) + p[2]) + p[3];
 }
 
 // y = x @ Pi^T (transpose 0) or x @ Pi (transpose 1) for M rows of 128, fp32
@@ -286,7 +277,6 @@ AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t max_len, int64_t 
                    int64_t max_split_tokens = 0);
 
 struct AttnCall {
-  const float* qrot;        // [B, Hq, 128] fp32 = q @ PiK^T (when PiK is null)
   const uint16_t* q;        // [B, Hq, 128] fp16 (the fp16 hot window uses the unrotated query)
   const uint8_t* k_codes;   // [B, Hkv, cap, 64]
   const float* k_norms;     // [B, Hkv, cap]
@@ -295,7 +285,7 @@ struct AttnCall {
   const uint16_t* k_hot;    // [B, Hkv, hot_cap, 128] ring, token t in slot t % hot_cap
   const uint16_t* v_hot;
   const float* PiV;         // [128, 128]
-  const float* PiK;         // non-null: rotate q in the split kernel (qrot unused); null: qrot given
+  const float* PiK;         // [128, 128]
   const float* centroids;   // [2^bits]
   const int32_t* seq_len;   // device scalar: tokens in the cache (after this step's append)
   float* partials;          // split records (workspace)

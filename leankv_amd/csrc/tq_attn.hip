@@ -11,28 +11,37 @@
 // rotated domain, and PiV is applied once per query head at the end.
 //
 // Launches (all on the caller's stream, no inter-block waits):
-//   1. split kernel, grid splits x kv_heads x batch, 4 waves per block, each
-//      block owning a contiguous range of cold tokens.  Its prologue rotates
-//      the G query heads of its kv head, q_rot = q @ PiK^T on fp32 MFMA
-//      (the decode step passes q_rot from its own QKV epilogue instead),
-//      while the first token blocks load.  Each wave then walks 32-token
-//      blocks with two register sets in turn (the next block's codes and
-//      norms load while the current one is computed):
+//   1. split kernel, grid splits x kv_heads x batch, 16 waves per block (one
+//      block per CU), each block owning a contiguous range of cold tokens.  Its
+//      prologue rotates the G query heads of its kv head, q_rot = q @ PiK^T on
+//      fp16 MFMA with PiK in two parts (the decode step sums the query from its
+//      GEMV partials and ropes it first), while the first token blocks load.
+//      Each wave then walks 32-token blocks; a block's registers are loaded for
+//      the next one as soon as they have been used:
 //      * scores, transposed: v_mfma_f32_16x16x32_f16 with A = 16 tokens x 32
 //        dims of centroid values and B = the rotated query (16 head
 //        columns, G used), so a lane holds one head's scores for 8 tokens.
 //        3-bit codes are decoded on the VALU with v_perm_b32 table lookups;
 //        4-bit codes through a 256-entry LDS table (byte -> fp16 pair);
-//      * online softmax in the exp2 domain, per lane, with the max taken
-//        across the 4 lanes of a head by two permlane swaps; the offset keeps
-//        a headroom above the max, so the rescale of the accumulators runs
-//        only when some head's score passes it;
+//      * online softmax in the exp2 domain, per lane, relative to an offset
+//        with headroom above the largest score seen; the max across the 4 lanes
+//        of a head (two permlane swaps) and the rescale of the accumulators
+//        run only when some lane's score passes the offset;
 //      * values, transposed: the same MFMA with A = 16 dims x 32 tokens of
-//        centroid values (a lane's 8 tokens of one dim, transposed from the
-//        decoded code dwords with v_perm_b32) and B = p * n_t taken straight
+//        centroid values (code bytes of 4 tokens transposed with v_perm_b32
+//        before the lookup) and B = p * n_t taken straight
 //        from the lane's own softmax registers (same 8 tokens);
-//      * the 4 waves merge through LDS and the block writes
+//      * the waves merge through LDS and the block writes
 //        (m, l, acc[G][128]) per head to the workspace;
+//      What bounds it: instruction issue, ~290 vector instructions per 32
+//      tokens.  One wave of a SIMD issues one every ~5 cycles, two together one
+//      every 2.4-3.5 and four one every 1.7-2.8, so the kernel is cut to 120
+//      registers for 4 waves per SIMD (one register set, no second block in
+//      flight: 2, 3 and 4 sets at 2 waves measured alike).  B = 16, 32/8
+//      heads, 4096 tokens, 3 bits, both kernels: 26.6 us with two 4-wave blocks
+//      of two register sets per CU, 25.2 with one 8-wave block of three, 21.8
+//      now; B = 1, 32768 tokens: 22.5 -> 20.0 -> 17.9.  Of the 21.8, 7.4 are
+//      the blocks' fixed part and the combine's launch and run 5.
 //   2. combine kernel, one block of 8 waves per (batch, query head): issues
 //      every load it needs at once (split maxima and sums, the rotated
 //      partial sums, the fp16 hot window and the PiV column slice), then
@@ -77,8 +86,8 @@ __device__ __forceinline__ void stamp(uint64_t* arr, int i) {
 #endif
 
 constexpr int kD = 128;
-constexpr int kThreads = 256;
-constexpr int kWaves = 4;
+constexpr int kWaves = 16;
+constexpr int kThreads = 64 * kWaves;
 constexpr int kBlk = 32;    // tokens per wave step
 constexpr int kHotMax = 256;  // hot-window slots the combine walks (64 per slot group)
 constexpr float kLog2e = 1.4426950408889634f;
@@ -88,7 +97,6 @@ __device__ __forceinline__ float group16_max(float v) { return row16_max(v); }
 __device__ __forceinline__ float group16_sum(float v) { return row16_sum(v); }
 
 struct AttnParams {
-  const float* qrot;        // [B, Hq, 128] fp32 = q @ PiK^T
   const uint16_t* q;        // [B, Hq, 128] fp16 (the hot window uses the unrotated query)
   const uint8_t* k_codes;   // [B, Hkv, cap, 64]
   const float* k_norms;     // [B, Hkv, cap]
@@ -97,7 +105,7 @@ struct AttnParams {
   const uint16_t* k_hot;    // [B, Hkv, hot_cap, 128]
   const uint16_t* v_hot;
   const float* PiV;         // [128, 128]
-  const float* PiK;         // non-null: the split kernel rotates q itself (qrot unused)
+  const float* PiK;         // [128, 128]
   const float* centroids;   // [2^bits]
   const int32_t* seq_len;
   float* partials;          // [B, Hkv, nsplit, rec]
@@ -135,10 +143,10 @@ struct ColdRsrc {
 
 // Registers of one 32-token block t0 .. t0+31 (two 16-token tiles tt) for
 // lane l = 16g + w:
-//   kraw[tt]    code bytes 16g .. 16g+15 of token t0 + 16tt + w  (score operand)
+//   kraw[tt]    codes of dims 32g .. 32g+31 of token t0 + 16tt + w, as stored  (score operand)
 //   kn[tt][i]   key norm   of token t0 + 16tt + 4g + i
 //   vn[tt][i]   value norm of token t0 + 16tt + 4g + i
-//   vdw[4tt+i]  code dword w (dims 8w .. 8w+7) of token t0 + 16tt + 4g + i
+//   vdw[4tt+i]  codes of dims 8w .. 8w+7 of token t0 + 16tt + 4g + i, as stored
 // The score MFMA leaves the score of token t0 + 16tt + 4g + i for head w in
 // lane l, element i of tile tt, so the softmax weights, the value norms and
 // the value codes a lane needs all belong to the same eight tokens: the value
@@ -149,199 +157,209 @@ struct BlockRegs {
   uint32_t vdw[8];
 };
 
-// Token -> row of the buffer resources.  Dense: the (batch, kv head) slice is
-// contiguous, row = token.  Paged: token t of the split lies in page
+// Token of a 16-token tile -> row of the buffer resources, for the tile's first
+// token.  Dense: the (batch, kv head) slice is contiguous, row = token; the
+// resources end with the split, so tokens past it read 0 without a memory
+// access.  Paged: token t of the split lies in page
 // s_pg[(t - t_begin) >> shift] at slot t % page_size, and the pools hold rows
 // (page * Hkv + kv head) * page_size + slot, so a 16-token tile (page size a
-// multiple of 16, tiles 16-aligned) is 16 consecutive rows.
+// multiple of 16, tiles 16-aligned) is 16 consecutive rows of a page that the
+// sequence owns; a tile at or past t_end gets kNoRow.
+constexpr int kNoRow = -1;
 struct DenseRows {
   __device__ __forceinline__ int operator()(int t) const { return t; }
 };
 struct PagedRows {
   const int* s_pg;
-  int t_begin, shift, kvh, Hkv;
+  int t_begin, t_end, shift, kvh, Hkv;
   __device__ __forceinline__ int operator()(int t) const {
+    if (t >= t_end) return kNoRow;
     const int pg = s_pg[(t - t_begin) >> shift];
     return ((pg * Hkv + kvh) << shift) + (t & ((1 << shift) - 1));
   }
 };
 
-// A block entirely below the valid end.  Each load's voffset is one of two
-// lane bases; everything that depends on the block or the load is in the
-// scalar soffset (so no per-load vector address registers stay live).
-template <int CB, typename Rows>
-__device__ __forceinline__ void load_full(BlockRegs& R, const ColdRsrc& rs, int t0, int lane, const Rows& rows) {
+// Byte offsets of a 32-token block's rows.  Loads are issued without a branch,
+// so that the wait for older ones counts them and leaves them in flight; the
+// row offset goes into the vector offset, which the buffer resource
+// range-checks (rows past its end read 0); offsets within a tile are immediates.
+struct BlockOff {
+  int code[2], norm[2];  // of the tiles' first rows
+};
+template <int CB, bool PAGED, typename Rows>
+__device__ __forceinline__ BlockOff block_off(int t0, const Rows& rows) {
   constexpr int RB = code_row_bytes<CB>();
-  const int g = lane >> 4, w = lane & 15;
-  const int vk = w * RB + 4 * CB * g;  // key codes: token w, dims 32g..
-  const int vv = 4 * g * RB + CB * w;  // value codes: token 4g, dims 8w..
-  const int vnrm = 16 * g;             // norms: token 4g
-  const int r0 = __builtin_amdgcn_readfirstlane(rows(t0)), r1 = __builtin_amdgcn_readfirstlane(rows(t0 + 16));
+  // past the end of any pool of fewer than 2^32 - 2^13 bytes, and valid last rows of a larger one; what the loads
+  // add stays under 2^13
+  constexpr int kPastEnd = static_cast<int>(0xFFFFE000u);
+  t0 = __builtin_amdgcn_readfirstlane(t0);  // wave-uniform
+  BlockOff o;
 #pragma unroll
   for (int tt = 0; tt < 2; ++tt) {
-    const int sc = (tt ? r1 : r0) * RB, sn = (tt ? r1 : r0) * 4;
-    R.kraw[tt] = load_codes32<CB>(rs.kc, vk, sc);
-    R.kn[tt] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs.kn, vnrm, sn, 0));
-    R.vn[tt] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs.vn, vnrm, sn, 0));
+    int r = rows(t0 + 16 * tt);
+    if constexpr (PAGED) r = __builtin_amdgcn_readfirstlane(r);
+    const bool none = PAGED && r == kNoRow;
+    o.code[tt] = none ? kPastEnd : r * RB;
+    o.norm[tt] = none ? kPastEnd : r * 4;
   }
-#pragma unroll
-  for (int j = 0; j < 8; ++j) R.vdw[j] = load_codes8<CB>(rs.vc, vv, ((j >> 2) ? r1 : r0) * RB + (j & 3) * RB);
+  return o;
 }
-
-// load_full for a block that may reach past the cold store (the prologue's
-// unconditional loads): the row offset goes into the vector offset, which the
-// buffer descriptor range-checks (rows at or past the end read 0), and the
-// scalar offset is 0.  Dense layout only.
 template <int CB>
-__device__ __forceinline__ void load_full_checked(BlockRegs& R, const ColdRsrc& rs, int t0, int lane) {
-  constexpr int RB = code_row_bytes<CB>();
-  const int g = lane >> 4, w = lane & 15;
-  const int vk = w * RB + 4 * CB * g, vv = 4 * g * RB + CB * w, vnrm = 16 * g;
+__device__ __forceinline__ void load_keys(BlockRegs& R, const ColdRsrc& rs, const BlockOff& o, int lane) {
 #pragma unroll
-  for (int tt = 0; tt < 2; ++tt) {
-    const int r = t0 + 16 * tt;
-    R.kraw[tt] = load_codes32<CB>(rs.kc, vk + r * RB, 0);
-    R.kn[tt] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs.kn, vnrm + r * 4, 0, 0));
-    R.vn[tt] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs.vn, vnrm + r * 4, 0, 0));
-  }
-#pragma unroll
-  for (int j = 0; j < 8; ++j) R.vdw[j] = load_codes8<CB>(rs.vc, vv + (t0 + 16 * (j >> 2) + (j & 3)) * RB, 0);
+  for (int tt = 0; tt < 2; ++tt)  // token w, dims 32g..
+    R.kraw[tt] = load_raw32<CB>(rs.kc, o.code[tt] + (lane & 15) * code_row_bytes<CB>() + 4 * CB * (lane >> 4));
 }
-
-// A block reaching past t_lim: tokens at or past t_lim read token t_lim - 1
-// (valid memory); the caller masks them.
-template <int CB, typename Rows>
-__device__ __forceinline__ void load_clamped(BlockRegs& R, const ColdRsrc& rs, int t0, int t_lim, int lane,
-                                             const Rows& rows) {
-  constexpr int RB = code_row_bytes<CB>();
-  const int g = lane >> 4, w = lane & 15;
+__device__ __forceinline__ void load_norms(f32x4 (&n)[2], __amdgpu_buffer_rsrc_t r, const BlockOff& o, int lane) {
 #pragma unroll
-  for (int tt = 0; tt < 2; ++tt) {
-    const int tk = min(t0 + 16 * tt + w, t_lim - 1);
-    R.kraw[tt] = load_codes32<CB>(rs.kc, rows(tk) * RB + 4 * CB * g, 0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int tn = min(t0 + 16 * tt + 4 * g + i, t_lim - 1);
-      const int rn = rows(tn);
-      R.kn[tt][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs.kn, rn * 4, 0, 0));
-      R.vn[tt][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs.vn, rn * 4, 0, 0));
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int tv = min(t0 + 16 * (j >> 2) + 4 * g + (j & 3), t_lim - 1);
-    R.vdw[j] = load_codes8<CB>(rs.vc, rows(tv) * RB + CB * w, 0);
-  }
+  for (int tt = 0; tt < 2; ++tt)  // tokens 4g..
+    n[tt] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, o.norm[tt] + 16 * (lane >> 4), 0, 0));
 }
-
-template <int CB, typename Rows>
-__device__ __forceinline__ void fetch_block(BlockRegs& R, const ColdRsrc& rs, int t0, int t_addr_end, int lane,
-                                            const Rows& rows) {
-  t0 = __builtin_amdgcn_readfirstlane(t0);  // wave-uniform: keeps the token offset scalar
-  if (t0 + kBlk <= t_addr_end)
-    load_full<CB>(R, rs, t0, lane, rows);
-  else
-    load_clamped<CB>(R, rs, t0, t_addr_end, lane, rows);
+template <int CB>
+__device__ __forceinline__ void load_values(BlockRegs& R, const ColdRsrc& rs, const BlockOff& o, int lane) {
+  constexpr int RB = code_row_bytes<CB>();
+#pragma unroll
+  for (int j = 0; j < 8; ++j)  // token 4g + j % 4, dims 8w..
+    R.vdw[j] = load_raw8<CB>(rs.vc, o.code[j >> 2] + 4 * (lane >> 4) * RB + CB * (lane & 15) + (j & 3) * RB);
 }
 
 // Online-softmax state of one lane: head w = lane % 16, output dims
-// 32g + 8i + dim(t) in o[t][i] (dim(t) = kPermDim[t] with PERM, else t).
+// 32g + 8i + t in o[t][i].
 struct SoftmaxState {
   float m, l;  // running max (log2 domain) and this lane's share of the sum
   f32x4 o[8];
 };
 
-// One 32-token block.  MASKED: tokens at or past t_end take no part.
-template <bool PERM, bool MASKED>
-__device__ __forceinline__ void attend_block(const BlockRegs& R, int t0, int t_end, const u32x4 (&qa)[4],
+// One 32-token block.  MASKED: tokens at or past t_end take no part, and it is the wave's last block; otherwise
+// each of its registers is loaded for the block at `next` as soon as it has been used.
+template <bool PERM, int CB, bool MASKED>
+__device__ __forceinline__ void attend_block(BlockRegs& R, int t0, int t_end, const u32x4 (&qa)[4],
                                              const uint32_t (&tab)[4], const uint32_t* s_lut, int lane,
-                                             SoftmaxState& S) {
+                                             SoftmaxState& S, const ColdRsrc& rs, const BlockOff& next) {
   const int g = lane >> 4;
   // ---- scores, transposed: A = 16 tokens x 32 dims of centroids, B = the
   // rotated query (16 heads); lane gets head lane%16, tokens 4g+i of tile tt.
-  float s[8];
+  f32x4 acc[2];
 #pragma unroll
   for (int tt = 0; tt < 2; ++tt) {
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    acc[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
       uint32_t dd[4];
-      decode_dw<PERM>(R.kraw[tt][kb], tab, s_lut, dd);
-      acc = mfma16x16x32(u32x4{dd[0], dd[1], dd[2], dd[3]}, qa[kb], acc);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float v = acc[i] * R.kn[tt][i];
-      s[4 * tt + i] = (!MASKED || t0 + 16 * tt + 4 * g + i < t_end) ? v : -INFINITY;
+      decode_dw<PERM>(widen32<CB>(R.kraw[tt], kb), tab, s_lut, dd);
+      acc[tt] = mfma16x16x32(u32x4{dd[0], dd[1], dd[2], dd[3]}, qa[kb], acc[tt]);
     }
   }
-  // ---- online softmax; the rescale runs only when some head's score passes
-  // its offset (the max plus kHeadroom when it last moved)
-  float bm = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
-  bm = xgroup_max(bm);  // finite: token t0 of the block is always valid
-  if (__builtin_amdgcn_ballot_w64(bm > S.m) != 0) {
+  if constexpr (!MASKED) load_keys<CB>(R, rs, next, lane);
+  auto valid = [&](int j) { return !MASKED || t0 + 16 * (j >> 2) + 4 * g + (j & 3) < t_end; };
+  // ---- online softmax.  s[j] = score - offset in one fma; the offset (the max
+  // plus kHeadroom when it last moved) and the accumulators change only when a
+  // lane sees a score above it, and only then is the max taken across lanes.
+  float s[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float v = fmaf(acc[j >> 2][j & 3], R.kn[j >> 2][j & 3], -S.m);  // +inf in the first block (m = -inf)
+    s[j] = valid(j) ? v : -INFINITY;
+  }
+  const float tm = vmax(vmax3(vmax3(s[0], s[1], s[2]), s[3], s[4]), vmax3(s[5], s[6], s[7]));
+  if (__builtin_amdgcn_ballot_w64(!(tm <= 0.f)) != 0) {
+    float bm = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float v = acc[j >> 2][j & 3] * R.kn[j >> 2][j & 3];
+      s[j] = valid(j) ? v : -INFINITY;
+      bm = fmaxf(bm, s[j]);
+    }
+    bm = xgroup_max(bm);  // token t0 of the block is always valid
     const float mn = bm > S.m ? bm + kHeadroom : S.m;
-    const float alpha = fast_exp2(S.m - mn);  // 0 on the first block (m = -inf)
+    const float alpha = fast_exp2(S.m - mn);  // 0 on the first block
 #pragma unroll
     for (int t = 0; t < 8; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) S.o[t][i] *= alpha;
     S.l *= alpha;
     S.m = mn;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s[j] -= mn;
   }
-  float pv[8];
+  if constexpr (!MASKED) load_norms(R.kn, rs.kn, next, lane);
+  u32x4 pb;
+  {
+    float p[8], vn[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const float p = fast_exp2(s[j] - S.m);  // masked: exp2(-inf) = 0
-    S.l += p;
-    const float v = p * R.vn[j >> 2][j & 3];
-    pv[j] = (!MASKED || t0 + 16 * (j >> 2) + 4 * g + (j & 3) < t_end) ? v : 0.f;
-  }
-  const u32x4 pb = u32x4{pack2h(pv[0], pv[1]), pack2h(pv[2], pv[3]), pack2h(pv[4], pv[5]), pack2h(pv[6], pv[7])};
-  // ---- values, transposed: A = 16 dims x 32 tokens of centroids (the
-  // lane's 8 tokens of dim 8w + dim(t)), B = p * n_v (the lane's 8 tokens).
-#pragma unroll
-  for (int half = 0; half < 2; ++half) {
-    uint32_t r[8][2];  // r[token j][q] = fp16 pair of positions 4half+2q, 4half+2q+1 of dims 8w..8w+7
-#pragma unroll
-    for (int j = 0; j < 8; ++j) decode_half<PERM>(R.vdw[j], half, tab, s_lut, r[j]);
-#pragma unroll
-    for (int tq = 0; tq < 4; ++tq) {
-      const int t = 4 * half + tq, q = tq >> 1;
-      u32x4 a;
-#pragma unroll
-      for (int pp = 0; pp < 4; ++pp) {
-        const uint32_t x0 = r[2 * pp][q], x1 = r[2 * pp + 1][q];
-        a[pp] = (t & 1) ? __builtin_amdgcn_perm(x1, x0, 0x07060302u) : __builtin_amdgcn_perm(x1, x0, 0x05040100u);
-      }
-      S.o[t] = mfma16x16x32(a, pb, S.o[t]);
+    for (int j = 0; j < 8; ++j) {
+      p[j] = fast_exp2(s[j]);  // masked: exp2(-inf) = 0
+      S.l += p[j];
+      vn[j] = valid(j) ? R.vn[j >> 2][j & 3] : 0.f;
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pb[i] = mul2h(p[2 * i], vn[2 * i], p[2 * i + 1], vn[2 * i + 1]);
+    if constexpr (!MASKED) load_norms(R.vn, rs.vn, next, lane);
+  }
+  // ---- values, transposed: A = 16 dims x 32 tokens of centroids (the
+  // lane's 8 tokens of dim 8w + t), B = p * n_v (the lane's 8 tokens).
+  if constexpr (PERM) {
+    // Code bytes transposed before the lookup: y[q][b] holds byte b (dims 2b, 2b+1) of the lane's tokens
+    // 4q .. 4q+3, so a lookup of its nibbles is already in the operand's token order (16 + 88 instructions a
+    // block; decoding token by token and pairing the fp16 values afterwards took 88 + 32).
+    uint32_t y[2][4];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      uint32_t x[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = valid(4 * q + i) ? widen8<CB>(R.vdw[4 * q + i]) : 0u;  // no NaN from a stale row
+      const uint32_t a0 = __builtin_amdgcn_perm(x[1], x[0], 0x05010400u), b0 = __builtin_amdgcn_perm(x[1], x[0], 0x07030602u);
+      const uint32_t a1 = __builtin_amdgcn_perm(x[3], x[2], 0x05010400u), b1 = __builtin_amdgcn_perm(x[3], x[2], 0x07030602u);
+      y[q][0] = __builtin_amdgcn_perm(a1, a0, 0x05040100u);
+      y[q][1] = __builtin_amdgcn_perm(a1, a0, 0x07060302u);
+      y[q][2] = __builtin_amdgcn_perm(b1, b0, 0x05040100u);
+      y[q][3] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+    }
+    if constexpr (!MASKED) load_values<CB>(R, rs, next, lane);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      uint32_t d[2][2][2];  // [q][nibble]: fp16 pairs of tokens 4q, 4q+1 and 4q+2, 4q+3
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) decode_half<true>(y[q][b], n, tab, s_lut, d[q][n]);
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+        S.o[2 * b + n] = mfma16x16x32(u32x4{d[0][n][0], d[0][n][1], d[1][n][0], d[1][n][1]}, pb, S.o[2 * b + n]);
+    }
+  } else {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      uint32_t r[8][2];  // r[token j][q] = fp16 pair of dims 4half+2q, 4half+2q+1 of dims 8w..8w+7
+#pragma unroll
+      for (int j = 0; j < 8; ++j) decode_half<false>(R.vdw[j], half, tab, s_lut, r[j]);
+#pragma unroll
+      for (int tq = 0; tq < 4; ++tq) {
+        const int t = 4 * half + tq, q = tq >> 1;
+        u32x4 a;
+#pragma unroll
+        for (int pp = 0; pp < 4; ++pp) {
+          const uint32_t x0 = r[2 * pp][q], x1 = r[2 * pp + 1][q];
+          a[pp] = (t & 1) ? __builtin_amdgcn_perm(x1, x0, 0x07060302u) : __builtin_amdgcn_perm(x1, x0, 0x05040100u);
+        }
+        S.o[t] = mfma16x16x32(a, pb, S.o[t]);
+      }
+    }
+    if constexpr (!MASKED) load_values<CB>(R, rs, next, lane);
   }
 }
 
-template <bool PERM>
-__device__ __forceinline__ void attend(const BlockRegs& R, int t0, int t_end, const u32x4 (&qa)[4],
-                                       const uint32_t (&tab)[4], const uint32_t* s_lut, int lane, SoftmaxState& S) {
-  if (t0 + kBlk <= t_end)
-    attend_block<PERM, false>(R, t0, t_end, qa, tab, s_lut, lane, S);
-  else
-    attend_block<PERM, true>(R, t0, t_end, qa, tab, s_lut, lane, S);
-}
-
-constexpr int kORow = kD + 4;  // padded LDS row of the per-wave outputs
-#ifndef LKV_ATTN_BLOCKS_PER_CU
-#define LKV_ATTN_BLOCKS_PER_CU 2
-#endif
-// Resident split blocks per CU (one wave per SIMD each): sets the register
-// budget and the split count.
-constexpr int kSplitBlocksPerCU = LKV_ATTN_BLOCKS_PER_CU;
+constexpr int kORow = kD + 4;   // padded LDS row of the per-wave outputs
+constexpr int kQRow = kD + 8;   // padded LDS row (fp16) of the query operand
+// Resident split blocks per CU: sets the register budget (4 waves per SIMD).
+constexpr int kSplitBlocksPerCU = 1;
 
 constexpr int kMaxPg = 256;  // pages of one split in the paged layout
 
 // QPRE (decode mode): q|k|v partial chunks loaded ahead of the codes, at least
 // the q|k|v GEMV's chunk count for the fast path (8 or 16).
 template <bool PERM, bool DECODE, bool PAGED, int CB, int QPRE = 16>
-__global__ __launch_bounds__(kThreads, kSplitBlocksPerCU) void tq_attn_split_kernel(AttnParams P) {
+__global__ __launch_bounds__(kThreads, 4 * kSplitBlocksPerCU) void tq_attn_split_kernel(AttnParams P) {
   static_assert(!(PAGED && DECODE), "the fused decode step uses the dense layout");
   static_assert(CB == 4 || PERM, "narrow code rows (1, 2 bits) decode through v_perm");
   constexpr int RB = code_row_bytes<CB>();
@@ -349,6 +367,7 @@ __global__ __launch_bounds__(kThreads, kSplitBlocksPerCU) void tq_attn_split_ker
   __shared__ int s_pg[PAGED ? kMaxPg : 1];
   __shared__ float s_m[kWaves][16], s_l[kWaves][16];
   __shared__ __align__(16) float s_o[kWaves][16][kORow];  // all 16 heads: rows >= G are never read
+  __shared__ __align__(16) uint16_t s_qa[16][kQRow];
 
   LKV_SPLIT_STAMP(0);
   // wave index made wave-uniform (scalar) so block offsets become scalar soffsets
@@ -358,24 +377,32 @@ __global__ __launch_bounds__(kThreads, kSplitBlocksPerCU) void tq_attn_split_ker
   const size_t bh = static_cast<size_t>(b) * P.Hkv + kvh;
   float* rec = P.partials + (bh * P.nsplit + split) * rec_floats(G);
 
-  // The split's token range is static; the current length only masks it.
-  // So the length load, the wave's first token block, the centroids and the
+  // Dense: the split's token range is static; the current length only masks it.
+  // So the length load, the wave's first token blocks, the centroids and the
   // rotated query are all in flight before the first wait.
   const int t_begin = split * P.split_tokens;
   int t_addr_end, seq_len;  // valid memory: tokens below t_addr_end
   ColdRsrc rs;
-  const PagedRows prow{s_pg, t_begin, P.page_shift, kvh, P.Hkv};
+  PagedRows prow{s_pg, t_begin, 0, P.page_shift, kvh, P.Hkv};
   if constexpr (PAGED) {
     // Sequence b owns pages indices[indptr[b] .. indptr[b + 1]); the split's
     // pages go to LDS, clamped to the pool; tokens past the sequence's pages
-    // are past t_addr_end (the page of a clamped load is always one it owns).
+    // are past t_addr_end.
     seq_len = __builtin_amdgcn_readfirstlane(P.seq_len[b]);
-    const int pbeg = P.indptr[b], npg_seq = max(0, P.indptr[b + 1] - pbeg);
+    const int pbeg = __builtin_amdgcn_readfirstlane(P.indptr[b]);
+    const int npg_seq = max(0, __builtin_amdgcn_readfirstlane(P.indptr[b + 1]) - pbeg);
     t_addr_end = min(t_begin + P.split_tokens, npg_seq << P.page_shift);
+    prow.t_end = min(min(seq_len, P.max_len) - P.hot_cap, t_addr_end);
+    if (t_begin >= prow.t_end) {  // nothing of this split is cold: sequences of a batch differ in length
+      if (tid < G) {
+        rec[tid] = -INFINITY;
+        rec[G + tid] = 0.f;
+      }
+      return;
+    }
     const int first = t_begin >> P.page_shift, npg = P.split_tokens >> P.page_shift;
     for (int i = tid; i < npg; i += kThreads) {
-      const int pi = min(first + i, npg_seq - 1);
-      const int pg = pi >= 0 ? P.indices[pbeg + pi] : 0;
+      const int pg = P.indices[pbeg + min(first + i, npg_seq - 1)];
       s_pg[i] = min(max(pg, 0), P.max_pages - 1);
     }
     rs.kc = make_rsrc(P.k_codes, P.pool_code_bytes);
@@ -386,37 +413,33 @@ __global__ __launch_bounds__(kThreads, kSplitBlocksPerCU) void tq_attn_split_ker
   } else {
     t_addr_end = min(t_begin + P.split_tokens, P.cap);
     seq_len = __builtin_amdgcn_readfirstlane(*P.seq_len);
-    rs.kc = make_rsrc(P.k_codes + bh * static_cast<size_t>(P.cap) * RB, static_cast<uint32_t>(P.cap) * RB);
-    rs.vc = make_rsrc(P.v_codes + bh * static_cast<size_t>(P.cap) * RB, static_cast<uint32_t>(P.cap) * RB);
-    rs.kn = make_rsrc(P.k_norms + bh * static_cast<size_t>(P.cap), static_cast<uint32_t>(P.cap) * 4);
-    rs.vn = make_rsrc(P.v_norms + bh * static_cast<size_t>(P.cap), static_cast<uint32_t>(P.cap) * 4);
+    rs.kc = make_rsrc(P.k_codes + bh * static_cast<size_t>(P.cap) * RB, static_cast<uint32_t>(t_addr_end) * RB);
+    rs.vc = make_rsrc(P.v_codes + bh * static_cast<size_t>(P.cap) * RB, static_cast<uint32_t>(t_addr_end) * RB);
+    rs.kn = make_rsrc(P.k_norms + bh * static_cast<size_t>(P.cap), static_cast<uint32_t>(t_addr_end) * 4);
+    rs.vn = make_rsrc(P.v_norms + bh * static_cast<size_t>(P.cap), static_cast<uint32_t>(t_addr_end) * 4);
   }
-  auto fetch = [&](BlockRegs& R, int t) {
+  auto off = [&](int t) {
     if constexpr (PAGED)
-      fetch_block<CB>(R, rs, t, t_addr_end, lane, prow);
+      return block_off<CB, true>(t, prow);
     else
-      fetch_block<CB>(R, rs, t, t_addr_end, lane, DenseRows{});
+      return block_off<CB, false>(t, DenseRows{});
   };
-  // The wave's first token block.  Dense layout: always the straight-line
-  // full-block load, whatever t is: rows past the cold store read 0 through
-  // the range-checked vector offset, and tokens at or past t_end are masked
-  // by selects in attend_block, so no branch separates these loads from the
-  // query's and the query's wait need not drain them.  Paged: page ids past
-  // the split are not staged, so the load keeps its guard.
-  auto fetch_first = [&](BlockRegs& R, int t) {
-    if constexpr (PAGED) {
-      if (t < t_addr_end) fetch(R, t);
-    } else {
-      load_full_checked<CB>(R, rs, __builtin_amdgcn_readfirstlane(t), lane);
-    }
-  };
-  BlockRegs ra, rb;
   constexpr int kStep = kWaves * kBlk;  // tokens between a wave's consecutive blocks
   int t0 = t_begin + wave * kBlk;
   // The first token block is fetched right after the query's own loads are
   // issued: memory results retire in issue order, so the query rotation then
-  // waits only for the (cached) rotation matrix and query, not for the first
-  // codes from HBM, and the codes keep streaming in while it computes.
+  // waits only for the (cached) rotation matrix and query, not for codes from
+  // HBM, and the codes keep streaming in while it computes.
+  BlockRegs R;
+  auto fetch_first = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    const BlockOff o = off(t0);
+    load_keys<CB>(R, rs, o, lane);
+    load_norms(R.kn, rs.kn, o, lane);
+    load_norms(R.vn, rs.vn, o, lane);
+    load_values<CB>(R, rs, o, lane);
+    __builtin_amdgcn_sched_barrier(0);
+  };
   float c_lo = 0.f, c_hi = 0.f;
   uint32_t tab[4] = {0u, 0u, 0u, 0u};
   if constexpr (PERM) {
@@ -430,46 +453,48 @@ __global__ __launch_bounds__(kThreads, kSplitBlocksPerCU) void tq_attn_split_ker
   } else {
     const int cmax = P.ncent - 1;
     c_lo = P.centroids[min(tid & 15, cmax)];
-    c_hi = P.centroids[min(tid >> 4, cmax)];
+    c_hi = P.centroids[min((tid & 255) >> 4, cmax)];
   }
   // B operand of the score MFMA: rotated query x scale*log2(e), head
   // h = lane%16, dims 32*(lane/16) + 8*kb + position (permuted with PERM).
+  // The rotation's partial sums (rotate_query_hilo: s_o is free until the
+  // merge) are added, scaled and packed once per block, one pair of dims a
+  // thread, and every wave reads the operand from LDS.
   const int h = lane & 15, g = lane >> 4;
-  u32x4 qa[4];
+  float* const s_part = &s_o[0][0][0];
   {
-    // rows h >= G read head G - 1 and are zeroed: unconditional loads
-    float4 f[8];
+    float4 pik[2][2];
+    load_pik_operand(P.PiK, wave, lane, pik);
+    u32x4 qb;
     if constexpr (DECODE) {
       // The G query heads from the q|k|v partials: sums, fp16, RoPE at pos,
-      // then the rotation below.  Thread pairs (head e / 64, dims e % 64 and
-      // e % 64 + 64).  The last split block also publishes the RoPE'd query
-      // (fp16, for the combine's hot-window scores) and puts the new key and
-      // value into their ring slot; evict_kernel has already quantized the
-      // token that slot held.
+      // then the rotation below.  Items 0 .. 64 G - 1: pairs (head e / 64, dims
+      // e % 64 and e % 64 + 64); 64 more: the new key's pairs; 64 more: the new
+      // value's.  The last split block also publishes the RoPE'd query (fp16,
+      // for the combine's hot-window scores) and puts the new key and value
+      // into their ring slot; evict_kernel has already quantized the token that
+      // slot held.  A thread's first kPre chunk partials (both dims of its item)
+      // come from clamped, always valid addresses, without a branch, ahead of
+      // the codes, so that no path drains the codes' loads before the query is
+      // ready.
       __shared__ float s_q[16][kD];
-      float4 pik[8][2];
-      load_pik_operand(P.PiK, wave, lane, pik);  // in flight while the partials are summed
       const int pos = __builtin_amdgcn_readfirstlane(*P.pos);
       const uint16_t* cos_row = P.rope_cos + static_cast<size_t>(pos) * kD;
       const uint16_t* sin_row = P.rope_sin + static_cast<size_t>(pos) * kD;
       const bool writer = split == P.nsplit - 1;
-      // this thread's first query element: its first kPre chunk partials (both
-      // dims of the RoPE pair) from clamped, always valid addresses, ahead of
-      // the codes; the rest of the chunks and elements are loaded after them
+      const int nq = G * (kD / 2), nitems = nq + kD;
+      const size_t slot = (static_cast<size_t>(kvh) * P.hot_cap + pos % P.hot_cap) * kD;
       constexpr int kPre = QPRE;
       float pre0[kPre], pre1[kPre];
-      uint16_t rc0, rc1, rs0, rs1;  // its RoPE factors
+      const int e0 = min(tid, nitems - 1), dd0 = e0 % (kD / 2);
+      const uint16_t rc0 = cos_row[dd0], rc1 = cos_row[dd0 + kD / 2], rs0 = sin_row[dd0], rs1 = sin_row[dd0 + kD / 2];
+      auto column = [&](int e) { return (e < nq ? kvh * G + e / (kD / 2) : kvh) * kD + e % (kD / 2); };
+      auto source = [&](int e) { return e < nq ? P.pq : e < nq + kD / 2 ? P.pk : P.pv; };
       {
-        const int e = min(tid, G * (kD / 2) - 1);
-        const int dd = e % (kD / 2);
-        rc0 = cos_row[dd];
-        rc1 = cos_row[dd + kD / 2];
-        rs0 = sin_row[dd];
-        rs1 = sin_row[dd + kD / 2];
-        const int col = (kvh * G + e / (kD / 2)) * kD + dd;
-        const float* p0 = P.pq + static_cast<size_t>(col / kGemvBN) * P.nchunk * kGemvBN + (col % kGemvBN);
-        const float* p1 = P.pq + static_cast<size_t>((col + kD / 2) / kGemvBN) * P.nchunk * kGemvBN +
-                          ((col + kD / 2) % kGemvBN);
+        const int c0 = column(e0), c1 = c0 + kD / 2;
+        const float* src = source(e0);
+        const float* p0 = src + static_cast<size_t>(c0 / kGemvBN) * P.nchunk * kGemvBN + (c0 % kGemvBN);
+        const float* p1 = src + static_cast<size_t>(c1 / kGemvBN) * P.nchunk * kGemvBN + (c1 % kGemvBN);
 #pragma unroll
         for (int i = 0; i < kPre; ++i) {
           const size_t o = static_cast<size_t>(min(i, P.nchunk - 1)) * kGemvBN;
@@ -477,29 +502,9 @@ __global__ __launch_bounds__(kThreads, kSplitBlocksPerCU) void tq_attn_split_ker
           pre1[i] = p1[o];
         }
       }
-      // the new key (threads 0..63, pair (t, t + 64)) and value (threads
-      // 64..127) of the ring write, which only the last split block stores:
-      // loaded by every block, without a branch, so that no path drains the
-      // codes' loads before the query is ready
-      float prk0[kPre], prk1[kPre];
-      {
-        const int t = tid & (kD - 1);
-        const float* src = t < kD / 2 ? P.pk : P.pv;
-        const int c0 = kvh * kD + (t & (kD / 2 - 1)), c1 = c0 + kD / 2;
-        const float* p0 = src + static_cast<size_t>(c0 / kGemvBN) * P.nchunk * kGemvBN + (c0 % kGemvBN);
-        const float* p1 = src + static_cast<size_t>(c1 / kGemvBN) * P.nchunk * kGemvBN + (c1 % kGemvBN);
-#pragma unroll
-        for (int i = 0; i < kPre; ++i) {
-          const size_t o = static_cast<size_t>(min(i, P.nchunk - 1)) * kGemvBN;
-          prk0[i] = p0[o];
-          prk1[i] = p1[o];
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);  // keep these loads ahead of the codes' (results retire in order)
-      fetch_first(ra, t0);
-      for (int e = tid; e < G * (kD / 2); e += kThreads) {
-        const int hh = e / (kD / 2), dd = e % (kD / 2);
-        const int col = (kvh * G + hh) * kD + dd;
+      fetch_first();
+      for (int e = tid; e < nitems; e += kThreads) {
+        const int c0 = column(e), dd = e % (kD / 2);
         float x0, x1, o0, o1;
         if (e == tid && P.nchunk <= kPre) {  // column_sum2's order: chunk order from 0
           x0 = 0.f;
@@ -511,95 +516,57 @@ __global__ __launch_bounds__(kThreads, kSplitBlocksPerCU) void tq_attn_split_ker
           }
           rope_pair_v(x0, x1, rc0, rc1, rs0, rs1, o0, o1);
         } else {
-          column_sum2(P.pq, col, col + kD / 2, P.nchunk, x0, x1);
+          column_sum2(source(e), c0, c0 + kD / 2, P.nchunk, x0, x1);
           rope_pair(x0, x1, cos_row, sin_row, dd, o0, o1);
         }
-        s_q[hh][dd] = o0;
-        s_q[hh][dd + kD / 2] = o1;
-        if (writer) {
-          P.q16[col] = f2h(o0);
-          P.q16[col + kD / 2] = f2h(o1);
-        }
-      }
-      if (writer) {
-        const size_t slot = (static_cast<size_t>(kvh) * P.hot_cap + pos % P.hot_cap) * kD;
-        float x0 = 0.f, x1 = 0.f;
-        if (tid < kD) {  // column_sum2's order: chunk order from 0
-          if (P.nchunk <= kPre) {
-#pragma unroll
-            for (int i = 0; i < kPre; ++i) {
-              x0 += i < P.nchunk ? prk0[i] : 0.f;
-              x1 += i < P.nchunk ? prk1[i] : 0.f;
-            }
-          } else {
-            const int c0 = kvh * kD + (tid & (kD / 2 - 1));
-            column_sum2(tid < kD / 2 ? P.pk : P.pv, c0, c0 + kD / 2, P.nchunk, x0, x1);
+        if (e < nq) {
+          s_q[e / (kD / 2)][dd] = o0;
+          s_q[e / (kD / 2)][dd + kD / 2] = o1;
+          if (writer) {
+            P.q16[c0] = f2h(o0);
+            P.q16[c0 + kD / 2] = f2h(o1);
           }
-        }
-        if (tid < kD / 2) {  // key pair (tid, tid + 64), RoPE'd (the factors of query element tid)
-          float o0, o1;
-          if (P.nchunk <= kPre)
-            rope_pair_v(x0, x1, rc0, rc1, rs0, rs1, o0, o1);
-          else
-            rope_pair(x0, x1, cos_row, sin_row, tid, o0, o1);
-          P.k_ring[slot + tid] = f2h(o0);
-          P.k_ring[slot + tid + kD / 2] = f2h(o1);
-        } else if (tid < kD) {  // value dims (tid - 64, tid): no RoPE
-          const int dd = tid - kD / 2;
-          P.v_ring[slot + dd] = f2h(x0);
-          P.v_ring[slot + dd + kD / 2] = f2h(x1);
+        } else if (writer) {  // the value takes no RoPE
+          const bool key = e < nq + kD / 2;
+          uint16_t* ring = (key ? P.k_ring : P.v_ring) + slot;
+          ring[dd] = f2h(key ? o0 : x0);
+          ring[dd + kD / 2] = f2h(key ? o1 : x1);
         }
       }
       __syncthreads();
-      LKV_SPLIT_STAMP(4);
-      u32x4 qb = u32x4{0u, 0u, 0u, 0u};
+      qb = u32x4{0u, 0u, 0u, 0u};
       if (h < G) {
-        const float* q = &s_q[h][32 * wave + 8 * g];
+        const float* q = &s_q[h][32 * (wave & 3) + 8 * g];
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj)
           qb[jj] = static_cast<uint32_t>(f2h(q[2 * jj])) | (static_cast<uint32_t>(f2h(q[2 * jj + 1])) << 16);
       }
-      rotate_query_hilo_loaded(pik, qb, wave, lane, &s_o[0][0][0], kORow, f);
-      __syncthreads();  // s_o is written again by the merge
-      LKV_SPLIT_STAMP(5);
-    } else if (P.PiK != nullptr) {
-      // q_rot on MFMA (rotate_query_hilo), overlapping the first block's
-      // loads; s_o is free until the merge.
-      float4 pik[8][2];
-      load_pik_operand(P.PiK, wave, lane, pik);
-      u32x4 qb;
-      {
-        const uint4 u = *reinterpret_cast<const uint4*>(
-            P.q + (static_cast<size_t>(b) * P.Hq + kvh * G + min(h, G - 1)) * kD + 32 * wave + 8 * g);
-        qb = h < G ? u32x4{u.x, u.y, u.z, u.w} : u32x4{0u, 0u, 0u, 0u};
-      }
-      fetch_first(ra, t0);
-      LKV_SPLIT_STAMP(4);
-      rotate_query_hilo_loaded(pik, qb, wave, lane, &s_o[0][0][0], kORow, f);
-      __syncthreads();  // s_o is written again by the merge
-      LKV_SPLIT_STAMP(5);
     } else {
-      const float4* src = reinterpret_cast<const float4*>(
-          P.qrot + (static_cast<size_t>(b) * P.Hq + kvh * G + min(h, G - 1)) * kD + 32 * g);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) f[i] = src[i];
-      fetch_first(ra, t0);
+      // rows h >= G read head G - 1 and are zeroed: unconditional loads
+      const uint4 u = *reinterpret_cast<const uint4*>(
+          P.q + (static_cast<size_t>(b) * P.Hq + kvh * G + min(h, G - 1)) * kD + 32 * (wave & 3) + 8 * g);
+      qb = h < G ? u32x4{u.x, u.y, u.z, u.w} : u32x4{0u, 0u, 0u, 0u};
+      fetch_first();
     }
-    if constexpr (!PERM) s_lut[tid] = pack2h(c_lo, c_hi);
-    const float sl = P.scale_log2;
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      const float4 f0 = f[2 * kb], f1 = f[2 * kb + 1];
-      const float x[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
-      u32x4 v;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int d0 = PERM ? kPermDim[2 * j] : 2 * j, d1 = PERM ? kPermDim[2 * j + 1] : 2 * j + 1;
-        v[j] = pack2h(x[d0] * sl, x[d1] * sl);
-      }
-      qa[kb] = h < G ? v : u32x4{0u, 0u, 0u, 0u};
-    }
+    LKV_SPLIT_STAMP(4);
+    rotate_query_partials(pik, qb, wave, lane, s_part, kORow);
   }
+  if constexpr (!PERM)
+    if (tid < 256) s_lut[tid] = pack2h(c_lo, c_hi);
+  __syncthreads();
+  {
+    const int hh = tid >> 6, pp = tid & 63, j = pp & 3;  // positions 2 pp, 2 pp + 1 of head hh
+    const int d0 = 8 * (pp >> 2) + (PERM ? (j < 2 ? 4 * j : 4 * j - 7) : 2 * j), d1 = d0 + (PERM ? 2 : 1);  // kPermDim
+    uint32_t v = 0u;
+    if (hh < G)
+      v = pack2h(rotated_sum(s_part, kORow, hh, d0) * P.scale_log2, rotated_sum(s_part, kORow, hh, d1) * P.scale_log2);
+    *reinterpret_cast<uint32_t*>(&s_qa[hh][2 * pp]) = v;
+  }
+  __syncthreads();
+  LKV_SPLIT_STAMP(5);
+  u32x4 qa[4];
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) qa[kb] = *reinterpret_cast<const u32x4*>(&s_qa[h][32 * g + 8 * kb]);
 
   const int L = min(seq_len, P.max_len);
   const int cold_len = max(0, L - P.hot_cap);
@@ -621,41 +588,26 @@ __global__ __launch_bounds__(kThreads, kSplitBlocksPerCU) void tq_attn_split_ker
   S.l = 0.f;
 #pragma unroll
   for (int t = 0; t < 8; ++t) S.o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if constexpr (!PERM) __syncthreads();  // LUT ready
-  // Two register sets in turn: the next block's loads are in flight while
-  // the current one is computed, with no register copies between them.
-  // (Loading both sets in the prologue measured 29.0 -> 29.5-30.1 us at
-  // config 4 and +0.2 % at config 5: the loop is not waiting on the second
-  // block's loads.)
-  while (t0 < t_end) {
-    const int t1 = t0 + kStep;
-    if (t1 < t_end) fetch(rb, t1);
-    attend<PERM>(ra, t0, t_end, qa, tab, s_lut, lane, S);
-    if (t1 >= t_end) break;
-    const int t2 = t1 + kStep;
-    if (t2 < t_end) fetch(ra, t2);
-    attend<PERM>(rb, t1, t_end, qa, tab, s_lut, lane, S);
-    t0 = t2;
-  }
+  // The loop has one exit and its body no branch around a load: a second path
+  // to its head would let the compiler wait for every load in flight there.
+  for (; t0 + kBlk <= t_end; t0 += kStep)
+    attend_block<PERM, CB, false>(R, t0, t_end, qa, tab, s_lut, lane, S, rs, off(t0 + kStep));
+  if (t0 < t_end) attend_block<PERM, CB, true>(R, t0, t_end, qa, tab, s_lut, lane, S, rs, BlockOff{});
   LKV_SPLIT_STAMP(2);
 
-  // ---- merge the 4 waves of the block through LDS.  A wave that had no
+  // ---- merge the waves of the block through LDS.  A wave that had no
   // block keeps m = -inf, l = 0, o = 0.
   const float lsum = xgroup_sum(S.l);
   if (g == 0) {
     s_m[wave][h] = S.m;
     s_l[wave][h] = lsum;
   }
+  if (h < G)
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     float4* dst = reinterpret_cast<float4*>(&s_o[wave][h][32 * g + 8 * i]);
-    if constexpr (PERM) {  // dims 0..7 sit in tiles 0, 4, 1, 5, 2, 6, 3, 7
-      dst[0] = make_float4(S.o[0][i], S.o[4][i], S.o[1][i], S.o[5][i]);
-      dst[1] = make_float4(S.o[2][i], S.o[6][i], S.o[3][i], S.o[7][i]);
-    } else {
-      dst[0] = make_float4(S.o[0][i], S.o[1][i], S.o[2][i], S.o[3][i]);
-      dst[1] = make_float4(S.o[4][i], S.o[5][i], S.o[6][i], S.o[7][i]);
-    }
+    dst[0] = make_float4(S.o[0][i], S.o[1][i], S.o[2][i], S.o[3][i]);
+    dst[1] = make_float4(S.o[4][i], S.o[5][i], S.o[6][i], S.o[7][i]);
   }
   __syncthreads();
   for (int e = tid; e < G * kD; e += kThreads) {
@@ -892,69 +844,34 @@ __global__ __launch_bounds__(kCombThreads, 4) void tq_attn_combine_kernel(AttnPa
   LKV_COMB_STAMP(3);
 }
 
-constexpr int kSplitGran = kWaves * kBlk;  // tokens one pass of a block covers
+constexpr int kSplitGran = 256;  // tokens of a split are a multiple of this (half a pass of a block)
 
-// Split count that gives ~4 blocks per CU (each wave's token loop is a
-// latency chain, so more resident waves overlap more of them), at most
-// kMaxSplits - 1.
-// Tuning knobs, read once.  LKV_ATTN_SPLIT_TARGET=k: aim for k split blocks
-// per CU (default: the resident count, kSplitBlocksPerCU).  LKV_ATTN_QROT=kernel:
-// lkv_tq_decode_attn rotates the query in its own launch instead of in every
-// split block's prologue.
+// Tuning knobs, read once.  LKV_ATTN_SPLIT_TARGET=k: k split blocks per CU instead of attn_plan's choice.
+// LKV_ATTN_MIN_SPLIT_TOKENS=n: at least n cold tokens per split (default 256: each split block repeats the query
+// prologue).
 int attn_split_target() {
   static const int k = [] {
     const char* env = getenv("LKV_ATTN_SPLIT_TARGET");
     const int v = env ? atoi(env) : 0;
-    return v > 0 && v <= 16 ? v : kSplitBlocksPerCU;
+    return v > 0 && v <= 16 ? v : 0;
   }();
   return k;
 }
-// At least 256 cold tokens per split (two passes of a block): at B = 1 the
-// target split count would give 128-token splits, and each split block repeats
-// the query prologue (q partial sums, RoPE, the rotation with PiK); 256 measured
-// 392 vs 384 tok/s at config 5 (512: 383, 1024: 365).  B >= 4 already gets
-// longer splits.  LKV_ATTN_MIN_SPLIT_TOKENS=n overrides (0: none).
 int64_t attn_min_split_tokens() {
   static const int64_t k = [] {
     const char* env = getenv("LKV_ATTN_MIN_SPLIT_TOKENS");
-    const long v = env ? atol(env) : 256;
+    const long v = env ? atol(env) : kSplitGran;
     return static_cast<int64_t>(v > 0 && v <= (1 << 20) ? v : 0);
   }();
   return k;
 }
-bool attn_qrot_kernel() {
-  static const bool k = [] {
-    const char* env = getenv("LKV_ATTN_QROT");
-    return env && env[0] == 'k';
-  }();
-  return k;
-}
-
-// q_rot = q @ PiK^T in a launch of its own: one 4-wave block per (kv head, batch).
-__global__ __launch_bounds__(kThreads) void qrot_hilo_kernel(const uint16_t* __restrict__ q,
-                                                             const float* __restrict__ PiK, float* __restrict__ qrot,
-                                                             int Hq, int Hkv) {
-  __shared__ __align__(16) float s_part[4 * 16 * kORow];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int kvh = blockIdx.x, b = blockIdx.y, G = Hq / Hkv;
-  const int h = lane & 15, g = lane >> 4;
-  const uint4 u = *reinterpret_cast<const uint4*>(q + (static_cast<size_t>(b) * Hq + kvh * G + min(h, G - 1)) * kD +
-                                                  32 * wave + 8 * g);
-  const u32x4 qb = h < G ? u32x4{u.x, u.y, u.z, u.w} : u32x4{0u, 0u, 0u, 0u};
-  float4 out[8];
-  rotate_query_hilo(PiK, qb, wave, lane, s_part, kORow, out);
-  if (h < G && wave == 0) {
-    float4* dst = reinterpret_cast<float4*>(qrot + (static_cast<size_t>(b) * Hq + kvh * G + h) * kD + 32 * g);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) dst[i] = out[i];
-  }
-}
-
-int64_t target_splits(int64_t B, int64_t Hkv) {
-  const int64_t target = attn_split_target() * static_cast<int64_t>(device_cu_count());
-  int64_t ns = (target + B * Hkv - 1) / (B * Hkv);
-  if (ns > kMaxSplits - 1) ns = kMaxSplits - 1;
-  return ns < 1 ? 1 : ns;
+// The most splits a (batch, kv head) is cut into: two blocks per CU over the whole launch (the workspace holds
+// their records whatever is chosen).
+int64_t max_splits(int64_t B, int64_t Hkv) {
+  const int k = attn_split_target();
+  const int64_t target = (k ? k : 2) * static_cast<int64_t>(device_cu_count());
+  const int64_t ns = (target + B * Hkv - 1) / (B * Hkv);
+  return ns > kMaxSplits - 1 ? kMaxSplits - 1 : ns < 1 ? 1 : ns;
 }
 
 }  // namespace
@@ -963,10 +880,29 @@ AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t max_len, int64_t 
   AttnPlan p{};
   const int64_t G = Hkv > 0 ? Hq / Hkv : 1;
   const int64_t cold_max = max_len > hot_cap ? max_len - hot_cap : 0;
-  int64_t ns_cap = target_splits(B, Hkv);
-  int64_t ts = (cold_max + ns_cap - 1) / ns_cap;
-  if (ts < attn_min_split_tokens()) ts = attn_min_split_tokens();
-  ts = (ts + kSplitGran - 1) / kSplitGran * kSplitGran;
+  int64_t ns_cap = max_splits(B, Hkv);
+  auto tokens_of = [&](int64_t n) {
+    int64_t t = (cold_max + n - 1) / n;
+    if (t < attn_min_split_tokens()) t = attn_min_split_tokens();
+    return (t + kSplitGran - 1) / kSplitGran * kSplitGran;
+  };
+  // One block is resident per CU, so a launch takes whole rounds of the CUs, each the tokens of a split plus the
+  // block's fixed part (prologue, merge and record: as long as kFixed tokens).  Candidates are the split counts that
+  // fill r rounds, r up to ns_cap's; of those with the least time, the smallest.
+  constexpr int64_t kFixed = 1024;
+  int64_t ts = tokens_of(ns_cap);
+  if (!attn_split_target()) {
+    const int64_t cus = device_cu_count(), bh = B * Hkv;
+    int64_t best = -1;
+    for (int64_t r = (bh + cus - 1) / cus; r <= (bh * ns_cap + cus - 1) / cus; ++r) {
+      const int64_t n = r * cus / bh, t = tokens_of(n < ns_cap ? n : ns_cap), blocks = bh * ((cold_max + t - 1) / t);
+      const int64_t cost = (blocks + cus - 1) / cus * (t + kFixed);
+      if (best < 0 || cost < best) {
+        best = cost;
+        ts = t;
+      }
+    }
+  }
   if (ts < kSplitGran) ts = kSplitGran;
   if (max_split_tokens > 0 && ts > max_split_tokens) ts = max_split_tokens / kSplitGran * kSplitGran;
   int64_t ns = (cold_max + ts - 1) / ts;
@@ -984,7 +920,6 @@ AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t max_len, int64_t 
 
 int attn_launch(const AttnCall& c, const AttnPlan& pl, hipStream_t st) {
   AttnParams P;
-  P.qrot = c.qrot;
   P.q = c.q;
   P.k_codes = c.k_codes;
   P.k_norms = c.k_norms;
@@ -1139,19 +1074,8 @@ extern "C" int lkv_tq_decode_attn(const void* q, const uint8_t* k_codes, const f
   LKV_REQUIRE(workspace_bytes >= pl.total, "tq_decode_attn: workspace of %zu bytes required, got %zu", pl.total,
               workspace_bytes);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  char* ws = static_cast<char*>(workspace);
   AttnCall c{};
-  if (attn_qrot_kernel()) {
-    float* qr = reinterpret_cast<float*>(ws + pl.qrot_off);
-    hipLaunchKernelGGL(qrot_hilo_kernel, dim3(static_cast<unsigned>(Hkv), static_cast<unsigned>(B)), dim3(kThreads), 0,
-                       st, static_cast<const uint16_t*>(q), PiK, qr, static_cast<int>(Hq), static_cast<int>(Hkv));
-    LKV_LAUNCH_CHECK("tq_decode_attn q rotation");
-    c.qrot = qr;
-    c.PiK = nullptr;
-  } else {
-    c.qrot = nullptr;
-    c.PiK = PiK;  // the split kernel rotates the query
-  }
+  c.PiK = PiK;
   c.q = static_cast<const uint16_t*>(q);
   c.k_codes = k_codes;
   c.k_norms = k_norms;
@@ -1162,7 +1086,7 @@ extern "C" int lkv_tq_decode_attn(const void* q, const uint8_t* k_codes, const f
   c.PiV = PiV;
   c.centroids = centroids;
   c.seq_len = seq_len;
-  c.partials = reinterpret_cast<float*>(ws + pl.part_off);
+  c.partials = reinterpret_cast<float*>(static_cast<char*>(workspace) + pl.part_off);
   c.out = static_cast<uint16_t*>(out);
   c.scale = scale;
   c.max_len = max_len;
@@ -1226,7 +1150,6 @@ extern "C" int lkv_tq_paged_decode_attn(const void* q, const uint8_t* k_codes, c
   LKV_REQUIRE(workspace_bytes >= pl.total, "tq_paged_decode_attn: workspace of %zu bytes required, got %zu",
               pl.total, workspace_bytes);
   AttnCall c{};
-  c.qrot = nullptr;
   c.PiK = PiK;
   c.q = static_cast<const uint16_t*>(q);
   c.k_codes = k_codes;

@@ -13,6 +13,14 @@ __device__ __forceinline__ uint32_t pack2h(float lo, float hi) {
   return static_cast<uint32_t>(f2h(lo)) | (static_cast<uint32_t>(f2h(hi)) << 16);
 }
 
+// fp16(a b) in the low half, fp16(c d) in the high half, each product rounded once.
+__device__ __forceinline__ uint32_t mul2h(float a, float b, float c, float d) {
+  uint32_t r;
+  asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(r) : "v"(a), "v"(b));
+  asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(r) : "v"(c), "v"(d));
+  return r;
+}
+
 // 2^x on the hardware exp (v_exp_f32); arguments here are <= 0 and results
 // below 2^-126 flush to 0, which only drops contributions < 1e-38 of the max.
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -90,30 +98,46 @@ __device__ __forceinline__ uint32_t nib_from1(uint32_t x) {
   t = (t | (t << 6)) & 0x03030303u;
   return (t | (t << 3)) & 0x11111111u;
 }
-// Dims 32k .. 32k+31 of a code row as 4 nibble dwords; voff/soff address the
-// row's byte 4*CB*k.
+// Dims 32k .. 32k+31 of a code row (voff: the row's byte 4*CB*k) as loaded, and widened to 4 nibble dwords.  The two
+// are apart so that a load can stay in flight until its codes are used.
 template <int CB>
-__device__ __forceinline__ u32x4 load_codes32(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+__device__ __forceinline__ u32x4 load_raw32(__amdgpu_buffer_rsrc_t r, int voff) {
   if constexpr (CB == 4) {
-    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
   } else if constexpr (CB == 2) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
-    const uint32_t lo = v[0], hi = v[1];
-    return u32x4{nib_from2(lo), nib_from2(lo >> 16), nib_from2(hi), nib_from2(hi >> 16)};
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0);
+    return u32x4{v[0], v[1], 0u, 0u};
   } else {
-    const uint32_t v = __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
-    return u32x4{nib_from1(v), nib_from1(v >> 8), nib_from1(v >> 16), nib_from1(v >> 24)};
+    return u32x4{__builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0), 0u, 0u, 0u};
   }
 }
-// Dims 8k .. 8k+7 of a code row as one nibble dword (row byte CB*k).
 template <int CB>
-__device__ __forceinline__ uint32_t load_codes8(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+__device__ __forceinline__ uint32_t widen32(const u32x4& v, int k) {
   if constexpr (CB == 4)
-    return __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
+    return v[k];
   else if constexpr (CB == 2)
-    return nib_from2(__builtin_amdgcn_raw_buffer_load_b16(r, voff, soff, 0));
+    return nib_from2(v[k >> 1] >> (16 * (k & 1)));
   else
-    return nib_from1(__builtin_amdgcn_raw_buffer_load_b8(r, voff, soff, 0));
+    return nib_from1(v[0] >> (8 * k));
+}
+// Dims 8k .. 8k+7 of a code row (row byte CB*k), the same way: one nibble dword.
+template <int CB>
+__device__ __forceinline__ uint32_t load_raw8(__amdgpu_buffer_rsrc_t r, int voff) {
+  if constexpr (CB == 4)
+    return __builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0);
+  else if constexpr (CB == 2)
+    return __builtin_amdgcn_raw_buffer_load_b16(r, voff, 0, 0);
+  else
+    return __builtin_amdgcn_raw_buffer_load_b8(r, voff, 0, 0);
+}
+template <int CB>
+__device__ __forceinline__ uint32_t widen8(uint32_t v) {
+  if constexpr (CB == 4)
+    return v;
+  else if constexpr (CB == 2)
+    return nib_from2(v);
+  else
+    return nib_from1(v);
 }
 
 // Buffer resource over `bytes` bytes at base (raw addressing, stride 0).

@@ -275,13 +275,6 @@ __device__ __forceinline__ float xhalf_sum(float v) {
   const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(a[0]) + __uint_as_float(a[1]);
 }
-// fp16(a b) in the low half, fp16(c d) in the high half, each product rounded once.
-__device__ __forceinline__ uint32_t mul2h(float a, float b, float c, float d) {
-  uint32_t r;
-  asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(r) : "v"(a), "v"(b));
-  asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(r) : "v"(c), "v"(d));
-  return r;
-}
 __device__ __forceinline__ void split_hl(float x, uint16_t& hi, uint16_t& lo) {
   hi = f2h(x);
   lo = f2h((x - h2f(hi)) * 2048.f);
@@ -366,12 +359,12 @@ __global__ __launch_bounds__(kPThreads, 1) void tq_prefill_attn_kernel(PrefillPa
     const int n = __builtin_amdgcn_readfirstlane(max(0, min(kKT, cold_len - t0)));  // (the clamp compiles to vector code)
     const __amdgpu_buffer_rsrc_t rc = make_rsrc(cod + static_cast<size_t>(t0) * RB, n * RB);
     if (key_thr) {
-      const u32x4 w = load_codes32<CB>(rc, voff, 0);
+      const u32x4 w = load_raw32<CB>(rc, voff);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) tw[u][e] = w[e];
+      for (int e = 0; e < 4; ++e) tw[u][e] = widen32<CB>(w, e);
     } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) tw[u][e] = load_codes8<CB>(rc, voff + e * RB, 0);
+      for (int e = 0; e < 4; ++e) tw[u][e] = widen8<CB>(load_raw8<CB>(rc, voff + e * RB));
     }
     if (nrm_thr)
       tn[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(make_rsrc(norms + t0, n * 4), 4 * lane, 0, 0));
