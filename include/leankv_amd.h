@@ -564,6 +564,17 @@ int lkv_tq_cache_evict(const lkv_cache_layer* layers, int64_t n_layers, int64_t 
 int lkv_rmsnorm(const void* x, const void* w, float eps, int64_t M, int64_t Z, void* y, void* stream);
 
 /*
+ * The start of a decode step of B rows at one position, one launch:
+ * x[b] = embed[tok[b]] (embed fp16 [vocab][Z], Z % 8 == 0), h = lkv_rmsnorm of
+ * x with norm_w and eps bit for bit, and the position's RoPE factors
+ * cos_row / sin_row [128] from the fp16 tables [max_len][128].  Tokens and the
+ * device position pos are clamped into the tables.  B < 65536.
+ */
+int lkv_batched_begin(const void* embed, int64_t vocab, const int64_t* tok, const void* norm_w, float eps, int64_t B,
+                      int64_t Z, const void* cos_tab, const void* sin_tab, int64_t max_len, const int32_t* pos,
+                      void* x, void* h, void* cos_row, void* sin_row, void* stream);
+
+/*
  * RoPE of B decode rows in place, one launch for the query and the key:
  * q fp16 [B][Hq][128], k fp16 [B][Hkv][128] (contiguous), cos_row / sin_row
  * the 128 fp16 factors of the tokens' position.  HF apply_rotary_pos_emb on

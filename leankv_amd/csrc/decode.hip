@@ -224,6 +224,38 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_kernel(const uint16_t* __res
   if (z < Z) y[row + z] = f2h(rms_apply(x[row + z], w[z], rstd));
 }
 
+// The start of a step of B rows: block (j, b) writes columns [256 j, 256 j + 256)
+// of x = embed[tok[b]] and of its RMSNorm (each block reads the whole row for
+// its rstd, as rmsnorm_kernel does), and the first block copies the position's
+// RoPE factors.  Token and position are clamped into the tables (begin_kernel).
+// A few KB: bound by its launch.  Three gathers and lkv_rmsnorm took 26 us of a
+// 16-row step, four launches of 4.5 to 12 us; this one takes 5.
+__global__ __launch_bounds__(kThreads) void batched_begin_kernel(
+    const uint16_t* __restrict__ embed, int64_t vocab, const int64_t* __restrict__ tok, const uint16_t* __restrict__ w,
+    float eps, int Z, const uint16_t* __restrict__ cos_tab, const uint16_t* __restrict__ sin_tab, int64_t max_len,
+    const int32_t* __restrict__ pos, uint16_t* __restrict__ x, uint16_t* __restrict__ h, uint16_t* __restrict__ cos_row,
+    uint16_t* __restrict__ sin_row) {
+  __shared__ float s_wsum[kThreads / kWave];
+  int64_t t = tok[blockIdx.y];
+  t = t < 0 ? 0 : (t >= vocab ? vocab - 1 : t);
+  const uint16_t* row = embed + t * Z;
+  const float rstd = rms_rstd(row, Z, eps, s_wsum);
+  const int z = blockIdx.x * kThreads + threadIdx.x;
+  const size_t o = static_cast<size_t>(blockIdx.y) * Z + z;
+  if (z < Z) {
+    const uint16_t v = row[z];
+    x[o] = v;
+    h[o] = f2h(rms_apply(v, w[z], rstd));
+  }
+  if (blockIdx.x == 0 && blockIdx.y == 0) {
+    static_assert(kThreads == 2 * kD, "one factor a thread");
+    int64_t p = *pos;
+    p = p < 0 ? 0 : (p >= max_len ? max_len - 1 : p);
+    const int d = threadIdx.x % kD;
+    (threadIdx.x < kD ? cos_row : sin_row)[d] = (threadIdx.x < kD ? cos_tab : sin_tab)[p * kD + d];
+  }
+}
+
 // The token leaving the hot window at this step, for up to kEvictLayers
 // layers per launch: the layer table travels as kernel arguments.
 constexpr int kEvictLayers = 32;
@@ -388,6 +420,26 @@ __global__ __launch_bounds__(kThreads) void argmax_kernel(const Cand* __restrict
 }  // namespace lkv
 
 using namespace lkv;
+
+extern "C" int lkv_batched_begin(const void* embed, int64_t vocab, const int64_t* tok, const void* norm_w, float eps,
+                                 int64_t B, int64_t Z, const void* cos_tab, const void* sin_tab, int64_t max_len,
+                                 const int32_t* pos, void* x, void* h, void* cos_row, void* sin_row, void* stream) {
+  LKV_REQUIRE(Z > 0 && Z % 8 == 0 && Z < (1 << 30), "batched_begin: Z=%lld must be a positive multiple of 8",
+              (long long)Z);
+  LKV_REQUIRE(B >= 0 && B < 65536, "batched_begin: B=%lld rows exceeds 65535", (long long)B);
+  LKV_REQUIRE(vocab > 0 && max_len > 0, "batched_begin: empty embedding or RoPE table");
+  if (B == 0) return LKV_OK;
+  LKV_REQUIRE(embed && tok && norm_w && cos_tab && sin_tab && pos && x && h && cos_row && sin_row && aligned16(embed),
+              "batched_begin: null pointer or embed not 16-byte aligned");
+  const dim3 grid(static_cast<unsigned>((Z + kThreads - 1) / kThreads), static_cast<unsigned>(B));
+  hipLaunchKernelGGL(batched_begin_kernel, grid, dim3(kThreads), 0, static_cast<hipStream_t>(stream),
+                     static_cast<const uint16_t*>(embed), vocab, tok, static_cast<const uint16_t*>(norm_w), eps,
+                     static_cast<int>(Z), static_cast<const uint16_t*>(cos_tab), static_cast<const uint16_t*>(sin_tab),
+                     max_len, pos, static_cast<uint16_t*>(x), static_cast<uint16_t*>(h),
+                     static_cast<uint16_t*>(cos_row), static_cast<uint16_t*>(sin_row));
+  LKV_LAUNCH_CHECK("batched_begin");
+  return LKV_OK;
+}
 
 extern "C" int lkv_rmsnorm(const void* x, const void* w, float eps, int64_t M, int64_t Z, void* y, void* stream) {
   LKV_REQUIRE(M >= 0 && Z > 0 && Z % 8 == 0 && Z < (1 << 30), "rmsnorm: Z=%lld must be a positive multiple of 8",

@@ -299,9 +299,13 @@ class BatchedEngine:
         self._ring = all(f is not None and f[0].shape[0] % 128 == 0 and f[1].shape[0] == self.Hkv * self.D
                          and f[2].shape[0] == self.Hkv * self.D for f in fus)
         self.tok = torch.zeros(B, dtype=torch.long, device=self.dev)
-        self.pos64 = torch.zeros(1, dtype=torch.long, device=self.dev)
-        self.pos32 = torch.zeros(1, dtype=torch.int32, device=self.dev)  # position of the token fed
-        self.len32 = torch.ones(1, dtype=torch.int32, device=self.dev)   # cache length after its append
+        # the position as parts of one buffer {int64 pos, pos, pos + 1}, moved by one launch
+        self._pos0 = torch.tensor([0, 0, 0, 1], dtype=torch.int32, device=self.dev)  # at position 0
+        self._pos1 = torch.tensor([1, 0, 1, 1], dtype=torch.int32, device=self.dev)  # what each position adds
+        self._pos = self._pos0.clone()
+        self.pos64 = self._pos[:2].view(torch.long)
+        self.pos32 = self._pos[2:3]  # position of the token fed
+        self.len32 = self._pos[3:]   # cache length after its append
         self.logits = None
         self.attn = torch.empty(B, self.Hq, self.D, dtype=torch.float16, device=self.dev)
         self.attn_ws = torch.empty(kernels.decode_attn_workspace_bytes(B, self.Hq, self.Hkv, self.max_len),
@@ -396,6 +400,13 @@ class BatchedEngine:
         out = residual + mlp(h)
         return out, (self._norm(norm, out) if norm is not None else None)
 
+    def _plain_embedding(self, emb) -> bool:
+        """Whether emb(tok) is the tokens' rows of its fp16 weight and nothing else."""
+        w = getattr(emb, "weight", None)
+        return (type(emb) is torch.nn.Embedding and "forward" not in emb.__dict__ and emb.max_norm is None
+                and not emb._forward_hooks and not emb._forward_pre_hooks and w.dtype == torch.float16
+                and w.device == self.tok.device and w.is_contiguous() and w.data_ptr() % 16 == 0)
+
     @staticmethod
     def _lkv_norm(mod, x: torch.Tensor) -> bool:
         """Whether _norm runs mod on x as lkv_rmsnorm."""
@@ -419,16 +430,21 @@ class BatchedEngine:
         from . import kernels
 
         m = self.model
-        x = m.model.embed_tokens(self.tok.view(self.B, 1))
-        cos = self.cos.index_select(0, self.pos64).unsqueeze(0)  # [1, 1, D]
-        sin = self.sin.index_select(0, self.pos64).unsqueeze(0)
         layers = m.model.layers
+        emb, norm = m.model.embed_tokens, layers[0].input_layernorm
+        if self._plain_embedding(emb) and self._fused_rope and self._lkv_norm(norm, emb.weight):
+            x, h, cos, sin = kernels.batched_begin(self.tok, emb.weight, norm.weight, norm.variance_epsilon, self.cos,
+                                                   self.sin, self.pos32)
+        else:
+            x = emb(self.tok.view(self.B, 1))
+            cos = self.cos.index_select(0, self.pos64).unsqueeze(0)  # [1, 1, D]
+            sin = self.sin.index_select(0, self.pos64).unsqueeze(0)
+            h = self._norm(norm, x)
         if self._ring:  # the token leaving every layer's hot window, before any layer writes its new one
             c = self.cache
             kernels.tq_cache_evict([(c._k_codes[i], c._k_norms[i], c._v_codes[i], c._v_norms[i], c._k_hot[i],
                                      c._v_hot[i], c.PiK[i], c.PiV[i]) for i in range(len(layers))],
                                    c.decision_boundaries, c.bits, self.pos32)
-        h = self._norm(layers[0].input_layernorm, x)
         for i, layer in enumerate(layers):
             nxt = layers[i + 1].input_layernorm if i + 1 < len(layers) else m.model.norm
             x, h = self._layer(i, layer, x, h, cos, sin, nxt)
@@ -436,15 +452,11 @@ class BatchedEngine:
         if self.logits is None:
             self.logits = torch.empty_like(logits)
         self.logits.copy_(logits)
-        self.pos64.add_(1)
-        self.pos32.add_(1)
-        self.len32.add_(1)
+        self._pos.add_(self._pos1)
 
     def set_position(self, pos: int) -> None:
         """The position of the next token fed (the cache length before it)."""
-        self.pos64.fill_(pos)
-        self.pos32.fill_(pos)
-        self.len32.fill_(pos + 1)
+        torch.add(self._pos0, self._pos1, alpha=int(pos), out=self._pos)
         self._host_pos = pos
 
     @torch.no_grad()

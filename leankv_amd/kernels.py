@@ -864,6 +864,29 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     return rms_norm_out(x, weight, eps, torch.empty_like(x, memory_format=torch.contiguous_format))
 
 
+def batched_begin(tok: torch.Tensor, embed: torch.Tensor, norm_w: torch.Tensor, eps: float, cos_tab: torch.Tensor,
+                  sin_tab: torch.Tensor, pos_dev: torch.Tensor):
+    """(x, h, cos, sin) at the start of a decode step of B rows, one launch (lkv_batched_begin): x [B, 1, Z] the
+    tokens' rows of embed [vocab, Z], h its RMSNorm as rms_norm gives it, cos / sin [1, 1, 128] the RoPE factors of
+    the int32 device position pos_dev; all fp16."""
+    require_cuda(tok, embed, norm_w, cos_tab, sin_tab, pos_dev)
+    if embed.dim() != 2 or any(t.dtype != torch.float16 or not t.is_contiguous()
+                               for t in (embed, norm_w, cos_tab, sin_tab)):
+        raise LeanKVError("batched_begin: embed, norm_w and the RoPE tables must be contiguous float16")
+    Z = embed.shape[1]
+    if norm_w.numel() != Z or cos_tab.dim() != 2 or cos_tab.shape[1] != HEAD_DIM or sin_tab.shape != cos_tab.shape:
+        raise LeanKVError("batched_begin: norm_w must have %d elements and the tables be [max_len, %d]" % (Z, HEAD_DIM))
+    if tok.dtype != torch.int64 or not tok.is_contiguous() or pos_dev.dtype != torch.int32 or pos_dev.numel() != 1:
+        raise LeanKVError("batched_begin: tok must be contiguous int64 and pos_dev one int32")
+    B = tok.numel()
+    x, h = embed.new_empty(B, 1, Z), embed.new_empty(B, 1, Z)
+    cos, sin = cos_tab.new_empty(1, 1, HEAD_DIM), cos_tab.new_empty(1, 1, HEAD_DIM)
+    check(_lib_handle().lkv_batched_begin(ptr(embed), embed.shape[0], ptr(tok), ptr(norm_w), float(eps), B, Z,
+                                          ptr(cos_tab), ptr(sin_tab), cos_tab.shape[0], ptr(pos_dev), ptr(x), ptr(h),
+                                          ptr(cos), ptr(sin), stream_handle(tok.device)), "lkv_batched_begin")
+    return x, h, cos, sin
+
+
 # ------------------------------------------------------------------ RoPE
 def rope_f16_(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> None:
     """In place: q [B, Hq, 128] and k [B, Hkv, 128] (contiguous fp16) rotated by the 128 fp16 factors of one
