@@ -457,7 +457,7 @@ __global__ __launch_bounds__(kThreads, 4 * kSplitBlocksPerCU) void tq_attn_split
   }
   // B operand of the score MFMA: rotated query x scale*log2(e), head
   // h = lane%16, dims 32*(lane/16) + 8*kb + position (permuted with PERM).
-  // The rotation's partial sums (rotate_query_hilo: s_o is free until the
+  // The rotation's partial sums (rotate_query_partials: s_o is free until the
   // merge) are added, scaled and packed once per block, one pair of dims a
   // thread, and every wave reads the operand from LDS.
   const int h = lane & 15, g = lane >> 4;
@@ -889,6 +889,9 @@ AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t max_len, int64_t 
   // One block is resident per CU, so a launch takes whole rounds of the CUs, each the tokens of a split plus the
   // block's fixed part (prologue, merge and record: as long as kFixed tokens).  Candidates are the split counts that
   // fill r rounds, r up to ns_cap's; of those with the least time, the smallest.
+  // Measured (us; this choice / just over one round / just over two): 16 x 8 kv heads x 4160 tokens 24.2 / 24.3 /
+  // 31.0, 20 x 8 x 4160 35.2 / 40.0 / 43.3, 40 x 8 x 2112 43.2 / 43.5 / 47.8, 3 x 8 x 4160 14.2 / 14.2 / 20.0, 1 x 8 x
+  // 32768 18.0 / 18.1 / 24.8.
   constexpr int64_t kFixed = 1024;
   int64_t ts = tokens_of(ns_cap);
   if (!attn_split_target()) {
@@ -911,7 +914,7 @@ AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t max_len, int64_t 
   p.nsplit = static_cast<int>(ns);
   p.split_tokens = static_cast<int>(ts);
   auto al = [](size_t v) { return (v + 255) / 256 * 256; };
-  p.qrot_off = kTicketBytes;  // keeps the shared workspace layout: ticket area first
+  p.qrot_off = kTicketBytes;  // room for a rotated query, no longer used: the workspace's layout and size stay
   p.part_off = p.qrot_off + al(static_cast<size_t>(B * Hq * kD) * 4);
   // sized for ns_cap so a workspace sized without hot_cap fits every call
   p.total = p.part_off + al(static_cast<size_t>(B * Hkv * ns_cap) * rec_floats(static_cast<int>(G)) * 4);
