@@ -339,7 +339,7 @@ __global__ __launch_bounds__(kThreads) void paged_split_kernel(PagedParams P) {
         for (int i = 0; i < 4; ++i) s[4 * tt + i] = c + 16 * tt + 4 * g + i < t_end ? sc[tt][i] : -INFINITY;
       float mx = s[0];
 #pragma unroll
-      for (int j = 1; j < 8; ++j) mx = vmax(mx, s[j]);
+      for (int j = 1; j < 8; ++j) mx = fmaxf(mx, s[j]);
       mx = xgroup_max(mx);
       const float mn = fmaxf(m, mx);  // finite: the chunk holds at least one token
       const float alpha = fast_exp2(m - mn);
@@ -404,7 +404,7 @@ __global__ __launch_bounds__(kThreads) void paged_split_kernel(PagedParams P) {
         for (int i = 0; i < 4; ++i) s[4 * tt + i] = c + 16 * tt + 4 * g + i < t_end ? sc[tt][i] : -INFINITY;
       float mx = s[0];
 #pragma unroll
-      for (int j = 1; j < 8; ++j) mx = vmax(mx, s[j]);
+      for (int j = 1; j < 8; ++j) mx = fmaxf(mx, s[j]);
       mx = xgroup_max(mx);
       const float mn = fmaxf(m, mx);  // finite: the chunk holds at least one token
       const float alpha = fast_exp2(m - mn);

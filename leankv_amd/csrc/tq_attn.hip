@@ -261,7 +261,7 @@ __device__ __forceinline__ void attend_block(BlockRegs& R, int t0, int t_end, co
     const float v = fmaf(acc[j >> 2][j & 3], R.kn[j >> 2][j & 3], -S.m);  // +inf in the first block (m = -inf)
     s[j] = valid(j) ? v : -INFINITY;
   }
-  const float tm = vmax(vmax3(vmax3(s[0], s[1], s[2]), s[3], s[4]), vmax3(s[5], s[6], s[7]));
+  const float tm = fmaxf(vmax3(vmax3(s[0], s[1], s[2]), s[3], s[4]), vmax3(s[5], s[6], s[7]));
   if (__builtin_amdgcn_ballot_w64(!(tm <= 0.f)) != 0) {
     float bm = -INFINITY;
 #pragma unroll

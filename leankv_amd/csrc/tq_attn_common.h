@@ -13,12 +13,13 @@ __device__ __forceinline__ uint32_t pack2h(float lo, float hi) {
   return static_cast<uint32_t>(f2h(lo)) | (static_cast<uint32_t>(f2h(hi)) << 16);
 }
 
-// fp16(a b) in the low half, fp16(c d) in the high half, each product rounded once.
+// fp16(a b) in the low half, fp16(c d) in the high half, each product rounded once: v_fma_mixlo / mixhi_f16, by the
+// compiler.  No arithmetic here is inline asm: the wait states that gfx950 needs between a v_exp_f32 and the vector
+// instruction that reads its result, a vector write and an MFMA or permlane swap that reads it, and an MFMA and a
+// reader of its result are put in by the compiler, and only around instructions that it knows.
 __device__ __forceinline__ uint32_t mul2h(float a, float b, float c, float d) {
-  uint32_t r;
-  asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(r) : "v"(a), "v"(b));
-  asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(r) : "v"(c), "v"(d));
-  return r;
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, f16x2{static_cast<_Float16>(fmaf(a, b, 0.f)), static_cast<_Float16>(fmaf(c, d, 0.f))});
 }
 
 // 2^x on the hardware exp (v_exp_f32); arguments here are <= 0 and results
@@ -158,16 +159,7 @@ __device__ __forceinline__ uint4 codes32(const uint8_t* p) {
     return uint4{nib_from1(v), nib_from1(v >> 8), nib_from1(v >> 16), nib_from1(v >> 24)};
   }
 }
-__device__ __forceinline__ float vmax(float a, float b) {
-  float r;
-  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
-}
-__device__ __forceinline__ float vmax3(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
+__device__ __forceinline__ float vmax3(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }  // v_max3_f32
 
 // Online-softmax offset headroom, log2 units.  When a block's score exceeds
 // the running offset m, m moves to that score plus the headroom, so the
@@ -186,9 +178,9 @@ constexpr float kHeadroom = LKV_SOFTMAX_HEADROOM;
 // hold the other tokens of the same head), result in all four.
 __device__ __forceinline__ float xgroup_max(float v) {
   const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = vmax(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
   const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return vmax(__uint_as_float(b[0]), __uint_as_float(b[1]));
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 __device__ __forceinline__ float xgroup_sum(float v) {
   const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);

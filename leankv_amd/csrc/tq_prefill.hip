@@ -264,12 +264,12 @@ __device__ __forceinline__ float max32(const float (&s)[32]) {
     a = vmax3(a, s[j], s[j + 1]);
     b = vmax3(b, s[j + 2], s[j + 3]);
   }
-  return vmax(vmax3(a, s[30], s[31]), b);
+  return fmaxf(vmax3(a, s[30], s[31]), b);
 }
 // Max / sum over the two lanes l, l ^ 32 that share a column.
 __device__ __forceinline__ float xhalf_max(float v) {
   const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return vmax(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
 }
 __device__ __forceinline__ float xhalf_sum(float v) {
   const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
