@@ -534,11 +534,15 @@ def tq_cache_append(k_new, v_new, k_hot, v_hot, k_codes, k_norms, v_codes, v_nor
     )
 
 
-def _row_strided(t: torch.Tensor) -> torch.Tensor:
-    """t itself where its last-dim rows are dense, 16-byte aligned and a multiple of 16 bytes apart, else a copy."""
-    if t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % 8 == 0 for s in t.stride()[:-1]):
-        return t
-    return t.contiguous()
+def _row_strided(t: torch.Tensor):
+    """(t, strides) of [B, H, S, 128] rows: t itself where its rows are dense, 16-byte aligned and a multiple of 16
+    bytes apart, else a copy (contiguous() is none: a view of any offset and free strides of single sizes are
+    contiguous).  Strides of B, H and S in elements, 0 where the size is 1."""
+    strides = [0 if n == 1 else s for n, s in zip(t.shape[:3], t.stride())]
+    if t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % 8 == 0 for s in strides):
+        return t, strides
+    t = t.clone(memory_format=torch.contiguous_format)
+    return t, t.stride()[:3]
 
 
 def tq_cache_bulk_update(k_new, v_new, p0: int, k_hot, v_hot, k_codes, k_norms, v_codes, v_norms, PiK, PiV, bounds,
@@ -559,12 +563,12 @@ def tq_cache_bulk_update(k_new, v_new, p0: int, k_hot, v_hot, k_codes, k_norms, 
         if t.dtype != dt or not t.is_contiguous() or t.numel() != B * H * n:
             raise LeanKVError("tq_cache_bulk_update: %s must be contiguous %s of %d rows" % (nm, dt, B * H))
     dev = k_new.device
-    k_new, v_new = _row_strided(k_new), _row_strided(v_new)
+    (k_new, k_strides), (v_new, v_strides) = _row_strided(k_new), _row_strided(v_new)
     PiK, PiV = _pi(PiK, dev), _pi(PiV, dev)
     bounds = _vec(bounds, dev, (1 << bits) - 1, "decision boundaries")
     check(
-        _lib_handle().lkv_tq_cache_bulk_update(ptr(k_new), _I64x3(*k_new.stride()[:3]), ptr(v_new),
-                                               _I64x3(*v_new.stride()[:3]), B, H, S, int(p0), ptr(k_hot), ptr(v_hot),
+        _lib_handle().lkv_tq_cache_bulk_update(ptr(k_new), _I64x3(*k_strides), ptr(v_new),
+                                               _I64x3(*v_strides), B, H, S, int(p0), ptr(k_hot), ptr(v_hot),
                                                ptr(k_codes), ptr(k_norms), ptr(v_codes), ptr(v_norms), ptr(PiK),
                                                ptr(PiV), ptr(bounds), int(bits), hot_cap, cap, stream_handle(dev)),
         "lkv_tq_cache_bulk_update",

@@ -72,3 +72,32 @@ def test_bulk_update_refuses_bad_calls():
         call(S=20)  # 18 cold tokens do not fit 8 rows
     with pytest.raises(LeanKVError):
         call(dtype=torch.float32)
+
+
+def _layouts(x):
+    """[B, H, S, 128] tensors equal to x that lie in memory as callers may hand them over."""
+    B, H, S, D = x.shape
+    off = torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)[1:].view(x.shape)
+    wide = torch.empty(B, H, S, 2 * D, dtype=x.dtype, device=x.device)[..., ::2]
+    odd = torch.empty(B, H, S, D + 1, dtype=x.dtype, device=x.device)[..., :D]
+    rows = torch.empty(S, H, B, D, dtype=x.dtype, device=x.device).permute(2, 1, 0, 3)
+    last = torch.empty(H, S, D, B, dtype=x.dtype, device=x.device).permute(3, 0, 1, 2)  # B = 1: strides (1, ..)
+    for nm, t in (("offset", off), ("strided", wide), ("odd rows", odd), ("seq first", rows), ("batch last", last)):
+        yield nm, t.copy_(x)
+
+
+@pytest.mark.parametrize("B,H,S", [(1, 3, 70), (2, 1, 5), (1, 1, 66), (2, 3, 130)])
+def test_update_takes_any_layout(B, H, S):
+    """Rows at any offset, of any strides, with free strides of single sizes."""
+    from leankv_amd.turboquant.cache import TurboQuantCache
+
+    def run(k, v):
+        c = TurboQuantCache(num_layers=1, hot_buffer_size=64, device="cuda", max_seq_len=256)
+        return c.update(k, v, 0)
+
+    g = torch.Generator(device="cuda").manual_seed(S)
+    k, v = (torch.randn(B, H, S, 128, generator=g, device="cuda").half() for _ in range(2))
+    want = run(k, v)
+    for (nm, kk), (_, vv) in zip(_layouts(k), _layouts(v)):
+        got = run(kk, vv)
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), nm
