@@ -534,6 +534,21 @@ def tq_cache_append(k_new, v_new, k_hot, v_hot, k_codes, k_norms, v_codes, v_nor
     )
 
 
+def _check_layer(what: str, dev, B: int, H: int, bits: int, k_codes, k_norms, v_codes, v_norms, k_hot, v_hot):
+    """(hot_cap, cap) of one layer's static ring layout of B x H rows, every part of its shape and on dev."""
+    if k_hot.dim() != 4 or k_codes.dim() != 4:
+        raise LeanKVError("%s: hot rings must be [B, H, hot_cap, %d], codes [B, H, cap, row bytes]" % (what, HEAD_DIM))
+    hot_cap, cap = k_hot.shape[2], k_codes.shape[2]
+    hot, codes, norms = (B, H, hot_cap, HEAD_DIM), (B, H, cap, packed_row_bytes(bits)), (B, H, cap)
+    for t, nm, dt, shape in ((k_hot, "k_hot", torch.float16, hot), (v_hot, "v_hot", torch.float16, hot),
+                             (k_codes, "k_codes", torch.uint8, codes), (v_codes, "v_codes", torch.uint8, codes),
+                             (k_norms, "k_norms", torch.float32, norms), (v_norms, "v_norms", torch.float32, norms)):
+        if t.dtype != dt or t.shape != shape or t.device != dev or not t.is_contiguous():
+            raise LeanKVError("%s: %s must be contiguous %s %s on %s, got %s %s on %s"
+                              % (what, nm, dt, shape, dev, t.dtype, tuple(t.shape), t.device))
+    return hot_cap, cap
+
+
 def _row_strided(t: torch.Tensor):
     """(t, strides) of [B, H, S, 128] rows: t itself where its rows are dense, 16-byte aligned and a multiple of 16
     bytes apart, else a copy (contiguous() is none: a view of any offset and free strides of single sizes are
@@ -550,18 +565,14 @@ def tq_cache_bulk_update(k_new, v_new, p0: int, k_hot, v_hot, k_codes, k_norms, 
     """S new tokens k_new, v_new fp16 [B, H, S, 128] (any row strides) appended at position p0 to one layer's static
     ring layout, keys and values in one launch (lkv_tq_cache_bulk_update): the tokens leaving the window are
     quantized into the cold rows, the newest take their ring slots."""
-    require_cuda(k_new, v_new, k_hot, v_hot, k_codes, v_codes)
+    require_cuda(k_new, v_new)
     if k_new.dim() != 4 or k_new.shape[-1] != HEAD_DIM or v_new.shape != k_new.shape:
         raise LeanKVError("tq_cache_bulk_update: k_new and v_new must be alike, [B, H, S, %d]" % HEAD_DIM)
-    if k_new.dtype != torch.float16 or v_new.dtype != torch.float16:
-        raise LeanKVError("tq_cache_bulk_update: k_new and v_new must be float16")
+    if k_new.dtype != torch.float16 or v_new.dtype != torch.float16 or v_new.device != k_new.device:
+        raise LeanKVError("tq_cache_bulk_update: k_new and v_new must be float16 on one device")
     B, H, S, _ = k_new.shape
-    hot_cap, cap, rb = k_hot.shape[-2], k_codes.shape[-2], packed_row_bytes(bits)
-    for t, nm, dt, n in ((k_hot, "k_hot", torch.float16, hot_cap * HEAD_DIM), (k_codes, "k_codes", torch.uint8, cap * rb),
-                         (k_norms, "k_norms", torch.float32, cap), (v_hot, "v_hot", torch.float16, hot_cap * HEAD_DIM),
-                         (v_codes, "v_codes", torch.uint8, cap * rb), (v_norms, "v_norms", torch.float32, cap)):
-        if t.dtype != dt or not t.is_contiguous() or t.numel() != B * H * n:
-            raise LeanKVError("tq_cache_bulk_update: %s must be contiguous %s of %d rows" % (nm, dt, B * H))
+    hot_cap, cap = _check_layer("tq_cache_bulk_update", k_new.device, B, H, bits, k_codes, k_norms, v_codes, v_norms,
+                                k_hot, v_hot)
     dev = k_new.device
     (k_new, k_strides), (v_new, v_strides) = _row_strided(k_new), _row_strided(v_new)
     PiK, PiV = _pi(PiK, dev), _pi(PiV, dev)
@@ -578,16 +589,12 @@ def tq_cache_bulk_update(k_new, v_new, p0: int, k_hot, v_hot, k_codes, k_norms, 
 def tq_cache_read(k_codes, k_norms, v_codes, v_norms, k_hot, v_hot, PiK, PiV, centroids, bits: int, n: int):
     """(K, V) fp16 [B, H, n, 128] of one layer's static ring layout in position order, one launch
     (lkv_tq_cache_read): cold tokens dequantized, the newest min(n, hot) from their ring slots."""
-    require_cuda(k_codes, v_codes, k_hot, v_hot)
-    B, H, cap, rb = k_codes.shape
-    hot_cap = k_hot.shape[-2]
-    _check_code_rows(k_codes, v_codes, bits, "tq_cache_read")
-    for t, nm, dt, m in ((k_codes, "k_codes", torch.uint8, cap * rb), (v_codes, "v_codes", torch.uint8, cap * rb),
-                         (k_norms, "k_norms", torch.float32, cap), (v_norms, "v_norms", torch.float32, cap),
-                         (k_hot, "k_hot", torch.float16, hot_cap * HEAD_DIM),
-                         (v_hot, "v_hot", torch.float16, hot_cap * HEAD_DIM)):
-        if t.dtype != dt or not t.is_contiguous() or t.numel() != B * H * m:
-            raise LeanKVError("tq_cache_read: %s must be contiguous %s of %d rows" % (nm, dt, B * H))
+    require_cuda(k_codes)
+    if k_codes.dim() != 4:
+        raise LeanKVError("tq_cache_read: k_codes must be [B, H, cap, row bytes], got %s" % (tuple(k_codes.shape),))
+    B, H = k_codes.shape[:2]
+    hot_cap, cap = _check_layer("tq_cache_read", k_codes.device, B, H, bits, k_codes, k_norms, v_codes, v_norms, k_hot,
+                                v_hot)
     dev = k_codes.device
     PiK, PiV = _pi(PiK, dev), _pi(PiV, dev)
     centroids = _vec(centroids, dev, 1 << bits, "centroids")

@@ -101,3 +101,17 @@ def test_update_takes_any_layout(B, H, S):
     for (nm, kk), (_, vv) in zip(_layouts(k), _layouts(v)):
         got = run(kk, vv)
         assert all(torch.equal(a, b) for a, b in zip(got, want)), nm
+
+
+def test_update_of_another_batch_is_refused():
+    """As many rows of another batch and head count: refused, the cache as it was."""
+    from leankv_amd._lib import LeanKVError
+    from leankv_amd.turboquant.cache import TurboQuantCache
+
+    c = TurboQuantCache(num_layers=1, hot_buffer_size=16, device="cuda", max_seq_len=64)
+    x = torch.randn(2, 4, 20, 128, device="cuda").half()
+    want = c.update(x, x, 0)
+    y = torch.randn(4, 2, 5, 128, device="cuda").half()
+    with pytest.raises(LeanKVError):
+        c.update(y, y, 0)
+    assert c.get_seq_length(0) == 20 and all(torch.equal(a, b) for a, b in zip(c[0], want))
