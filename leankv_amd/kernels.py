@@ -921,7 +921,8 @@ _LIB_DEF = None
 # Schemas of torch.ops.leankv.*: the reference's kernel contracts (sparse_gemv.py:143-181,
 # quantizer.py:119-137, rotation.py:45-52, cache.py:84-189 + sdpa_attention.py:79-105) as
 # dispatcher ops.  Every functional op has an ``.out`` overload that writes caller-owned buffers,
-# so a captured HIP graph holds no allocation; ``tq_cache_append`` mutates the cache in place.
+# so a captured HIP graph holds no allocation; ``tq_cache_append`` and ``tq_cache_bulk_update``
+# mutate the cache in place, and ``tq_cache_read`` returns new tensors of the length asked for.
 _SCHEMAS = (
     "sparse_gemv(Tensor x, Tensor weight, float threshold) -> Tensor",
     "sparse_gemv.out(Tensor x, Tensor weight, float threshold, *, Tensor(a!) out) -> Tensor(a!)",
@@ -940,6 +941,10 @@ _SCHEMAS = (
     "tq_cache_append(Tensor k_new, Tensor v_new, Tensor(a!) k_hot, Tensor(b!) v_hot, Tensor(c!) k_codes, "
     "Tensor(d!) k_norms, Tensor(e!) v_codes, Tensor(f!) v_norms, Tensor PiK, Tensor PiV, Tensor bounds, int bits, "
     "Tensor pos) -> ()",
+    "tq_cache_bulk_update(Tensor k_new, Tensor v_new, int p0, Tensor(a!) k_hot, Tensor(b!) v_hot, Tensor(c!) k_codes, "
+    "Tensor(d!) k_norms, Tensor(e!) v_codes, Tensor(f!) v_norms, Tensor PiK, Tensor PiV, Tensor bounds, int bits) -> ()",
+    "tq_cache_read(Tensor k_codes, Tensor k_norms, Tensor v_codes, Tensor v_norms, Tensor k_hot, Tensor v_hot, "
+    "Tensor PiK, Tensor PiV, Tensor centroids, int bits, int n) -> (Tensor, Tensor)",
     "tq_decode_attn(Tensor q, Tensor k_codes, Tensor k_norms, Tensor v_codes, Tensor v_norms, Tensor k_hot, "
     "Tensor v_hot, Tensor PiK, Tensor PiV, Tensor centroids, int bits, Tensor seq_len, int max_len, float scale) "
     "-> Tensor",
@@ -988,6 +993,10 @@ def _impls():
     def m_append(*args):
         return None
 
+    def m_read(kc, kn, vc, vn, kh, vh, PiK, PiV, c, bits, n):
+        k = kh.new_empty(*kh.shape[:2], n, kh.shape[-1])
+        return k, torch.empty_like(k)
+
     def m_attn(q, *args, out=None):
         return out if out is not None else torch.empty_like(q)
 
@@ -1008,6 +1017,8 @@ def _impls():
         "tq_rotate": (lambda x, Pi, tr: tq_rotate(x, Pi, tr), m_rotate),
         "rms_norm": (lambda x, w, eps: rms_norm(x, w, eps), m_rms),
         "tq_cache_append": (lambda *a: tq_cache_append(*a), m_append),
+        "tq_cache_bulk_update": (lambda *a: tq_cache_bulk_update(*a), m_append),
+        "tq_cache_read": (lambda *a: tq_cache_read(*a), m_read),
         "tq_decode_attn": (lambda *a: tq_decode_attn(*a), m_attn),
         "tq_decode_attn.out": (lambda *a, out: tq_decode_attn_out(*a, out), m_attn),
         "tq_prefill_attn": (lambda *a: tq_prefill_attn(*a), m_attn),

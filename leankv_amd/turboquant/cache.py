@@ -188,16 +188,16 @@ class TurboQuantCache:
 
     def _bulk_update(self, li: int, k16: torch.Tensor, v16: torch.Tensor, p0: int) -> None:
         """Append S > 1 tokens: quantize every token that leaves the hot window, refill the ring (one launch)."""
-        _k.tq_cache_bulk_update(k16, v16, p0, self._k_hot[li], self._v_hot[li], self._k_codes[li], self._k_norms[li],
-                                self._v_codes[li], self._v_norms[li], self.PiK[li], self.PiV[li],
-                                self.decision_boundaries, self.bits)
+        torch.ops.leankv.tq_cache_bulk_update(
+            k16, v16, p0, self._k_hot[li], self._v_hot[li], self._k_codes[li], self._k_norms[li], self._v_codes[li],
+            self._v_norms[li], self.PiK[li], self.PiV[li], self.decision_boundaries, self.bits)
 
     def _get_full_cache(self, layer_idx: int):
         """cat(dequantize(cold).fp16, hot) in position order (cache.py:169-189)."""
         li = layer_idx
-        k, v = _k.tq_cache_read(self._k_codes[li], self._k_norms[li], self._v_codes[li], self._v_norms[li],
-                                self._k_hot[li], self._v_hot[li], self.PiK[li], self.PiV[li], self.centroids,
-                                self.bits, self._seq_lengths[li])
+        k, v = torch.ops.leankv.tq_cache_read(
+            self._k_codes[li], self._k_norms[li], self._v_codes[li], self._v_norms[li], self._k_hot[li],
+            self._v_hot[li], self.PiK[li], self.PiV[li], self.centroids, self.bits, self._seq_lengths[li])
         return k.to(self._dtype), v.to(self._dtype)
 
     # ----------------------------------------------------------- fused decode attention

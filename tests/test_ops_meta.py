@@ -39,6 +39,9 @@ def _calls():
         "rms_norm": (lambda: o.rms_norm(_e(3, 4096), _e(4096), 1e-5), [((3, 4096), F16)]),
         "tq_cache_append": (lambda: o.tq_cache_append(_e(8, 128), _e(8, 128), hot, hot, kc, kn, kc, kn, Pi, Pi, b, 3,
                                                       seq), []),
+        "tq_cache_bulk_update": (lambda: o.tq_cache_bulk_update(_e(1, 8, 5, 128), _e(1, 8, 5, 128), 3, hot, hot, kc, kn,
+                                                                kc, kn, Pi, Pi, b, 3), []),
+        "tq_cache_read": (lambda: o.tq_cache_read(*attn, 150), [((1, 8, 150, 128), F16)] * 2),
         "tq_decode_attn": (lambda: o.tq_decode_attn(q1, *attn, seq, 164, 0.1), [((1, 32, 128), F16)]),
         "tq_decode_attn.out": (lambda: o.tq_decode_attn.out(q1, *attn, seq, 164, 0.1, out=_e(1, 32, 128)),
                                [((1, 32, 128), F16)]),
@@ -62,3 +65,14 @@ def test_out_overloads_return_the_given_buffer():
     o = torch.ops.leankv
     out = _e(1024)
     assert o.sparse_gemv.out(_e(4096), _e(1024, 4096), 0.1, out=out) is out
+
+
+def test_the_cache_runs_on_meta_tensors():
+    """The cache's kernels all go through the dispatcher: shapes without data, window and cold store, both ways."""
+    from leankv_amd.turboquant.cache import TurboQuantCache
+
+    c = TurboQuantCache(num_layers=1, hot_buffer_size=16, device="meta", max_seq_len=8)
+    for S, n in ((10, 10), (30, 40), (1, 41)):
+        k, v = c.update(_e(2, 4, S, 128), _e(2, 4, S, 128), 0)
+        assert k.shape == v.shape == (2, 4, n, 128) and k.dtype == v.dtype == F16 and k.is_meta
+    assert c[0][0].shape == (2, 4, 41, 128)
