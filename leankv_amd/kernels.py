@@ -360,7 +360,7 @@ def _pi(Pi: torch.Tensor, device) -> torch.Tensor:
     torch.linalg.qr returns Q column-major, so a rotation built from it must be
     made contiguous before its pointer reaches a kernel.
     """
-    if tuple(Pi.shape) != (HEAD_DIM, HEAD_DIM):
+    if Pi.shape != (HEAD_DIM, HEAD_DIM):
         raise LeanKVError("TurboQuant: rotation must be [128, 128], got %s" % (tuple(Pi.shape),))
     if Pi.dtype == torch.float32 and Pi.device == device and Pi.is_contiguous():
         return Pi

@@ -34,6 +34,7 @@ import math
 import weakref
 
 import torch
+from torch.autograd import forward_ad
 
 from .. import kernels as _k  # also registers torch.ops.leankv (the cache's kernels go through the dispatcher)
 from .codebook import get_codebook_tensors
@@ -105,7 +106,8 @@ class TurboQuantCache:
         for n in sizes:
             at.append(at[-1] + -(-n // 256) * 256)
         buf = torch.zeros(at[-1], dtype=torch.uint8, device=self._device)
-        return [buf[o:o + n].view(dtype).view(shape) for o, n, (shape, dtype) in zip(at, sizes, specs)]
+        # detached: autograd may follow one part and not the others
+        return [buf[o:o + n].view(dtype).view(shape).detach() for o, n, (shape, dtype) in zip(at, sizes, specs)]
 
     def _alloc(self, layer: int, B: int, H: int, cap: int) -> None:
         rows = (B, H, cap)
@@ -186,18 +188,57 @@ class TurboQuantCache:
             return key_states, value_states
         return self._get_full_cache(layer_idx)
 
+    def _torch_window(self, *tensors) -> bool:
+        """Whether the window moves through torch operations: where autograd follows a tensor (in backward or forward
+        mode), since the kernels pass by it, and on the host, where a prompt inside the window needs no kernel."""
+        if self._device.type == "cpu":
+            return True
+        if torch.is_grad_enabled():
+            for t in tensors:
+                if t.requires_grad:
+                    return True
+        # (unpack_dual, called for each tensor at any time, costs a read-back 2 us)
+        return getattr(forward_ad, "_current_level", 0) >= 0 and any(
+            forward_ad.unpack_dual(t).tangent is not None for t in tensors)
+
     def _bulk_update(self, li: int, k16: torch.Tensor, v16: torch.Tensor, p0: int) -> None:
         """Append S > 1 tokens: quantize every token that leaves the hot window, refill the ring (one launch)."""
-        torch.ops.leankv.tq_cache_bulk_update(
-            k16, v16, p0, self._k_hot[li], self._v_hot[li], self._k_codes[li], self._k_norms[li], self._v_codes[li],
-            self._v_norms[li], self.PiK[li], self.PiV[li], self.decision_boundaries, self.bits)
+        kh, vh = self._k_hot[li], self._v_hot[li]
+        if not self._torch_window(k16, v16, kh, vh):
+            torch.ops.leankv.tq_cache_bulk_update.default(
+                k16, v16, p0, kh, vh, self._k_codes[li], self._k_norms[li], self._v_codes[li], self._v_norms[li],
+                self.PiK[li], self.PiV[li], self.decision_boundaries, self.bits)
+            return
+        hot, T = self.hot_buffer_size, p0 + k16.shape[2]
+        c0, c1 = self._cold_len(p0), self._cold_len(T)
+        first = max(p0, T - hot)  # the newest min(S, hot) tokens enter the ring, each in slot p % hot
+        leave = torch.arange(c0, max(c0, min(c1, p0)), device=self._device) % hot  # ring tokens that leave the window
+        enter = torch.arange(first, T, device=self._device) % hot
+        for new, ring, codes, norms, pi in ((k16, kh, self._k_codes[li], self._k_norms[li], self.PiK[li]),
+                                            (v16, vh, self._v_codes[li], self._v_norms[li], self.PiV[li])):
+            if c1 > c0:
+                cold = torch.cat([ring.index_select(2, leave), new[:, :, : max(0, c1 - p0)]], dim=2).detach()
+                codes[:, :, c0:c1], norms[:, :, c0:c1] = torch.ops.leankv.tq_quantize(
+                    cold.float().contiguous(), pi, self.decision_boundaries, self.bits)
+            ring.index_copy_(2, enter, new[:, :, first - p0:])
 
     def _get_full_cache(self, layer_idx: int):
         """cat(dequantize(cold).fp16, hot) in position order (cache.py:169-189)."""
-        li = layer_idx
-        k, v = torch.ops.leankv.tq_cache_read(
-            self._k_codes[li], self._k_norms[li], self._v_codes[li], self._v_norms[li], self._k_hot[li],
-            self._v_hot[li], self.PiK[li], self.PiV[li], self.centroids, self.bits, self._seq_lengths[li])
+        li, n = layer_idx, self._seq_lengths[layer_idx]
+        kh, vh = self._k_hot[li], self._v_hot[li]
+        if not self._torch_window(kh, vh):
+            k, v = torch.ops.leankv.tq_cache_read.default(
+                self._k_codes[li], self._k_norms[li], self._v_codes[li], self._v_norms[li], kh, vh, self.PiK[li],
+                self.PiV[li], self.centroids, self.bits, n)
+            return (k, v) if self._dtype == torch.float16 else (k.to(self._dtype), v.to(self._dtype))
+        c = self._cold_len(n)
+        slots = torch.arange(c, n, device=self._device) % self.hot_buffer_size  # in position order
+        k, v = kh.index_select(2, slots), vh.index_select(2, slots)
+        if c:
+            ck, cv = torch.ops.leankv.tq_cache_read(
+                self._k_codes[li], self._k_norms[li], self._v_codes[li], self._v_norms[li], kh.detach(), vh.detach(),
+                self.PiK[li], self.PiV[li], self.centroids, self.bits, n)
+            k, v = torch.cat([ck[:, :, :c], k], dim=2), torch.cat([cv[:, :, :c], v], dim=2)
         return k.to(self._dtype), v.to(self._dtype)
 
     # ----------------------------------------------------------- fused decode attention
