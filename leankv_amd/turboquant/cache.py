@@ -40,6 +40,8 @@ from .. import kernels as _k  # also registers torch.ops.leankv (the cache's ker
 from .codebook import get_codebook_tensors
 from .rotation import generate_rotation_matrices
 
+_SHARED_BYTES = 32 << 20  # parts of a layer's store in one buffer (TurboQuantCache._zeros)
+
 _ACTIVE = None  # weakref to the cache whose update() ran last (read by the attention function)
 
 
@@ -99,9 +101,14 @@ class TurboQuantCache:
 
     # ----------------------------------------------------------- storage
     def _zeros(self, *specs) -> list:
-        """Zeroed tensors of (shape, dtype) as 256-byte-aligned parts of one buffer, cleared by one launch (a queued
-        launch costs ~4.5 us however small).  Tensors replaced together when the store grows share a buffer."""
+        """Zeroed tensors of (shape, dtype).  Up to _SHARED_BYTES in all they are 256-byte-aligned parts of one buffer,
+        cleared by one launch: a launch costs about 5 us however small, and clearing more than that takes longer.
+        Larger ones are buffers of their own: when the store grows, codes and norms are replaced one after the other
+        and each old buffer is free before the next is allocated (a shared one lives until the last is replaced, a
+        sixth more at the peak)."""
         sizes = [math.prod(shape) * dtype.itemsize for shape, dtype in specs]
+        if sum(sizes) > _SHARED_BYTES:
+            return [torch.zeros(shape, dtype=dtype, device=self._device) for shape, dtype in specs]
         at = [0]
         for n in sizes:
             at.append(at[-1] + -(-n // 256) * 256)
