@@ -27,6 +27,7 @@ import contextlib
 import ctypes
 import gc
 import math
+import threading
 
 import torch
 import torch.nn.functional as F
@@ -37,19 +38,29 @@ from .turboquant.cache import TurboQuantCache
 STEP_BITS = (1, 2, 3, 4)  # code widths the fused B = 1 decode step (lkv_decode_*) is built for
 
 
+_capture_lock = threading.Lock()
+_captures = [0, False]  # captures running, and whether the collector was on before the first of them
+
+
 @contextlib.contextmanager
 def _capture(graph, stream):
     """torch.cuda.graph without cyclic garbage collection meanwhile: an older engine's graph that only the collector
     can free (a model, its fast-path forward and its engine refer to each other) synchronizes the device when it is
-    destroyed, which fails during a capture and, in a destructor, ends the process."""
-    on = gc.isenabled()
-    gc.disable()
+    destroyed, which fails during a capture and, in a destructor, ends the process.  The collector stays off until
+    the last of several threads' captures has ended."""
+    with _capture_lock:
+        if _captures[0] == 0:
+            _captures[1] = gc.isenabled()
+            gc.disable()
+        _captures[0] += 1
     try:
         with torch.cuda.graph(graph, stream=stream):
             yield
     finally:
-        if on:
-            gc.enable()
+        with _capture_lock:
+            _captures[0] -= 1
+            if _captures[0] == 0 and _captures[1]:
+                gc.enable()
 
 
 def _rms(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:

@@ -37,3 +37,34 @@ def test_no_collection_during_a_capture(monkeypatch, on):
     finally:
         gc.set_threshold(*old[0])
         (gc.enable if old[1] else gc.disable)()
+
+
+def test_no_collection_while_another_thread_captures(monkeypatch):
+    """The first capture to end leaves the collector off for the one still running."""
+    import threading
+
+    from leankv_amd.engine import _capture
+
+    monkeypatch.setattr(torch.cuda, "graph", lambda graph, stream=None: contextlib.nullcontext())
+    first_in, second_in, first_out = threading.Event(), threading.Event(), threading.Event()
+
+    def first():
+        with _capture(None, None):
+            first_in.set()
+            second_in.wait(10)
+        first_out.set()
+
+    was = gc.isenabled()
+    try:
+        gc.enable()
+        t = threading.Thread(target=first)
+        t.start()
+        assert first_in.wait(10)
+        with _capture(None, None):
+            second_in.set()
+            assert first_out.wait(10)
+            assert not gc.isenabled()
+        assert gc.isenabled()
+        t.join(10)
+    finally:
+        (gc.enable if was else gc.disable)()
