@@ -340,12 +340,16 @@ def sparse_qkv(x: torch.Tensor, wq: torch.Tensor, wk: torch.Tensor, wv: torch.Te
 
 
 # ----------------------------------------------------------------- TurboQuant
-@functools.lru_cache(maxsize=None)
-def packed_row_bytes(bits: int) -> int:
-    n = _lib_handle().lkv_tq_packed_row_bytes(int(bits))
+@functools.lru_cache(maxsize=8)
+def _row_bytes(bits: int) -> int:
+    n = _lib_handle().lkv_tq_packed_row_bytes(bits)
     if n < 0:
         raise LeanKVError("TurboQuant: bits=%d cannot be bit-packed (1..4 supported)" % bits)
     return n
+
+
+def packed_row_bytes(bits: int) -> int:
+    return _row_bytes(int(bits))  # by value: a tensor or array is no key
 
 
 def _rows(x: torch.Tensor, what: str) -> int:
