@@ -291,11 +291,13 @@ __global__ __launch_bounds__(kThreads, 2) void bulk_update_kernel(BulkArgs P) {
     }
     const float nrm = normalize_row<false>(a);
     if (slot_p) {  // the old token is in registers (the norm has used it)
-      uint4 nw[4];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) nw[v] = reinterpret_cast<const uint4*>(refill)[v];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) reinterpret_cast<uint4*>(slot_p)[v] = nw[v];
+      const uint4* const src = reinterpret_cast<const uint4*>(refill);
+      uint4* const dst = reinterpret_cast<uint4*>(slot_p);
+      const uint4 n0 = src[0], n1 = src[1], n2 = src[2], n3 = src[3];  // (an array here ends in scratch memory)
+      dst[0] = n0;
+      dst[1] = n1;
+      dst[2] = n2;
+      dst[3] = n3;
     }
     if (g == 0 && r < M) norms[cold_row(r)] = nrm;
     f32x4 acc[8];
