@@ -269,7 +269,7 @@ int rotate_rows(const void* x, bool x_f16, int64_t M, const float* Pi, int trans
 
 struct AttnPlan {
   int nsplit, split_tokens;
-  size_t qrot_off, part_off, total;
+  size_t part_off, total;
 };
 // max_split_tokens > 0 caps the tokens of one split (the paged layout stages a
 // split's page ids in LDS); the split count then grows past the target.
@@ -296,7 +296,7 @@ struct AttnCall {
   // Decode step (B = 1), set when pq is non-null: the query, key and value
   // of the new token arrive as q|k|v GEMV partials ([slab][chunk][kGemvBN]).
   // The split kernel sums them, applies RoPE at position *pos, rotates the
-  // query with PiK (q_rot and q are then unused as inputs); its last split
+  // query with PiK (q is then unused as an input); its last split
   // block writes the RoPE'd query to q16 (read by the combine as q) and the
   // new key / value into ring slot *pos % hot_cap.
   const float* pq;

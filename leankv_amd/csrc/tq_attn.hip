@@ -914,8 +914,7 @@ AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t max_len, int64_t 
   p.nsplit = static_cast<int>(ns);
   p.split_tokens = static_cast<int>(ts);
   auto al = [](size_t v) { return (v + 255) / 256 * 256; };
-  p.qrot_off = kTicketBytes;  // room for a rotated query, no longer used: the workspace's layout and size stay
-  p.part_off = p.qrot_off + al(static_cast<size_t>(B * Hq * kD) * 4);
+  p.part_off = kTicketBytes;
   // sized for ns_cap so a workspace sized without hot_cap fits every call
   p.total = p.part_off + al(static_cast<size_t>(B * Hkv * ns_cap) * rec_floats(static_cast<int>(G)) * 4);
   return p;

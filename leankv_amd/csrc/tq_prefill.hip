@@ -92,60 +92,44 @@ struct PrefillParams {
   int S, Hq, Hkv, G, cap, hot_cap, kv_len, cold_len, ncent;
 };
 
-// y = scale * (x @ Pi^T) (TRANS false) or scale * (x @ Pi) (TRANS true) for M
-// rows of 128, on fp16 MFMA: Pi split exactly into hi + lo / 2048 fp16 parts,
-// and x too when it is fp32, fp32 accumulate (error ~2^-22 relative, the
-// x_lo * Pi_lo term dropped).  Wave w computes output dims 32 w .. 32 w + 31
-// with its Pi operands in registers; a block takes 64-row tiles, staged
-// through LDS both ways so every row is read once and written with 16-byte
-// stores.
-// Up to 3 independent row sets (segments) per launch, blockIdx.y picking one:
-// the query and the two hot rings are rotated by a single launch.
+// y = x @ Pi^T for fp16 rows of 128, on fp16 MFMA: Pi split into fp16 parts hi +
+// lo / 2048 (22 bits and more of the 24), fp32 accumulate.  Wave w computes output
+// dims 32 w .. 32 w + 31 with its Pi operands in registers; a block takes 64-row
+// tiles, staged through LDS both ways so every row is read once and written
+// with 16-byte stores.  The two hot rings are rotated by one launch, blockIdx.y
+// picking the ring.
 constexpr int kRotRows = 64;
-constexpr int kMaxRotSegs = 3;
 struct RotSeg {
-  const void* x;
+  const uint16_t* x;
   const float* Pi;
-  void* y;
-  int64_t M;
-  float scale;
+  uint16_t* y;
 };
 struct RotSegs {
-  RotSeg s[kMaxRotSegs];
+  RotSeg s[2];
+  int64_t M;  // rows of each
 };
-template <bool IN_F16, bool OUT_F16, bool TRANS>
 __global__ __launch_bounds__(kThreads) void rotate16_kernel(RotSegs segs) {
   const RotSeg& sg = segs.s[blockIdx.y];
-  const void* __restrict__ x = sg.x;
+  const uint16_t* __restrict__ x = sg.x;
   const float* __restrict__ Pi = sg.Pi;
-  void* __restrict__ y = sg.y;
-  const int64_t M = sg.M;
-  const float scale = sg.scale;
-  if (static_cast<int64_t>(blockIdx.x) * kRotRows >= M) return;  // uniform: this segment has fewer tiles
-  constexpr int kInB = IN_F16 ? 2 : 4, kOutB = OUT_F16 ? 2 : 4;
-  constexpr int kInRow = kD * kInB + 16, kOutRow = kD * kOutB + 16;  // padded LDS rows (bytes)
-  __shared__ __align__(16) uint8_t s_in[kRotRows * kInRow];
-  __shared__ __align__(16) uint8_t s_out[kRotRows * kOutRow];
+  uint16_t* __restrict__ y = sg.y;
+  const int64_t M = segs.M;
+  constexpr int kRow = kD + 8;  // padded LDS row
+  __shared__ __align__(16) uint16_t s_in[kRotRows * kRow];
+  __shared__ __align__(16) uint16_t s_out[kRotRows * kRow];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c16 = lane & 15, g = lane >> 4;
-  // B operands: column d = 32 wave + 16 dt + c16, k = input dim e = 32 kb + 8 g + i
+  // B operands: column d = 32 wave + 16 dt + c16, k = input dim e = 32 kb + 8 g + i: B[e][d] = Pi[d][e]
   u32x4 bh[2][4], bl[2][4];
 #pragma unroll
   for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
       const int d = 32 * wave + 16 * dt + c16, e0 = 32 * kb + 8 * g;
-      float p[8];
-      if constexpr (!TRANS) {  // B[e][d] = Pi[d][e]
-        const float4 u0 = *reinterpret_cast<const float4*>(Pi + d * kD + e0);
-        const float4 u1 = *reinterpret_cast<const float4*>(Pi + d * kD + e0 + 4);
-        p[0] = u0.x; p[1] = u0.y; p[2] = u0.z; p[3] = u0.w;
-        p[4] = u1.x; p[5] = u1.y; p[6] = u1.z; p[7] = u1.w;
-      } else {  // B[e][d] = Pi[e][d]
-#pragma unroll
-        for (int i = 0; i < 8; ++i) p[i] = Pi[(e0 + i) * kD + d];
-      }
+      const float4 u0 = *reinterpret_cast<const float4*>(Pi + d * kD + e0);
+      const float4 u1 = *reinterpret_cast<const float4*>(Pi + d * kD + e0 + 4);
+      const float p[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const uint16_t h0 = f2h(p[2 * j]), h1 = f2h(p[2 * j + 1]);
@@ -153,101 +137,52 @@ __global__ __launch_bounds__(kThreads) void rotate16_kernel(RotSegs segs) {
         bl[dt][kb][j] = pack2h((p[2 * j] - h2f(h0)) * 2048.f, (p[2 * j + 1] - h2f(h1)) * 2048.f);
       }
     }
-  constexpr int kInChunks = kRotRows * kD * kInB / 16 / kThreads;    // 16-byte loads per thread
-  constexpr int kOutChunks = kRotRows * kD * kOutB / 16 / kThreads;  // 16-byte stores per thread
-  constexpr int kInPerRow = kD * kInB / 16, kOutPerRow = kD * kOutB / 16;
+  constexpr int kPerRow = kD / 8;                            // 16-byte chunks of a row
+  constexpr int kChunks = kRotRows * kPerRow / kThreads;     // per thread, in and out
   const int64_t ntiles = (M + kRotRows - 1) / kRotRows;
   for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     const int64_t row0 = tile * kRotRows;
     // ---- rows in (rows past M read row M - 1, never stored)
 #pragma unroll
-    for (int c = 0; c < kInChunks; ++c) {
-      const int f = c * kThreads + tid, r = f / kInPerRow, q = f % kInPerRow;
+    for (int c = 0; c < kChunks; ++c) {
+      const int f = c * kThreads + tid, r = f / kPerRow, q = f % kPerRow;
       const int64_t gr = min(row0 + r, M - 1);
-      const uint4 u = *reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(x) + gr * (kD * kInB) + 16 * q);
-      *reinterpret_cast<uint4*>(s_in + r * kInRow + 16 * q) = u;
+      *reinterpret_cast<uint4*>(s_in + r * kRow + 8 * q) = *reinterpret_cast<const uint4*>(x + gr * kD + 8 * q);
     }
     __syncthreads();
 #pragma unroll
     for (int rg = 0; rg < kRotRows / 16; ++rg) {
-      u32x4 ah[4], al[4];
-      const uint8_t* arow = s_in + (16 * rg + c16) * kInRow;
+      u32x4 a[4];
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        if constexpr (IN_F16) {
-          const uint4 u = *reinterpret_cast<const uint4*>(arow + 2 * (32 * kb + 8 * g));
-          ah[kb] = u32x4{u.x, u.y, u.z, u.w};
-        } else {
-          const float4 u0 = *reinterpret_cast<const float4*>(arow + 4 * (32 * kb + 8 * g));
-          const float4 u1 = *reinterpret_cast<const float4*>(arow + 4 * (32 * kb + 8 * g) + 16);
-          const float v[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const uint16_t h0 = f2h(v[2 * j]), h1 = f2h(v[2 * j + 1]);
-            ah[kb][j] = static_cast<uint32_t>(h0) | (static_cast<uint32_t>(h1) << 16);
-            al[kb][j] = pack2h((v[2 * j] - h2f(h0)) * 2048.f, (v[2 * j + 1] - h2f(h1)) * 2048.f);
-          }
-        }
-      }
+      for (int kb = 0; kb < 4; ++kb)
+        a[kb] = *reinterpret_cast<const u32x4*>(s_in + (16 * rg + c16) * kRow + 32 * kb + 8 * g);
 #pragma unroll
       for (int dt = 0; dt < 2; ++dt) {
         f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f}, accl = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb) {
-          acc = mfma16x16x32(ah[kb], bh[dt][kb], acc);
-          accl = mfma16x16x32(ah[kb], bl[dt][kb], accl);
-          if constexpr (!IN_F16) accl = mfma16x16x32(al[kb], bh[dt][kb], accl);
+          acc = mfma16x16x32(a[kb], bh[dt][kb], acc);
+          accl = mfma16x16x32(a[kb], bl[dt][kb], accl);
         }
         // D: column d = 32 wave + 16 dt + c16, rows 16 rg + 4 g + i
-        const int d = 32 * wave + 16 * dt + c16;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float v = (acc[i] + accl[i] * (1.f / 2048.f)) * scale;
-          uint8_t* dst = s_out + (16 * rg + 4 * g + i) * kOutRow + kOutB * d;
-          if constexpr (OUT_F16)
-            *reinterpret_cast<uint16_t*>(dst) = f2h(v);
-          else
-            *reinterpret_cast<float*>(dst) = v;
+          float v = acc[i] + accl[i] * (1.f / 2048.f);
+          __asm__ volatile("" : "+v"(v));  // rounded to fp32 before fp16, as a scaled product is
+          s_out[(16 * rg + 4 * g + i) * kRow + 32 * wave + 16 * dt + c16] = f2h(v);
         }
       }
     }
     __syncthreads();
     // ---- rows out
 #pragma unroll
-    for (int c = 0; c < kOutChunks; ++c) {
-      const int f = c * kThreads + tid, r = f / kOutPerRow, q = f % kOutPerRow;
+    for (int c = 0; c < kChunks; ++c) {
+      const int f = c * kThreads + tid, r = f / kPerRow, q = f % kPerRow;
       if (row0 + r < M)
-        *reinterpret_cast<uint4*>(static_cast<uint8_t*>(y) + (row0 + r) * (kD * kOutB) + 16 * q) =
-            *reinterpret_cast<const uint4*>(s_out + r * kOutRow + 16 * q);
+        *reinterpret_cast<uint4*>(y + (row0 + r) * kD + 8 * q) = *reinterpret_cast<const uint4*>(s_out + r * kRow + 8 * q);
     }
     __syncthreads();  // s_in and s_out are rewritten by the next tile
   }
-}
-
-// One launch over n segments (n <= kMaxRotSegs; empty segments are skipped).
-template <bool IN_F16, bool OUT_F16, bool TRANS>
-int rotate16_segs(const RotSeg* segs, int n, hipStream_t st) {
-  RotSegs S{};
-  int k = 0;
-  int64_t tiles = 0;
-  for (int i = 0; i < n; ++i) {
-    if (segs[i].M <= 0) continue;
-    S.s[k++] = segs[i];
-    tiles = std::max<int64_t>(tiles, (segs[i].M + kRotRows - 1) / kRotRows);
-  }
-  if (k == 0) return LKV_OK;
-  const int64_t cap = 2 * static_cast<int64_t>(device_cu_count());
-  const int64_t g = tiles < cap ? tiles : cap;
-  hipLaunchKernelGGL((rotate16_kernel<IN_F16, OUT_F16, TRANS>), dim3(static_cast<unsigned>(g), static_cast<unsigned>(k)),
-                     dim3(kThreads), 0, st, S);
-  LKV_LAUNCH_CHECK("tq_prefill_attn rotation");
-  return LKV_OK;
-}
-
-template <bool IN_F16, bool OUT_F16, bool TRANS>
-int rotate16(const void* x, int64_t M, const float* Pi, float scale, void* y, hipStream_t st) {
-  const RotSeg seg{x, Pi, y, M, scale};
-  return rotate16_segs<IN_F16, OUT_F16, TRANS>(&seg, 1, st);
 }
 
 // fp16 positions 0..7 of a natural-order group reordered to kPermDim.
@@ -728,9 +663,12 @@ extern "C" int lkv_tq_prefill_attn(const void* q, const uint8_t* k_codes, const 
 
   // the hot rings in the rotated domains (one launch; every hot slot is rotated, only the current tokens' are read)
   {
-    const int64_t nhot = B * Hkv * hot_cap;
-    const RotSeg segs[2] = {{k_hot, PiK, hk, nhot, 1.f}, {v_hot, PiV, hv, nhot, 1.f}};
-    if (int e = rotate16_segs<true, true, false>(segs, 2, st)) return e;
+    const RotSegs segs{{{static_cast<const uint16_t*>(k_hot), PiK, hk}, {static_cast<const uint16_t*>(v_hot), PiV, hv}},
+                       B * Hkv * hot_cap};
+    const int64_t tiles = (segs.M + kRotRows - 1) / kRotRows, most = 2 * static_cast<int64_t>(device_cu_count());
+    hipLaunchKernelGGL(rotate16_kernel, dim3(static_cast<unsigned>(tiles < most ? tiles : most), 2), dim3(kThreads), 0, st,
+                       segs);
+    LKV_LAUNCH_CHECK("tq_prefill_attn rotation");
   }
   PrefillParams P;
   P.q16 = static_cast<const uint16_t*>(q);
