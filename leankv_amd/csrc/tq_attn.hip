@@ -11,7 +11,7 @@
 // rotated domain, and PiV is applied once per query head at the end.
 //
 // Launches (all on the caller's stream, no inter-block waits):
-//   1. split kernel, grid splits x kv_heads x batch, 16 waves per block (one
+//   1. split kernel, grid splits x kv_heads x batch, 16 or 8 waves per block (one
 //      block per CU), each block owning a contiguous range of cold tokens.  Its
 //      prologue rotates the G query heads of its kv head, q_rot = q @ PiK^T on
 //      fp16 MFMA with PiK in two parts (the decode step sums the query from its
@@ -33,15 +33,14 @@
 //        from the lane's own softmax registers (same 8 tokens);
 //      * the waves merge through LDS and the block writes
 //        (m, l, acc[G][128]) per head to the workspace;
-//      What bounds it: instruction issue, ~290 vector instructions per 32
-//      tokens.  One wave of a SIMD issues one every ~5 cycles, two together one
-//      every 2.4-3.5 and four one every 1.7-2.8, so the kernel is cut to 120
-//      registers for 4 waves per SIMD (one register set, no second block in
-//      flight: 2, 3 and 4 sets at 2 waves measured alike).  B = 16, 32/8
+//      What bounds it: instruction issue, 239 vector instructions per 32
+//      tokens at 3 bits.  One wave of a SIMD issues one every ~5 cycles, two
+//      together one every 2.4-3.5 and four one every 1.7-2.8, so the kernel is
+//      cut to 120 registers for 4 waves per SIMD (one register set, no second
+//      block in flight: 2, 3 and 4 sets at 2 waves measured alike).  B = 16, 32/8
 //      heads, 4096 tokens, 3 bits, both kernels: 26.6 us with two 4-wave blocks
 //      of two register sets per CU, 25.2 with one 8-wave block of three, 21.8
-//      now; B = 1, 32768 tokens: 22.5 -> 20.0 -> 17.9.  Of the 21.8, 7.4 are
-//      the blocks' fixed part and the combine's launch and run 5.
+//      now; B = 1, 32768 tokens: 22.5 -> 20.0 -> 17.9.
 //   2. combine kernel, one block of 8 waves per (batch, query head): issues
 //      every load it needs at once (split maxima and sums, the rotated
 //      partial sums, the fp16 hot window and the PiV column slice), then
@@ -86,8 +85,6 @@ __device__ __forceinline__ void stamp(uint64_t* arr, int i) {
 #endif
 
 constexpr int kD = 128;
-constexpr int kWaves = 16;
-constexpr int kThreads = 64 * kWaves;
 constexpr int kBlk = 32;    // tokens per wave step
 constexpr int kHotMax = 256;  // hot-window slots the combine walks (64 per slot group)
 constexpr float kLog2e = 1.4426950408889634f;
@@ -351,15 +348,14 @@ __device__ __forceinline__ void attend_block(BlockRegs& R, int t0, int t_end, co
 
 constexpr int kORow = kD + 4;   // padded LDS row of the per-wave outputs
 constexpr int kQRow = kD + 8;   // padded LDS row (fp16) of the query operand
-// Resident split blocks per CU: sets the register budget (4 waves per SIMD).
-constexpr int kSplitBlocksPerCU = 1;
-
 constexpr int kMaxPg = 256;  // pages of one split in the paged layout
 
 // QPRE (decode mode): q|k|v partial chunks loaded ahead of the codes, at least
 // the q|k|v GEMV's chunk count for the fast path (8 or 16).
-template <bool PERM, bool DECODE, bool PAGED, int CB, int QPRE = 16>
-__global__ __launch_bounds__(kThreads, 4 * kSplitBlocksPerCU) void tq_attn_split_kernel(AttnParams P) {
+// kWaves: waves of a block, one block per CU (16: 4 waves per SIMD, which sets the register budget).
+template <bool PERM, bool DECODE, bool PAGED, int CB, int kWaves, int QPRE = 16>
+__global__ __launch_bounds__(64 * kWaves, kWaves / 4) void tq_attn_split_kernel(AttnParams P) {
+  constexpr int kThreads = 64 * kWaves;
   static_assert(!(PAGED && DECODE), "the fused decode step uses the dense layout");
   static_assert(CB == 4 || PERM, "narrow code rows (1, 2 bits) decode through v_perm");
   constexpr int RB = code_row_bytes<CB>();
@@ -463,7 +459,7 @@ __global__ __launch_bounds__(kThreads, 4 * kSplitBlocksPerCU) void tq_attn_split
   const int h = lane & 15, g = lane >> 4;
   float* const s_part = &s_o[0][0][0];
   {
-    float4 pik[2][2];
+    float4 pik[32 / kWaves][2];
     load_pik_operand(P.PiK, wave, lane, pik);
     u32x4 qb;
     if constexpr (DECODE) {
@@ -554,8 +550,9 @@ __global__ __launch_bounds__(kThreads, 4 * kSplitBlocksPerCU) void tq_attn_split
   if constexpr (!PERM)
     if (tid < 256) s_lut[tid] = pack2h(c_lo, c_hi);
   __syncthreads();
-  {
-    const int hh = tid >> 6, pp = tid & 63, j = pp & 3;  // positions 2 pp, 2 pp + 1 of head hh
+#pragma unroll
+  for (int hh = tid >> 6; hh < 16; hh += kWaves) {
+    const int pp = tid & 63, j = pp & 3;  // positions 2 pp, 2 pp + 1 of head hh
     const int d0 = 8 * (pp >> 2) + (PERM ? (j < 2 ? 4 * j : 4 * j - 7) : 2 * j), d1 = d0 + (PERM ? 2 : 1);  // kPermDim
     uint32_t v = 0u;
     if (hh < G)
@@ -874,6 +871,62 @@ int64_t max_splits(int64_t B, int64_t Hkv) {
   return ns > kMaxSplits - 1 ? kMaxSplits - 1 : ns < 1 ? 1 : ns;
 }
 
+// Waves of a split block where one pass of that many covers a split and every block has a CU of its own: more of them
+// would have no tokens, and only lengthen the prologue's barriers and the merge.  Both kernels, 32/8 heads, us with 8 /
+// with 16 waves (two 4-wave blocks before): 1 x 4160 tokens 11.3 / 12.4 (12.1) at 3 bits, 11.7 / 12.9 (12.4) at 4, 11.7
+// / 12.6 (13.3) at 1; 1 x 164 tokens 10.1 / 11.0 (10.7) and 10.3 / 11.4 (10.5); 16 query heads on one kv head, 2000
+// tokens 12.1 / 13.4 (12.7).
+constexpr int kSmallWaves = 8;
+
+template <int W>
+void split_launch(const AttnParams& P, const AttnCall& c, dim3 grid, hipStream_t st) {
+#define LKV_SPLIT(...) hipLaunchKernelGGL((tq_attn_split_kernel<__VA_ARGS__>), grid, dim3(64 * W), 0, st, P)
+  if (c.pq != nullptr) {
+    // the fewest partial loads ahead of the codes that still cover every chunk
+    const bool pre8 = c.nchunk <= 8;
+    switch (c.bits) {
+      case 1:
+        if (pre8)
+          LKV_SPLIT(true, true, false, 1, W, 8);
+        else
+          LKV_SPLIT(true, true, false, 1, W, 16);
+        break;
+      case 2:
+        if (pre8)
+          LKV_SPLIT(true, true, false, 2, W, 8);
+        else
+          LKV_SPLIT(true, true, false, 2, W, 16);
+        break;
+      case 3:
+        if (pre8)
+          LKV_SPLIT(true, true, false, 4, W, 8);
+        else
+          LKV_SPLIT(true, true, false, 4, W, 16);
+        break;
+      default:
+        if (pre8)
+          LKV_SPLIT(false, true, false, 4, W, 8);
+        else
+          LKV_SPLIT(false, true, false, 4, W, 16);
+    }
+  } else if (c.indptr != nullptr) {
+    switch (c.bits) {
+      case 1: LKV_SPLIT(true, false, true, 1, W); break;
+      case 2: LKV_SPLIT(true, false, true, 2, W); break;
+      case 3: LKV_SPLIT(true, false, true, 4, W); break;
+      default: LKV_SPLIT(false, false, true, 4, W);
+    }
+  } else {
+    switch (c.bits) {
+      case 1: LKV_SPLIT(true, false, false, 1, W); break;
+      case 2: LKV_SPLIT(true, false, false, 2, W); break;
+      case 3: LKV_SPLIT(true, false, false, 4, W); break;
+      default: LKV_SPLIT(false, false, false, 4, W);
+    }
+  }
+#undef LKV_SPLIT
+}
+
 }  // namespace
 
 AttnPlan attn_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t max_len, int64_t hot_cap, int64_t max_split_tokens) {
@@ -967,48 +1020,12 @@ int attn_launch(const AttnCall& c, const AttnPlan& pl, hipStream_t st) {
     P.q = c.q16;  // the combine's hot-window query
     P.k_hot = c.k_ring;
     P.v_hot = c.v_ring;
-    // the fewest partial loads ahead of the codes that still cover every chunk
-    const bool pre8 = c.nchunk <= 8;
-    switch (c.bits) {
-      case 1:
-        if (pre8)
-          hipLaunchKernelGGL((tq_attn_split_kernel<true, true, false, 1, 8>), grid, dim3(kThreads), 0, st, P);
-        else
-          hipLaunchKernelGGL((tq_attn_split_kernel<true, true, false, 1, 16>), grid, dim3(kThreads), 0, st, P);
-        break;
-      case 2:
-        if (pre8)
-          hipLaunchKernelGGL((tq_attn_split_kernel<true, true, false, 2, 8>), grid, dim3(kThreads), 0, st, P);
-        else
-          hipLaunchKernelGGL((tq_attn_split_kernel<true, true, false, 2, 16>), grid, dim3(kThreads), 0, st, P);
-        break;
-      case 3:
-        if (pre8)
-          hipLaunchKernelGGL((tq_attn_split_kernel<true, true, false, 4, 8>), grid, dim3(kThreads), 0, st, P);
-        else
-          hipLaunchKernelGGL((tq_attn_split_kernel<true, true, false, 4, 16>), grid, dim3(kThreads), 0, st, P);
-        break;
-      default:
-        if (pre8)
-          hipLaunchKernelGGL((tq_attn_split_kernel<false, true, false, 4, 8>), grid, dim3(kThreads), 0, st, P);
-        else
-          hipLaunchKernelGGL((tq_attn_split_kernel<false, true, false, 4, 16>), grid, dim3(kThreads), 0, st, P);
-    }
-  } else if (c.indptr != nullptr) {
-    switch (c.bits) {
-      case 1: hipLaunchKernelGGL((tq_attn_split_kernel<true, false, true, 1>), grid, dim3(kThreads), 0, st, P); break;
-      case 2: hipLaunchKernelGGL((tq_attn_split_kernel<true, false, true, 2>), grid, dim3(kThreads), 0, st, P); break;
-      case 3: hipLaunchKernelGGL((tq_attn_split_kernel<true, false, true, 4>), grid, dim3(kThreads), 0, st, P); break;
-      default: hipLaunchKernelGGL((tq_attn_split_kernel<false, false, true, 4>), grid, dim3(kThreads), 0, st, P);
-    }
-  } else {
-    switch (c.bits) {
-      case 1: hipLaunchKernelGGL((tq_attn_split_kernel<true, false, false, 1>), grid, dim3(kThreads), 0, st, P); break;
-      case 2: hipLaunchKernelGGL((tq_attn_split_kernel<true, false, false, 2>), grid, dim3(kThreads), 0, st, P); break;
-      case 3: hipLaunchKernelGGL((tq_attn_split_kernel<true, false, false, 4>), grid, dim3(kThreads), 0, st, P); break;
-      default: hipLaunchKernelGGL((tq_attn_split_kernel<false, false, false, 4>), grid, dim3(kThreads), 0, st, P);
-    }
   }
+  const int64_t blocks = static_cast<int64_t>(pl.nsplit) * c.Hkv * c.B;
+  if (pl.split_tokens <= kSmallWaves * kBlk && blocks <= device_cu_count())
+    split_launch<kSmallWaves>(P, c, grid, st);
+  else
+    split_launch<16>(P, c, grid, st);
   LKV_LAUNCH_CHECK("tq_decode_attn split");
   if (c.hot_cap <= 64)
     hipLaunchKernelGGL(tq_attn_combine_kernel<1>, cgrid, dim3(kCombThreads), 0, st, P);
