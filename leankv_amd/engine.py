@@ -414,9 +414,10 @@ class BatchedEngine:
     def _plain_embedding(self, emb) -> bool:
         """Whether emb(tok) is the tokens' rows of its fp16 weight and nothing else."""
         w = getattr(emb, "weight", None)
-        return (type(emb) is torch.nn.Embedding and "forward" not in emb.__dict__ and emb.max_norm is None
-                and not emb._forward_hooks and not emb._forward_pre_hooks and w.dtype == torch.float16
-                and w.device == self.tok.device and w.is_contiguous() and w.data_ptr() % 16 == 0)
+        return (type(emb) is torch.nn.Embedding and type(w) is torch.nn.Parameter and "forward" not in emb.__dict__
+                and emb.max_norm is None and not emb._forward_hooks and not emb._forward_pre_hooks
+                and w.dtype == torch.float16 and w.device == self.tok.device and w.is_contiguous()
+                and w.data_ptr() % 16 == 0)
 
     @staticmethod
     def _lkv_norm(mod, x: torch.Tensor) -> bool:
