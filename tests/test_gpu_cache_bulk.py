@@ -115,3 +115,41 @@ def test_update_of_another_batch_is_refused():
     with pytest.raises(LeanKVError):
         c.update(y, y, 0)
     assert c.get_seq_length(0) == 20 and all(torch.equal(a, b) for a, b in zip(c[0], want))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_update_of_other_types(dtype):
+    """Keys and values of a model's own type: the cache of their fp16 values, handed back in the cache's type."""
+    from leankv_amd.turboquant.cache import TurboQuantCache
+
+    g = torch.Generator(device="cuda").manual_seed(5)
+    parts = [[torch.randn(2, 3, S, 128, generator=g, device="cuda").to(dtype) for _ in range(2)] for S in (30, 50, 1, 20)]
+    a = TurboQuantCache(num_layers=1, hot_buffer_size=16, device="cuda", max_seq_len=128, dtype=dtype)
+    b = TurboQuantCache(num_layers=1, hot_buffer_size=16, device="cuda", max_seq_len=128)
+    for k, v in parts:
+        got, want = a.update(k, v, 0), b.update(k.half(), v.half(), 0)
+        assert all(x.dtype == dtype and torch.equal(x, y.to(dtype)) for x, y in zip(got, want))
+
+
+def test_update_and_read_on_another_stream():
+    """Layouts that are copied first, on a stream that is kept busy: launched there, temporaries kept until used."""
+    from leankv_amd.turboquant.cache import TurboQuantCache
+
+    g = torch.Generator(device="cuda").manual_seed(6)
+    parts = [[torch.randn(2, 3, 256, S, generator=g, device="cuda").half()[:, :, ::2].transpose(2, 3) for _ in range(2)]
+             for S in (300, 40, 7)]
+
+    def run():
+        c = TurboQuantCache(num_layers=1, hot_buffer_size=64, device="cuda", max_seq_len=512)
+        return [t for k, v in parts for t in c.update(k, v, 0)]
+
+    want = run()
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        x = torch.randn(4096, 4096, device="cuda")
+        for _ in range(4):
+            x = x @ x * 1e-3
+        got = run()
+    s.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
