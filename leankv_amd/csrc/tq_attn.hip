@@ -845,7 +845,7 @@ constexpr int kSplitGran = 256;  // tokens of a split are a multiple of this (ha
 
 // Tuning knobs, read once.  LKV_ATTN_SPLIT_TARGET=k: k split blocks per CU instead of attn_plan's choice.
 // LKV_ATTN_MIN_SPLIT_TOKENS=n: at least n cold tokens per split (default 256: each split block repeats the query
-// prologue).
+// prologue; splits are whole 256-token units, so less has no effect).
 int attn_split_target() {
   static const int k = [] {
     const char* env = getenv("LKV_ATTN_SPLIT_TARGET");

@@ -14,8 +14,8 @@
 // and one un-rotation by PiV finishes each output row.
 //
 // Launches of lkv_tq_prefill_attn (two, on the caller's stream):
-//   1. rotate16_kernel (fp16 MFMA, PiK / PiV split exactly into fp16 hi + lo
-//      parts): the hot rings k @ PiK^T and v @ PiV^T (fp16);
+//   1. rotate16_kernel (fp16 MFMA, PiK / PiV split into fp16 hi + lo parts, 22
+//      bits and more): the hot rings k @ PiK^T and v @ PiV^T (fp16);
 //   2. tq_prefill_attn_kernel: grid (query tiles, kv heads, batch), 8 waves.
 //      A block owns 256 (query, head) columns: 256 / G consecutive queries x
 //      the G heads of one kv head, 32 columns per wave.  Its prologue rotates
@@ -569,7 +569,7 @@ __global__ __launch_bounds__(kPThreads, 1) void tq_prefill_attn_kernel(PrefillPa
   // ---- normalise, un-rotate (out = o_rot @ PiV) and write fp16 rows: A = 32
   // output dims of PiV^T, B = the lane's own normalised sums (k slots of step
   // (db, u): its dims 32 db + 16 u + 4 hf + .., and 8 further on), both split
-  // exactly into fp16 hi + lo / 2048 (hi.hi + hi.lo + lo.hi, the lo.lo term
+  // into fp16 hi + lo / 2048 (hi.hi + hi.lo + lo.hi, the lo.lo term
   // dropped: ~2^-22 relative).
   const float L = xhalf_sum(l);
   const float inv = L > 0.f ? 1.f / L : 0.f;

@@ -73,7 +73,8 @@ __device__ __forceinline__ void rotate_wave_tile(const float (&a)[32], const PiT
 
 // #(b < y) over the 2^BITS - 1 sorted decision boundaries: the count of
 // bucket<BITS>, by binary search from 3 bits on.  3 bits: every boundary index
-// is a compile-time constant (selects, no indexing).  4 bits: a table in LDS,
+// is a compile-time constant; the compiler makes branches of the selects (about 30
+// per tile).  4 bits: a table in LDS,
 // the next boundary addressed by the bucket so far (kept in registers, the
 // selects between boundaries compile to an indexed load from a private,
 // memory-backed copy of the table).
@@ -165,7 +166,8 @@ __global__ __launch_bounds__(kThreads, 2) void quantize_wave_kernel(const void* 
     f32x4 acc[8];
     rotate_wave_tile(a, s_b, lane, acc);
     const int64_t next = tile + static_cast<int64_t>(gridDim.x) * 4;
-    if (next < ntiles) load_a(next);  // in flight during the bucketing and stores
+    // fp32 rows are in flight during the bucketing and stores; fp16 rows are waited for here, where they are widened
+    if (next < ntiles) load_a(next);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int64_t row = row0 + 4 * g + i;
@@ -190,13 +192,14 @@ __global__ __launch_bounds__(kThreads, 2) void quantize_wave_kernel(const void* 
 // they arrived, so no slot is written before it was read.  New tokens whose
 // slot held none are copied first, by all threads.
 //
-// Bound by the fp32 MFMA chains (13.4 us for the 2 x 32 K vectors of a 4096-token
-// prompt layer at 154 TFLOP/s); it reads fp16 rows where they are (any row
-// strides) and writes the cache in place.  Measured against two widening
-// copies, two quantize launches, four strided copies into the store, index
-// arithmetic and two ring scatters per layer update: a 4096-token prompt layer
-// (8 kv heads, update and attention) 304 -> 244 us, four prompts of 1201
-// tokens in three chunks 536 -> 241 us.
+// The fp32 MFMA chains take 13.4 us for the 2 x 32 K vectors of a 4096-token prompt
+// layer at 154 TFLOP/s, the kernel 30: at two blocks per CU the staging of the
+// matrix, the norm, the product and the bucketing of a wave's few tiles follow
+// one another.  It reads fp16 rows where they are (any row strides) and writes the
+// cache in place.  Measured against two widening copies, two quantize launches,
+// four strided copies into the store, index arithmetic and two ring scatters per
+// layer update: a 4096-token prompt layer (8 kv heads, update and attention) 304 ->
+// 244 us, four prompts of 1201 tokens in three chunks 536 -> 241 us.
 struct BulkSide {
   const uint16_t* x;  // [R / H][H][S] rows of 128, strides sb, sh, ss (elements)
   int64_t sb, sh, ss;
@@ -303,7 +306,8 @@ __global__ __launch_bounds__(kThreads, 2) void bulk_update_kernel(BulkArgs P) {
     f32x4 acc[8];
     rotate_wave_tile(a, s_b, lane, acc);
     const uint32_t next = tile + gridDim.x * 4;
-    if (next < ntiles) load_a(next);  // in flight during the bucketing and stores
+    // in flight until the first store of codes; at 3 bits waited for at the first branch of the bucketing
+    if (next < ntiles) load_a(next);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const uint32_t rr = row0 + 4 * g + i;

@@ -5,11 +5,12 @@
 // fp32 rounded to fp16, then the fp16 hot window).
 //
 // The rotation of 128-dim centroid rows runs on v_mfma_f32_16x16x32_f16 with
-// both operands split exactly into fp16 parts, v = hi + lo / 2048 (22 bits and
-// more), all four products of the parts kept in fp32 accumulators: 64 MFMA
-// cycles per 32 input dims where the fp32 MFMA chain takes 256.  It is the more
-// exact of the two: of 4.2 M values, 2341-2678 are not the 64-bit result
-// rounded to fp16 (1 to 4 bits), of the fp32 chain's 4197-4267.
+// both operands split into fp16 parts, v = hi + lo / 2048 (v itself but for the
+// last bit of a quarter of the fp32 values, 2^-23 relative), all four products of
+// the parts kept in fp32 accumulators: 64 MFMA cycles per 32 input dims where
+// the fp32 MFMA chain takes 256.  Its results are the closer ones: of 4.2 M
+// values, 2341-2678 are not the 64-bit result rounded to fp16 (1 to 4 bits), of
+// the fp32 chain's 4197-4267.
 //
 // One block of 4 waves walks tiles of 16 tokens; wave w owns output dims 32 w
 // .. 32 w + 31, its parts of Pi in registers.  Transposed products: A = 16
@@ -18,11 +19,12 @@
 // ends with 8 consecutive dims of one token and stores them as 16 bytes.  Input
 // dims are taken in the order that a lane's 16 code bytes hold them.
 //
-// Bound by latency and the launch at one sequence (21 MB, 4.4 us at the copy
-// rate of 4.9 TB/s).  One launch for both sides, read where the cache holds
-// them and written in place: 15.3 us per 4096-token layer (8 kv heads, 3 bits,
-// back to back), against 88 us for four copies of the strided store, two
-// fp32-MFMA dequantize launches, two ring gathers and two concatenations.
+// Bound by the chain of a wave's tiles (codes, lookup, products, 16-byte stores;
+// 8 tiles each at one sequence), not by bytes: 21 MB, 4.4 us at the copy rate of
+// 4.9 TB/s.  One launch for both sides, read where the cache holds them and written
+// in place: 15 us per 4096-token layer (8 kv heads, 3 bits, back to back, on the
+// card and on the host alike), against 88 us for four copies of the strided store,
+// two fp32-MFMA dequantize launches, two ring gathers and two concatenations.
 #include <algorithm>
 
 #include "kernels.h"
