@@ -550,7 +550,7 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 4) void tq_attn_split_kernel(
   if constexpr (!PERM)
     if (tid < 256) s_lut[tid] = pack2h(c_lo, c_hi);
   __syncthreads();
-#pragma unroll
+#pragma unroll 1  // (unrolled, the 8-wave decode step spills scalars and so reserves scratch)
   for (int hh = tid >> 6; hh < 16; hh += kWaves) {
     const int pp = tid & 63, j = pp & 3;  // positions 2 pp, 2 pp + 1 of head hh
     const int d0 = 8 * (pp >> 2) + (PERM ? (j < 2 ? 4 * j : 4 * j - 7) : 2 * j), d1 = d0 + (PERM ? 2 : 1);  // kPermDim
